@@ -198,7 +198,9 @@ int pmnb_kernel_timing(pmnb_ctx *ctx, int32_t enable, double *ms,
 /* Pair path a context's evaluations take (known after pmnb_set_box):
    PMNB_PATH_TILE: the algorithm cutoff reaches every pair within the
      switching cutoff, so the pair set does not depend on the cell grid,
-     and at most 8 LJ types: the path's own column grid and tile kernel;
+     and at most 8 LJ types: the path's own column grid and tile kernel
+     (9 .. 256 types run that kernel too, with the LJ table in memory, and
+     are reported as the path of their cell grid below);
    PMNB_PATH_LIST: the reference's cell grid and delta list
      (topology/CellListEnumeratorPeriodicBoundaries.h:46-83) drive a
      neighbour list per evaluation;
@@ -301,10 +303,9 @@ int pmnb_batch_run_graph(pmnb_batch *b, const double *d_positions,
                          double *d_forces, double *d_out, uint32_t flags,
                          int32_t n_steps, void *stream);
 
-/* Autotuner: times every pair-kernel shape (the shell, and the buffered
-   candidates per wave with the waves per SIMD its LDS allows: mixed 0 full
-   shell 256 / 3, 1 full shell 128 / 4, 2 half shell 192 / 3; FP64 0 full
-   shell 192 / 3, 1 half shell 128 / 2) and persistent grid size on these
+/* Autotuner: times every pair-kernel shape (0 chosen by the number of work
+   items, 1 a wave per item, 2, mixed only, a block per item; all give the
+   same bits) and persistent grid size on these
    positions and keeps the fastest for later evaluations; returns the shape
    index,
    the grid cap in blocks (0 = one block per work group of items) and its
@@ -315,10 +316,7 @@ int pmnb_batch_autotune(pmnb_batch *b, const double *d_positions,
                         int32_t *shape, int32_t *grid_blocks, double *ms);
 
 /* Sets the pair-kernel shape (mixed 0 .. 2, FP64 0 .. 1, as the autotuner
-   numbers them) and grid cap by hand.  The shape (autotuned or set) is the
-   one of evaluations that form energies; a mixed evaluation whose energies
-   nobody reads (a dynamics step before the last of a run) takes shape 0
-   without energy sums, the fastest there. */
+   numbers them) and grid cap by hand. */
 int pmnb_batch_set_shape(pmnb_batch *b, int32_t shape, int32_t grid_blocks);
 
 /* pmnb_force_pairs for the whole batch at device positions d_positions:

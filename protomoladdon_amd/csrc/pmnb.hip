@@ -32,7 +32,7 @@
 #include "pmnb_tile.h"
 #include "pmnb_queue.h"
 #include "pmnb_adjoint.h"
-#include "pmnb_tilemask.h"
+#include "pmnb_cluster.h"
 #include "pmnb_leapfrog.h"
 #include "pmnb_ewald.h"
 #include "pmnb_pme.h"
@@ -177,10 +177,14 @@ int host_crew_size() {
 // pmnb_evaluate shares its host copy and add over the crew for systems of
 // at least kHostCrewMin coordinates
 constexpr int kHostCrewMin = 1 << 16;
-// Above this many cells the tile path scans the cell counts over the
-// columns in three launches instead of one block (512 water replicas,
-// about 63,000 cells in 5,500 columns: 146 us in one block)
-constexpr int kScanCellsOneBlock = 16384;
+// A pair launch of fewer work items than this takes a block per item (a wave
+// per stream of candidates) instead of a wave per item: the chip holds 1,024
+// SIMDs, and below about three items each the longest wave decides.  A block
+// per item repeats the item's setup in four waves.  A whole evaluation with
+// energies of water, a wave / a block per item: 187 items 88 / 43 us, 1,500
+// items 94 / 75, 2,250 101 / 93, 3,000 112.5 / 112.4, 3,750 120 / 132, 6,000
+// 176 / 187.
+constexpr int kSplitItems = 3000;
 
 struct pmnb_ctx {
   pmnb_params prm{};
@@ -196,35 +200,35 @@ struct pmnb_ctx {
   std::vector<int4> shell;  // (0,0,0) then the reference's delta list
   int per_pair_wrap = 0;
   long long last_pairs = 0;
-  // device counter of the last evaluation's pairs (pmnb_last_pair_count)
+  // device counter of the last evaluation's pairs (pmnb_last_pair_count);
+  // it holds last_np_per counts per pair (the tile path's pair kernel counts
+  // both visits)
   const unsigned long long *last_np = nullptr;
+  int last_np_per = 1;
   // device: topology (original order)
   DevBuf d_type, d_q, d_mol, d_xfull, d_xmod, d_xown, d_lj, d_ljf;
   // device: per evaluation
   DevBuf d_pos, d_force, d_out, d_com, d_cell_of, d_count, d_start, d_fill,
       d_sorted, d_sx, d_sy, d_sz, d_loc, d_stype, d_sq, d_smol, d_scell,
       d_srec, d_shell, d_partial, d_npairs, d_pairs, d_list, d_ncount, d_partial2,
-      d_shell_off, d_box;
+      d_shell_off;
   int shell_uploaded = 0;
   std::vector<float4> shell_off;  // FP32 cell offsets of the shell entries
   bool use_list = false;          // neighbour-list path available
   bool use_tile = false;          // LDS-staged path (own column grid)
-  TileGrid tile{};
+  bool tile_types = false;        // ... and its types fit the LDS table
+  int ref_shell = 0;              // entries of the reference grid's shell
   // tile path geometry: one replica for a single system, several for a
   // batch (atoms of replica r then carry r in d_rep_of)
   std::vector<TileRep> reps;
-  std::vector<int> col_rep;       // replica of each global column
-  int ncol_total = 0;
+  std::vector<int> bin_rep;       // replica of each bin
+  int nbin = 0, nslots = 0;       // bins, work-item slots of all replicas
+  int bucket_cap = 64;            // atom slots per bin
   bool batch = false;
   DevBuf d_rep_of;
-  int rep_uploaded = 0;           // reps and col_rep are on the device
+  int rep_uploaded = 0;           // reps and bin_rep are on the device
   DevBuf d_partial_lj;            // adjoint: LJ-parameter partials per item
-  // tile path: per sorted slot the 64-bit fixed-point force (3 words mixed,
-  // 6 FP64), all zero between evaluations (the finish kernel clears it)
-  DevBuf d_ffix;
-  const void *ffix_zeroed = nullptr;  // allocation last cleared
-  DevBuf d_bucket;                    // tile path: cap atoms per cell
-  int bucket_cap = 64;
+  DevBuf d_bucket, d_ccount;
   // d_count holds zeros at the start of the next evaluation on the tile path
   // (the finish kernel clears it after the pair kernel): no clearing launch
   bool counts_zero = false;
@@ -238,9 +242,9 @@ struct pmnb_ctx {
   hipEvent_t h_ev[1] = {};  // pmnb_evaluate: results are on the host
   HostCrew crew;             // pmnb_evaluate: host threads (started once)
   bool crew_started = false;
-  int shape = 0;                  // tile-path kernel shape (mixed)
+  int shape = 0;                  // tile-path kernel shape
   int grid_cap = 0;               // persistent pair grid: max blocks (0: none)
-  DevBuf d_items, d_nitems, d_reps, d_col_rep, d_rep_first, d_colscan;
+  DevBuf d_items, d_reps, d_bin_rep, d_rep_items;
   double box_key[12] = {0};       // e1, e2, e3, origin of the current box
   unsigned long long topo_gen = 0;  // pmnb_set_topology calls so far
   int cap = 0;                    // list slots per atom
@@ -339,24 +343,29 @@ ForceParams make_params_for(const pmnb_params &prm, double csf) {
   return P;
 }
 
-// z cell size of the tile path over the pair cutoff: the mixed kernel is as
-// fast with rcp / 3 as with rcp / 4 and the cell build is faster with fewer
-// cells; the FP64 kernel is faster with rcp / 4 (measured on the 96k water)
-double tile_zfrac(const pmnb_params &prm) {
-  return prm.precision == PMNB_PREC_MIXED ? 1.0 / 3.0 : 0.25;
-}
-
-// Column grid of the tile path for box b and pair cutoff rcp: x/y columns
-// at least rcp wide, z cells of about zfrac * rcp.  An axis with a single column
-// is marked for per-pair minimum image.  shell receives the distinct
-// cell offsets within reach ((0,0,0) first), which the pair-set extraction
-// walks.  Returns false when the grid is too large.
-bool make_tile_rep(const Box &b, double rcp, double zfrac, TileRep &rep,
+// Column grid of the tile path for box b, pair cutoff rcp and n atoms: x/y
+// columns at least rcp / 2 wide, z cells of about rcp / 8.  A thin gas gets
+// wider columns and z cells (16 atoms per column, one per z cell on average),
+// so that a work item still holds several atoms.  An axis with fewer than
+// five columns is marked for the per-pair minimum image.  A column's z cells
+// are split into bins of at most 256 cells and about 256 atoms.  shell
+// receives the distinct cell offsets within reach ((0,0,0) first), which the
+// pair-set extraction walks.
+void make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
                    std::vector<int4> &shell) {
-  const int tx = std::max(1, (int)std::floor(b.H[0] / rcp));
-  const int ty = std::max(1, (int)std::floor(b.H[1] / rcp));
-  const int tz = std::max(1, (int)std::floor(b.H[2] / (zfrac * rcp)));
-  if ((long long)tx * ty * tz >= (1ll << 26)) return false;
+  auto cells = [](double len, double w) {
+    return (int)std::max(1.0, std::min(std::floor(len / w), 1e5));
+  };
+  int tx = cells(b.H[0], 0.5 * rcp), ty = cells(b.H[1], 0.5 * rcp);
+  const double most = std::max(1.0, n / 16.0);
+  while ((double)tx * ty > most && (tx > 5 || ty > 5)) {
+    int &k = tx >= ty ? tx : ty;
+    k = std::max(5, std::min(k - 1, (int)(k * 0.9)));
+  }
+  const int ncol = tx * ty;
+  const int col_atoms = (n + ncol - 1) / ncol;
+  const int tz = std::min(cells(b.H[2], 0.125 * rcp),
+                          std::max(col_atoms, std::min(cells(b.H[2], rcp), 64)));
   rep = TileRep{};
   const double csz = b.H[2] / tz;
   const int rz = (int)std::floor(rcp / csz) + 1;
@@ -377,27 +386,34 @@ bool make_tile_rep(const Box &b, double rcp, double zfrac, TileRep &rep,
   rep.tg.csx = (float)tg.cs[0];
   rep.tg.csy = (float)tg.cs[1];
   rep.tg.csz = (float)tg.cs[2];
+  rep.tg.lox = (float)(tg.cs[0] - (double)rep.tg.csx);
+  rep.tg.loy = (float)(tg.cs[1] - (double)rep.tg.csy);
+  rep.tg.loz = (float)(tg.cs[2] - (double)rep.tg.csz);
   for (int k = 0; k < 3; k++) {
     rep.L[k] = (float)b.e[k];
+    rep.Llo[k] = (float)(b.e[k] - (double)rep.L[k]);
     rep.iL[k] = (float)b.er[k];
   }
-  // one column per axis (box < 2 rcp): per-pair minimum image; with two,
-  // the column offsets -1 and +1 reach the same column at images one box
-  // length (>= 2 rcp) apart, so at most one of them is within the cutoff
-  rep.wrap[0] = tx == 1;
-  rep.wrap[1] = ty == 1;
-  rep.ncol = tx * ty;
+  rep.wrap[0] = tx < 5;
+  rep.wrap[1] = ty < 5;
+  const int want = std::max((tz + kBinCells - 1) / kBinCells,
+                            (col_atoms + 255) / 256);
+  rep.fz = std::max(1, (tz + want - 1) / want);
+  rep.ns = (tz + rep.fz - 1) / rep.fz;
+  rep.nbin = ncol * rep.ns;
+  rep.natom = n;
+  rep.item_max = n / kTileAtoms + std::min(n, rep.nbin);
   // distinct offsets per axis
-  auto offsets = [](int n, int reach) {
+  auto offsets = [](int m, int reach) {
     std::vector<int> o;
-    if (n >= 2 * reach + 1) {
+    if (m >= 2 * reach + 1) {
       for (int d = -reach; d <= reach; d++) o.push_back(d);
     } else {
-      for (int d = 0; d < n; d++) o.push_back(d);
+      for (int d = 0; d < m; d++) o.push_back(d);
     }
     return o;
   };
-  const std::vector<int> ox = offsets(tx, 1), oy = offsets(ty, 1),
+  const std::vector<int> ox = offsets(tx, 2), oy = offsets(ty, 2),
                          oz = offsets(tz, rz);
   shell.clear();
   shell.push_back(make_int4(0, 0, 0, 0));
@@ -405,7 +421,6 @@ bool make_tile_rep(const Box &b, double rcp, double zfrac, TileRep &rep,
     for (int dy : oy)
       for (int dz : oz)
         if (dx || dy || dz) shell.push_back(make_int4(dx, dy, dz, 0));
-  return true;
 }
 
 // Box + grid + shell offsets exactly as PeriodicBoundaryConditions::set,
@@ -519,6 +534,7 @@ int build_box(pmnb_ctx *ctx, const double *e1, const double *e2,
   ctx->shell.clear();
   ctx->shell.push_back(make_int4(0, 0, 0, 0));
   ctx->shell.insert(ctx->shell.end(), dl.begin(), dl.end());
+  ctx->ref_shell = (int)ctx->shell.size();
   // The mixed kernel takes the image of a neighbour atom from its cell's
   // offset; that is the minimum image only when every cell offset a pair
   // within the cutoff can have, [-reach, reach] with reach taken before the
@@ -527,27 +543,26 @@ int build_box(pmnb_ctx *ctx, const double *e1, const double *e2,
   ctx->per_pair_wrap = 0;
   for (int k = 0; k < 3; k++)
     if (g.n[k] < 2 * reach[k] + 1) ctx->per_pair_wrap = 1;
-  // Tile path: its own grid of x/y columns at least one cutoff wide and z
-  // cells of about a quarter cutoff.  Used when the pair set does not depend
-  // on the cell grid (algorithm cutoff >= switching cutoff).
+  // Tile path: its own column grid, used when the pair set does not depend
+  // on the cell grid (algorithm cutoff >= switching cutoff) and type and atom
+  // index fit one word.  More LJ types than the pair kernel's LDS table holds
+  // are read from memory (pmnb_pair_path counts them to the general path).
   {
     const ForceParams P0 = make_params_for(ctx->prm, ctx->csf);
     const double rcp = std::sqrt(P0.cut2);
-    // the pair kernel packs type and sorted index into 32 bits and holds
-    // the LJ table in LDS
-    const bool packs = ctx->ntypes * ctx->ntypes <= kQLj &&
-                       ctx->n < (1 << kQTypeShift);
-    std::vector<int4> tshell;
-    TileRep rep{};
-    ctx->use_tile = ctx->prm.algorithm_cutoff >= rcp && packs &&
-                    make_tile_rep(b, rcp, tile_zfrac(ctx->prm), rep, tshell);
+    const bool packs = ctx->ntypes <= 256 && ctx->n < (1 << kQTypeShift);
+    ctx->use_tile = ctx->prm.algorithm_cutoff >= rcp && packs;
+    ctx->tile_types = ctx->ntypes * ctx->ntypes <= kQLj;
     if (ctx->use_tile) {
-      ctx->tile = rep.tg;
+      std::vector<int4> tshell;
+      TileRep rep{};
+      make_tile_rep(b, rcp, ctx->n, rep, tshell);
       g = rep.grid;
       ctx->shell = tshell;  // pair-set extraction walks it
       ctx->reps.assign(1, rep);
-      ctx->col_rep.assign(rep.ncol, 0);
-      ctx->ncol_total = rep.ncol;
+      ctx->bin_rep.clear();
+      ctx->nbin = rep.nbin;
+      ctx->nslots = rep.item_max;
     }
   }
   ctx->shell_off.clear();
@@ -560,6 +575,7 @@ int build_box(pmnb_ctx *ctx, const double *e1, const double *e2,
   ctx->grid = g;
   ctx->shell_uploaded = 0;
   ctx->rep_uploaded = 0;
+  ctx->counts_zero = false;  // more bins may be counted than were cleared
   ctx->have_box = true;
   return PMNB_OK;
 }
@@ -607,6 +623,8 @@ ForceParams make_params(const pmnb_ctx *ctx, uint32_t flags) {
   F.s3e = (float)P.sw_el.s3;
   F.alpha = (float)P.alpha;
   F.tapi = (float)P.two_alpha_pi;
+  F.pal = (float)(0.3275911 * P.alpha);
+  F.ea2 = (float)(-P.alpha * P.alpha * 1.4426950408889634);
   F.csf = (float)P.csf;
   F.same_switch = P.sw_lj.on2 == P.sw_el.on2 && P.sw_lj.cut2 == P.sw_el.cut2 &&
                   ctx->prm.elec_switch == PMNB_SWITCH_C2;
@@ -619,13 +637,15 @@ void launch_fill_i32(int *p, int n, int v, hipStream_t s) {
                        n, v);
 }
 
-// Atom slots per cell of the tile path's buckets: at least 4 times the mean
-// occupancy, a power of two in [64, kSortLds] (a fuller cell is read back
-// from the cell index of every atom instead).
-int tile_bucket_cap(int n, int nc) {
-  const long long mean = ((long long)n + std::max(nc, 1) - 1) / std::max(nc, 1);
+// Atom slots per bin of the tile path's buckets: twice the mean occupancy of
+// the fullest replica's bins and 64 more, a power of two up to kBinSort (a
+// fuller bin is read back from the bin index of every atom instead).
+int tile_bucket_cap(const std::vector<TileRep> &reps) {
+  long long mean = 0;
+  for (const TileRep &r : reps)
+    mean = std::max<long long>(mean, (r.natom + r.nbin - 1) / r.nbin);
   int cap = 64;
-  while (cap < 4 * mean && cap < kSortLds) cap *= 2;
+  while (cap < 2 * mean + 64 && cap < kBinSort) cap *= 2;
   return cap;
 }
 
@@ -633,7 +653,7 @@ int ensure_eval_buffers(pmnb_ctx *ctx) {
   const int n = ctx->n, nc = ctx->grid.ncell;
   const size_t N = (size_t)std::max(n, 1);
   HIPCHK(ctx->d_cell_of.ensure(N * sizeof(int)));
-  HIPCHK(ctx->d_count.ensure((size_t)nc * sizeof(int)));
+  HIPCHK(ctx->d_count.ensure((size_t)std::max(nc, ctx->nbin) * sizeof(int)));
   if (ctx->count_seen != ctx->d_count.p) {
     ctx->counts_zero = false;
     ctx->count_seen = ctx->d_count.p;
@@ -649,36 +669,21 @@ int ensure_eval_buffers(pmnb_ctx *ctx) {
   HIPCHK(ctx->d_sq.ensure(N * sizeof(double)));
   HIPCHK(ctx->d_smol.ensure(N * sizeof(int)));
   HIPCHK(ctx->d_scell.ensure(N * sizeof(int)));
+  const int slots = ctx->use_tile ? std::max(ctx->nslots, 1) : 0;
   if (ctx->use_tile) {
-    HIPCHK(ctx->d_srec.ensure(N * sizeof(int2)));
-    ctx->bucket_cap = tile_bucket_cap(n, nc);
-    HIPCHK(ctx->d_bucket.ensure((size_t)std::max(nc, 1) * ctx->bucket_cap *
+    HIPCHK(ctx->d_srec.ensure(N * sizeof(unsigned)));
+    HIPCHK(ctx->d_ccount.ensure((size_t)nc * sizeof(int)));
+    ctx->bucket_cap = tile_bucket_cap(ctx->reps);
+    HIPCHK(ctx->d_bucket.ensure((size_t)ctx->nbin * ctx->bucket_cap *
                                 sizeof(int)));
-    const int W = ctx->prm.precision == PMNB_PREC_FP64 ? FixWords<true>::W
-                                                        : FixWords<false>::W;
-    HIPCHK(ctx->d_ffix.ensure(N * W * sizeof(long long)));
-    if (ctx->ffix_zeroed != ctx->d_ffix.p) {
-      const long long nw = (long long)(ctx->d_ffix.bytes / sizeof(long long));
-      hipLaunchKernelGGL(k_zero_i64, dim3((unsigned)((nw + kBlock - 1) / kBlock)),
-                         dim3(kBlock), 0, ctx->stream, ctx->d_ffix.as<long long>(),
-                         nw);
-      HIPCHK(hipGetLastError());
-      HIPCHK(hipStreamSynchronize(ctx->stream));
-      ctx->ffix_zeroed = ctx->d_ffix.p;
-    }
   }
-  const int ncol_t = ctx->use_tile ? ctx->ncol_total : 0;
-  const int tile_items = n / kTileAtoms + ncol_t + 1;  // partial row per item
-  HIPCHK(ctx->d_partial.ensure((size_t)std::max(blocks_for(n), tile_items) *
+  HIPCHK(ctx->d_partial.ensure((size_t)std::max(blocks_for(n), slots) *
                                ACC_N * sizeof(double)));
-  HIPCHK(ctx->d_npairs.ensure(sizeof(unsigned long long)));
+  HIPCHK(ctx->d_npairs.ensure(2 * sizeof(unsigned long long)));
   if (!ctx->shell_uploaded) {
     HIPCHK(ctx->d_shell.ensure(ctx->shell.size() * sizeof(int4)));
     HIPCHK(hipMemcpy(ctx->d_shell.p, ctx->shell.data(),
                      ctx->shell.size() * sizeof(int4), hipMemcpyHostToDevice));
-    HIPCHK(ctx->d_box.ensure(sizeof(Box)));
-    HIPCHK(hipMemcpy(ctx->d_box.p, &ctx->box, sizeof(Box),
-                     hipMemcpyHostToDevice));
     HIPCHK(ctx->d_shell_off.ensure(ctx->shell_off.size() * sizeof(float4)));
     HIPCHK(hipMemcpy(ctx->d_shell_off.p, ctx->shell_off.data(),
                      ctx->shell_off.size() * sizeof(float4),
@@ -686,19 +691,19 @@ int ensure_eval_buffers(pmnb_ctx *ctx) {
     ctx->shell_uploaded = 1;
   }
   if (ctx->use_tile) {
-    const int ncol = ctx->ncol_total, nrep = (int)ctx->reps.size();
-    HIPCHK(ctx->d_items.ensure((size_t)(n / kTileAtoms + ncol + 1) *
-                               sizeof(int4)));
-    HIPCHK(ctx->d_nitems.ensure(sizeof(int)));
-    HIPCHK(ctx->d_rep_first.ensure((size_t)(nrep + 1) * sizeof(int)));
-    HIPCHK(ctx->d_colscan.ensure((size_t)3 * std::max(ncol, 1) * sizeof(int)));
+    const int nrep = (int)ctx->reps.size();
+    HIPCHK(ctx->d_items.ensure((size_t)slots * sizeof(int4)));
+    HIPCHK(ctx->d_rep_items.ensure((size_t)nrep * sizeof(int)));
     if (!ctx->rep_uploaded) {
       HIPCHK(ctx->d_reps.ensure((size_t)nrep * sizeof(TileRep)));
       HIPCHK(hipMemcpy(ctx->d_reps.p, ctx->reps.data(),
                        (size_t)nrep * sizeof(TileRep), hipMemcpyHostToDevice));
-      HIPCHK(ctx->d_col_rep.ensure((size_t)ncol * sizeof(int)));
-      HIPCHK(hipMemcpy(ctx->d_col_rep.p, ctx->col_rep.data(),
-                       (size_t)ncol * sizeof(int), hipMemcpyHostToDevice));
+      const size_t nb = ctx->bin_rep.size();
+      if (nb) {
+        HIPCHK(ctx->d_bin_rep.ensure(nb * sizeof(int)));
+        HIPCHK(hipMemcpy(ctx->d_bin_rep.p, ctx->bin_rep.data(),
+                         nb * sizeof(int), hipMemcpyHostToDevice));
+      }
       ctx->rep_uploaded = 1;
     }
   }
@@ -716,135 +721,92 @@ int ensure_eval_buffers(pmnb_ctx *ctx) {
   return PMNB_OK;
 }
 
-// Pair-kernel shapes of the tile path: {shell, buffered records per wave,
-// waves per SIMD the register allocation must allow}.  LDS per record: 32
-// bytes (mixed full shell), 56 (mixed half shell: + 3 fixed-point slots),
-// 64 / 112 (FP64), four waves per block.  Mixed: 0 full 256 / 3, 1 full
-// 128 / 4, 2 half 192 / 3; FP64: 0 full 192 / 3, 1 half 128 / 2.  A single
-// system uses its context's shape (0 unless set); the batch autotuner
-// chooses among them.
+// Pair-kernel shapes of the tile path, all with the same results bit for bit:
+// 0 by the number of work items (a block per item below kSplitItems), 1 a wave
+// per item, 2 (mixed) a block per item.  A single system uses its context's
+// shape (0 unless set); the batch autotuner chooses among them.
 constexpr int kMixedShapes = 3, kF64Shapes = 2;
 
-struct HalfArgs {
-  int max_items;   // upper bound of the work items
-  int grid_cap;    // persistent grid (batch): at most this many blocks
+struct PairArgs {
   hipStream_t s;
   const ForceParams *P;
   const Sorted *S;
   const TileRep *reps;
   const int4 *items;
-  const int *nitems;
-  long long *ffix;
-  double *partial;
+  int nslots, shape, grid_cap;
+  double *forces, *partial;
   unsigned long long *npairs;
-  int pstride;     // partial row stride (items)
-  bool single;     // one replica without wrapped x/y
-  TileGrid G;      // its column grid
   PairLog log;
-  double *forces;  // the caller's forces (k_tile adds into them)
-  // no energy or virial rows are read: the mixed kernels leave them out
-  bool forces_only = false;
+  int mode;        // PairMode
+  bool big_types;  // the LJ table is read from memory
 };
 
-// The single-system full-shell kernel adds its forces straight into the
-// caller's array; every other shape goes through the fixed-point array.
-bool direct_forces(const HalfArgs &a, int shape, bool mixed) {
-  return a.single && (mixed ? shape != 2 : shape != 1);
-}
-
-template <bool F64, int EL, int SW, int BUF, int OCC, bool HALF, bool LOG>
-void launch_half_log(const HalfArgs &a) {
-  if (a.single) {
-    // a multiple of 8 blocks (FP64 maps blocks to XCD-contiguous items)
-    const int nb = 8 * blocks_for(std::max(1, blocks_for(a.max_items,
-                                                         kTmWaves)), 8);
-    if constexpr (!HALF && !F64 && !LOG) {
-      if (a.forces_only)
-        hipLaunchKernelGGL((k_tile<false, EL, SW, 256, false, false>),
-                           dim3(nb), dim3(kBlock), 0, a.s, *a.P, *a.S, a.G,
-                           a.items, a.nitems, a.forces, a.partial, a.pstride,
-                           a.npairs, a.log);
-      else
-        hipLaunchKernelGGL((k_tile<false, EL, SW, 256, false>), dim3(nb),
-                           dim3(kBlock), 0, a.s, *a.P, *a.S, a.G, a.items,
-                           a.nitems, a.forces, a.partial, a.pstride,
-                           a.npairs, a.log);
-    } else if constexpr (!HALF)
-      hipLaunchKernelGGL((k_tile<F64, EL, SW, F64 ? 192 : 256, LOG>),
-                         dim3(nb), dim3(kBlock), 0, a.s, *a.P, *a.S, a.G,
-                         a.items, a.nitems, a.forces, a.partial, a.pstride,
-                         a.npairs, a.log);
-    else
-      hipLaunchKernelGGL((k_half<F64, EL, SW, BUF, OCC, false, HALF, LOG>),
-                         dim3(nb), dim3(kBlock), 0, a.s, *a.P, *a.S, a.reps,
-                         a.G, a.items, a.nitems, a.ffix, a.partial,
-                         a.pstride, a.npairs, a.log);
-    return;
-  }
-  int nb = blocks_for(a.max_items, kTmWaves);
+template <bool F64, int EL, int SW, int MODE, bool BIGT, bool LOG>
+void launch_pairs_as(const PairArgs &a) {
+  const bool split = a.shape == 2 || (a.shape == 0 && a.nslots < kSplitItems);
+  // a multiple of 8 blocks (blocks map to XCD-contiguous items)
+  int nb = split ? a.nslots : blocks_for(a.nslots, kTmWaves);
   if (a.grid_cap > 0) nb = std::min(nb, a.grid_cap);
-  nb = std::max(nb, 1);
-  if constexpr (!F64 && !LOG) {
-    if (a.forces_only) {
-      hipLaunchKernelGGL((k_half<false, EL, SW, BUF, OCC, true, HALF, false,
-                                 false>),
-                         dim3(nb), dim3(kBlock), 0, a.s, *a.P, *a.S, a.reps,
-                         a.G, a.items, a.nitems, a.ffix, a.partial, a.pstride,
-                         a.npairs, a.log);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((k_half<F64, EL, SW, BUF, OCC, true, HALF, LOG>),
-                     dim3(nb), dim3(kBlock), 0, a.s, *a.P, *a.S, a.reps, a.G,
-                     a.items, a.nitems, a.ffix, a.partial, a.pstride, a.npairs,
-                     a.log);
+  nb = 8 * std::max(1, blocks_for(nb, 8));
+  hipLaunchKernelGGL((k_pairs<F64, EL, SW, MODE, BIGT, LOG>), dim3(nb),
+                     dim3(kBlock), 0, a.s, *a.P, *a.S, a.reps, a.items,
+                     a.nslots, (int)split, a.forces, a.partial, a.nslots,
+                     a.npairs, a.log);
 }
 
-// The pair record (a.log.out set) runs the same kernel code with the
-// record compiled in.
-template <bool F64, int EL, int SW, int BUF, int OCC, bool HALF>
-void launch_half_shape(const HalfArgs &a) {
-  if (a.log.out) launch_half_log<F64, EL, SW, BUF, OCC, HALF, true>(a);
-  else launch_half_log<F64, EL, SW, BUF, OCC, HALF, false>(a);
+template <bool F64, int EL, int SW, bool BIGT>
+void launch_pairs_mode(const PairArgs &a) {
+  if (a.log.out) launch_pairs_as<F64, EL, SW, kForces, BIGT, true>(a);
+  else if (a.mode == kForces)
+    launch_pairs_as<F64, EL, SW, kForces, BIGT, false>(a);
+  else if (a.mode == kEnergies)
+    launch_pairs_as<F64, EL, SW, kEnergies, BIGT, false>(a);
+  else launch_pairs_as<F64, EL, SW, kMolVirial, BIGT, false>(a);
 }
 
 template <bool F64, int EL, int SW>
-void launch_half(int shape, const HalfArgs &a) {
-  if constexpr (F64) {
-    if (shape == 1) launch_half_shape<true, EL, SW, 128, 2, true>(a);
-    else launch_half_shape<true, EL, SW, 192, 3, false>(a);
-  } else {
-    if (shape == 1) launch_half_shape<false, EL, SW, 128, 4, false>(a);
-    else if (shape == 2) launch_half_shape<false, EL, SW, 192, 3, true>(a);
-    else launch_half_shape<false, EL, SW, 256, 3, false>(a);
-  }
+void launch_pairs_types(const PairArgs &a) {
+  // the FP64 kernel always reads the table from memory
+  if constexpr (F64) launch_pairs_mode<true, EL, SW, false>(a);
+  else if (a.big_types) launch_pairs_mode<false, EL, SW, true>(a);
+  else launch_pairs_mode<false, EL, SW, false>(a);
 }
 
 // Pair kernel of the tile path for the force's precision and functors.
-void launch_pair_half(bool mixed, int el, int sw, int shape,
-                      const HalfArgs &a) {
+void launch_pairs(bool mixed, int el, int sw, const PairArgs &a) {
   if (mixed) {
-    if (el == PMNB_ELEC_NONE) launch_half<false, 0, 0>(shape, a);
-    else if (el == PMNB_ELEC_COULOMB) launch_half<false, 1, 0>(shape, a);
-    else launch_half<false, 2, 0>(shape, a);
+    if (el == PMNB_ELEC_NONE) launch_pairs_types<false, 0, 0>(a);
+    else if (el == PMNB_ELEC_COULOMB) launch_pairs_types<false, 1, 0>(a);
+    else launch_pairs_types<false, 2, 0>(a);
   } else {
-    if (el == PMNB_ELEC_NONE) launch_half<true, 0, 0>(shape, a);
+    if (el == PMNB_ELEC_NONE) launch_pairs_types<true, 0, 0>(a);
     else if (el == PMNB_ELEC_COULOMB && sw == PMNB_SWITCH_C2)
-      launch_half<true, 1, 0>(shape, a);
-    else if (el == PMNB_ELEC_COULOMB) launch_half<true, 1, 1>(shape, a);
-    else if (sw == PMNB_SWITCH_C2) launch_half<true, 2, 0>(shape, a);
-    else launch_half<true, 2, 1>(shape, a);
+      launch_pairs_types<true, 1, 0>(a);
+    else if (el == PMNB_ELEC_COULOMB) launch_pairs_types<true, 1, 1>(a);
+    else if (sw == PMNB_SWITCH_C2) launch_pairs_types<true, 2, 0>(a);
+    else launch_pairs_types<true, 2, 1>(a);
   }
 }
 
-// Cell-list build on the device from d_pos (original order).
+// Exclusions as one code per atom: the class of partner a + d, |d| <= 15, in
+// bits 2 d + 30 and 2 d + 31, the atom itself marked FULL.  xown: per atom
+// {forward FULL, forward MODIFIED, reverse FULL, reverse MODIFIED} masks.
+__global__ void k_xcode(const unsigned long long *__restrict__ xown, int n,
+                        unsigned long long *__restrict__ xcode) {
+  const int a = blockIdx.x * blockDim.x + threadIdx.x;
+  if (a >= n) return;
+  unsigned long long c = 2ull << 30;
+  for (int d = -15; d <= 15; d++)
+    if (d)
+      c |= (unsigned long long)excl_own(xown + 4 * (size_t)a, d) << (30 + 2 * d);
+  xcode[a] = c;
+}
+
 // FP32 copy of the LJ table (T*T records {A, B, A14, B14}).
 __global__ void k_lj_to_f32(const double *__restrict__ lj, int n,
-                            float4 *__restrict__ ljf) {
+                            int elec, float4 *__restrict__ ljf) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n)
-    ljf[k] = make_float4((float)lj[4 * k], (float)lj[4 * k + 1],
-                         (float)lj[4 * k + 2], (float)lj[4 * k + 3]);
+  if (k < n) ljf[k] = lj_record(lj + 4 * k, elec);
 }
 
 template <typename R>
@@ -903,24 +865,22 @@ void launch_adj_t(int T, int max_items, hipStream_t s, const ForceParams &P,
 // (ctx_bufs, allocated by ensure_eval_buffers) or, for
 // pmnb_evaluate_device_noalloc, carved from the static scratch array.
 struct EvalBufs {
-  int *cell_of, *count, *start, *rank, *sorted;
-  int *bucket;  // tile path: cap atom slots per cell, in arrival order
+  int *cell_of;           // cell (tile path: bin) of each atom
+  int *count;             // atoms per cell (tile path: per bin)
+  int *start;             // first slot per cell
+  int *ccount;            // tile path: atoms per z cell
+  int *rank, *sorted;
+  int *bucket;            // tile path: cap atom slots per bin
   int cap;
   double *sx, *sy, *sz, *sq;
   float4 *loc;
   int *stype, *smol, *scell;
-  int2 *srec;
-  long long *ffix;
+  unsigned *srec;
   double *partial;
-  unsigned long long *npairs;
+  unsigned long long *npairs;  // [0] pairs, [1] visits of the tile path
   int4 *items;
-  int *nitems, *rep_first;
-  // 3 ints per global column (atoms, first atom, first item) for the
-  // column scan of many cells; null: the one-block scan
-  int *colscan;
+  int *rep_items;
   const TileRep *reps;
-  const int *col_rep;
-  const Box *box;
 };
 
 EvalBufs ctx_bufs(const pmnb_ctx *ctx) {
@@ -928,6 +888,7 @@ EvalBufs ctx_bufs(const pmnb_ctx *ctx) {
   B.cell_of = ctx->d_cell_of.as<int>();
   B.count = ctx->d_count.as<int>();
   B.start = ctx->d_start.as<int>();
+  B.ccount = ctx->d_ccount.as<int>();
   B.rank = ctx->d_fill.as<int>();
   B.sorted = ctx->d_sorted.as<int>();
   B.bucket = ctx->d_bucket.as<int>();
@@ -940,25 +901,20 @@ EvalBufs ctx_bufs(const pmnb_ctx *ctx) {
   B.stype = ctx->d_stype.as<int>();
   B.smol = ctx->d_smol.as<int>();
   B.scell = ctx->d_scell.as<int>();
-  B.srec = ctx->d_srec.as<int2>();
-  B.ffix = ctx->d_ffix.as<long long>();
+  B.srec = ctx->d_srec.as<unsigned>();
   B.partial = ctx->d_partial.as<double>();
   B.npairs = ctx->d_npairs.as<unsigned long long>();
   B.items = ctx->d_items.as<int4>();
-  B.nitems = ctx->d_nitems.as<int>();
-  B.rep_first = ctx->d_rep_first.as<int>();
-  B.colscan = ctx->d_colscan.as<int>();
+  B.rep_items = ctx->d_rep_items.as<int>();
   B.reps = ctx->d_reps.as<TileRep>();
-  B.col_rep = ctx->d_col_rep.as<int>();
-  B.box = ctx->d_box.as<Box>();
   return B;
 }
 
 // On the tile path every replica's cells are numbered from its offset
 // (ctx->grid.ncell is then the total).  counts_zero: B.count is known to
 // hold zeros (tile path only), so no clearing launch is needed; the
-// work-item kernel clears the pair counter.  assigned (tile path): the
-// counts, cells and ranks of these positions are already in B (written by
+// sorting kernel clears the counter of visits.  assigned (tile path): the
+// bin counts and buckets of these positions are already in B (written by
 // the integrator's kernel that produced them).  pos_copy (not with
 // assigned): d_pos is read once, by the cell assignment, which stores the
 // positions there for the kernels after it (d_pos may then be host memory
@@ -968,79 +924,49 @@ int build_cells(pmnb_ctx *ctx, const EvalBufs &B, const double *d_pos,
                 hipStream_t s, bool counts_zero = false,
                 bool assigned = false, double *pos_copy = nullptr) {
   const int n = ctx->n, nc = ctx->grid.ncell;
-  const TileRep *reps = B.reps;
-  const int *rep_of = ctx->batch ? ctx->d_rep_of.as<int>() : nullptr;
   int *rank = B.rank;
   ctx->counts_zero = false;
   assigned = assigned && ctx->use_tile;
-  if (!((counts_zero || assigned) && ctx->use_tile))
-    hipLaunchKernelGGL(k_clear, dim3(blocks_for(nc)), dim3(kBlock), 0, s,
-                       B.count, nc, B.npairs);
-  if (assigned) {
-    // cells and buckets came with the positions (the integrator's kernel)
-  } else if (n > 0 && ctx->use_tile) {
-    hipLaunchKernelGGL(k_assign_r<TileRep>, dim3(blocks_for(n)), dim3(kBlock),
-                       0, s, reps, rep_of, d_pos, n, B.cell_of,
-                       B.count, B.bucket, B.cap, pos_copy);
-  } else if (n > 0) {
+  if (!((counts_zero || assigned) && ctx->use_tile)) {
+    const int nk = ctx->use_tile ? ctx->nbin : nc;
+    hipLaunchKernelGGL(k_clear, dim3(blocks_for(nk)), dim3(kBlock), 0, s,
+                       B.count, nk, B.npairs);
+  }
+  if (ctx->use_tile) {
+    if (n > 0 && !assigned) {
+      const int *rep_of = ctx->batch ? ctx->d_rep_of.as<int>() : nullptr;
+      hipLaunchKernelGGL(k_assign_bins, dim3(blocks_for(n)), dim3(kBlock), 0, s,
+                         B.reps, rep_of, d_pos, n, B.cell_of, B.count, B.bucket,
+                         B.cap, pos_copy);
+      if (pos_copy) d_pos = pos_copy;
+    }
+    BinOut O{B.sorted, B.sx,   B.sy,    B.sz,     B.sq,    B.loc,
+             B.stype,  B.smol, B.scell, B.srec,   B.start, B.ccount,
+             B.items,  B.rep_items,     B.npairs + 1};
+    const int *bin_rep = ctx->batch ? ctx->d_bin_rep.as<int>() : nullptr;
+    hipLaunchKernelGGL(k_sort_bins, dim3(ctx->nbin), dim3(kBlock), 0, s, B.reps,
+                       bin_rep, d_pos, B.count, B.bucket, B.cap, B.cell_of,
+                       ctx->d_type.as<int>(), ctx->d_q.as<double>(),
+                       ctx->d_mol.as<int>(), O);
+    HIPCHK(hipGetLastError());
+    return PMNB_OK;
+  }
+  if (n > 0)
     hipLaunchKernelGGL(k_assign, dim3(blocks_for(n)), dim3(kBlock), 0, s,
                        ctx->box, ctx->grid, d_pos, n, B.cell_of,
                        B.count, rank, pos_copy);
-  }
-  if (pos_copy && !assigned) d_pos = pos_copy;
-  if (ctx->use_tile && B.colscan && nc > kScanCellsOneBlock) {
-    // starts and work items over the columns (many cells: a batch)
-    const int ncol = ctx->ncol_total;
-    int *col_n = B.colscan, *col_a0 = col_n + ncol, *col_i0 = col_a0 + ncol;
-    hipLaunchKernelGGL(k_col_atoms, dim3(blocks_for(ncol)), dim3(kBlock), 0,
-                       s, B.count, reps, B.col_rep, ncol, col_n);
-    hipLaunchKernelGGL(k_col_scan, dim3(1), dim3(1024), 0, s, col_n, ncol,
-                       (int)ctx->reps.size(), col_a0, col_i0, B.nitems,
-                       B.rep_first, B.npairs);
-    hipLaunchKernelGGL(k_col_fill, dim3(blocks_for(ncol)), dim3(kBlock), 0,
-                       s, B.count, B.start, reps, B.col_rep, ncol, col_a0,
-                       col_i0, B.items, B.rep_first);
-  } else if (ctx->use_tile) {
-    // starts and the work items of the tile path in one block
-    hipLaunchKernelGGL(k_scan_items, dim3(1), dim3(1024), 0, s,
-                       B.count, B.start, nc,
-                       reps, B.col_rep, ctx->ncol_total,
-                       (int)ctx->reps.size(), B.items,
-                       B.nitems, B.rep_first, B.npairs);
-  } else if (!ctx->use_tile) {
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s,
-                       B.count, B.start, nc);
-  }
-  if (n > 0 && !ctx->use_tile) {
+  if (pos_copy) d_pos = pos_copy;
+  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, B.count, B.start, nc);
+  if (n > 0) {
     hipLaunchKernelGGL(k_scatter, dim3(blocks_for(n)), dim3(kBlock), 0, s,
-                       B.cell_of, n, B.start,
-                       rank, B.sorted);
-  }
-  if (n > 0 && ctx->use_tile) {
-    hipLaunchKernelGGL(k_sort_gather_r<TileRep>,
-                       dim3(blocks_for(nc, kBlock / 64)), dim3(kBlock), 0, s,
-                       reps, rep_of, d_pos, B.start,
-                       B.count, nc, B.bucket, B.cap, B.cell_of, n,
-                       ctx->d_type.as<int>(),
-                       ctx->d_q.as<double>(), ctx->d_mol.as<int>(),
-                       B.sorted, B.sx,
-                       B.sy, B.sz,
-                       B.loc, B.stype,
-                       B.sq, B.smol,
-                       B.scell, B.srec);
-  } else if (n > 0) {
+                       B.cell_of, n, B.start, rank, B.sorted);
     hipLaunchKernelGGL(k_sort_cells, dim3(blocks_for(nc, kBlock / 64)),
-                       dim3(kBlock), 0, s,
-                       B.start, B.count, nc,
-                       B.sorted);
+                       dim3(kBlock), 0, s, B.start, B.count, nc, B.sorted);
     hipLaunchKernelGGL(k_gather, dim3(blocks_for(n)), dim3(kBlock), 0, s,
-                       ctx->box, ctx->grid, d_pos, B.sorted,
-                       B.cell_of, ctx->d_type.as<int>(),
-                       ctx->d_q.as<double>(), ctx->d_mol.as<int>(), n,
-                       B.sx, B.sy,
-                       B.sz, B.loc,
-                       B.stype, B.sq,
-                       B.smol, B.scell);
+                       ctx->box, ctx->grid, d_pos, B.sorted, B.cell_of,
+                       ctx->d_type.as<int>(), ctx->d_q.as<double>(),
+                       ctx->d_mol.as<int>(), n, B.sx, B.sy, B.sz, B.loc,
+                       B.stype, B.sq, B.smol, B.scell);
   }
   HIPCHK(hipGetLastError());
   return PMNB_OK;
@@ -1060,15 +986,15 @@ Sorted make_sorted(const pmnb_ctx *ctx, const EvalBufs &B,
   S.cell = B.scell;
   S.rec = B.srec;
   S.cstart = B.start;
-  S.ccount = B.count;
+  S.ccount = ctx->use_tile ? B.ccount : B.count;
   S.delta = ctx->d_shell.as<int4>();
   S.xfull = ctx->d_xfull.as<unsigned long long>();
   S.xmod = ctx->d_xmod.as<unsigned long long>();
   S.xown = ctx->d_xown.as<unsigned long long>();
+  S.xcode = S.xown + 4 * (size_t)ctx->n;
   S.lj = ctx->d_lj.as<double>();
   S.ljf = ctx->d_ljf.as<float4>();
   S.com = d_com;
-  S.box = B.box;
   return S;
 }
 
@@ -1081,17 +1007,15 @@ int check_ready(pmnb_ctx *ctx) {
   return PMNB_OK;
 }
 
-// own: B are the context's buffers (not the static scratch), whose cell
+// own: B are the context's buffers (not the static scratch), whose bin
 // counts the finish kernel leaves cleared for the next evaluation.  fresh:
-// on the tile path the forces and the 20 output doubles are written, not
+// on the tile path the forces and the output doubles are written, not
 // added to (the caller's arrays need no clearing).  np_out (tile path):
 // the finish kernel also stores the pair count there.  finish_skipped
-// (given): no energies or virial are wanted in d_out; the mixed pair
-// kernels form none, a single-system tile evaluation whose pair kernel
-// wrote the forces itself launches no finish kernel (the caller clears the
-// cell counts before the next evaluation), and a batch's finish kernel
-// sums no energies; *finish_skipped tells whether the finish was left
-// out.
+// (given): no energies or virial are wanted in d_out; on the tile path the
+// pair kernel forms none and no finish kernel is launched (the caller clears
+// the bin counts before the next evaluation); *finish_skipped tells whether
+// the finish was left out.
 int run_device_bufs(pmnb_ctx *ctx, const EvalBufs &B, const double *d_pos,
                     double *d_forces, double *d_out, const double *d_com,
                     uint32_t flags, hipStream_t s, bool own,
@@ -1121,7 +1045,10 @@ int run_device_bufs(pmnb_ctx *ctx, const EvalBufs &B, const double *d_pos,
   rc = build_cells(ctx, B, d_pos, s, own && ctx->counts_zero, assigned,
                    pos_copy);
   if (rc) return rc;
-  if (own) ctx->last_np = B.npairs;  // not the shared scratch's counter
+  if (own) {  // not the shared scratch's counter
+    ctx->last_np = B.npairs + (ctx->use_tile ? 1 : 0);
+    ctx->last_np_per = ctx->use_tile ? 2 : 1;
+  }
   const ForceParams P = make_params(ctx, flags);
   const Sorted S = make_sorted(ctx, B, d_com);
   const int nb = std::max(1, blocks_for(ctx->n));
@@ -1135,55 +1062,30 @@ int run_device_bufs(pmnb_ctx *ctx, const EvalBufs &B, const double *d_pos,
   unsigned *lst = ctx->d_list.as<unsigned>();
   int *cnt = ctx->d_ncount.as<int>();
   if (ctx->use_tile) {
-    const int ncol = ctx->ncol_total, nrep = (int)ctx->reps.size();
-    const int max_items = ctx->n / kTileAtoms + ncol + 1;
-    const TileRep *reps = B.reps;
-    int4 *items = B.items;
-    int *nitems = B.nitems;
-    int *rep_first = B.rep_first;
-    long long *ffix = B.ffix;
-    bool direct = false;
+    const int nrep = (int)ctx->reps.size();
     if (ev_built) HIPCHK(hipEventRecord(ev_built, s));
     if (ctx->n > 0) {
-      const bool single = !ctx->batch && nrep == 1 &&
-                          !ctx->reps[0].wrap[0] && !ctx->reps[0].wrap[1];
-      HalfArgs a{max_items, ctx->grid_cap, s, &P, &S, reps, items, nitems,
-                 ffix, part, np, max_items, single, ctx->tile, ctx->plog,
-                 d_forces};
-      // no energies wanted: the mixed kernels leave them out, in the full
-      // shell of 256 records whatever shape the evaluations with energies
-      // use (114 VGPRs, four waves per SIMD; the half shell's fixed-point
-      // slots in LDS hold it to three: 3.8 against 4.8 ms per dynamics step
-      // of the 512 water replicas).  A single system's kernel then needs
-      // no finish; a batch's finish still converts the forces but sums no
-      // energies.
-      a.forces_only = finish_skipped != nullptr;
-      const int shape = a.forces_only && mixed ? 0 : ctx->shape;
-      direct = direct_forces(a, shape, mixed);
-      launch_pair_half(mixed, el, sw, shape, a);
+      PairArgs a{s, &P, &S, B.reps, B.items, ctx->nslots, ctx->shape,
+                 ctx->grid_cap, d_forces, part, B.npairs + 1, ctx->plog,
+                 finish_skipped ? kForces
+                 : (flags & PMNB_FLAG_MOLVIRIAL) ? kMolVirial : kEnergies,
+                 !ctx->tile_types};
+      launch_pairs(mixed, el, sw, a);
     }
     if (ev_stop) HIPCHK(hipEventRecord(ev_stop, s));
+    HIPCHK(hipGetLastError());
     if (finish_skipped) {
-      *finish_skipped = direct;
-      if (direct) return PMNB_OK;
+      *finish_skipped = true;
+      return PMNB_OK;
     }
-    // fixed-point forces into the caller's array (unless the pair kernel
-    // added them itself), per-replica sums
-    // and the cell counts cleared for the next evaluation
-    const int ab = direct ? 0 : blocks_for(ctx->n, 1024);
-    const int rb = finish_skipped ? 0 : nrep * ACC_N, nc = ctx->grid.ncell;
+    // per-replica sums and the bin counts cleared for the next evaluation
+    const int rb = nrep * ACC_N;
     const int fresh = (flags & kFlagFresh) ? 1 : 0;
-    const dim3 fg((unsigned)(ab + rb + blocks_for(nc, 1024)));
-    if (mixed)
-      hipLaunchKernelGGL(k_half_finish<false>, fg, dim3(1024), 0, s, ffix,
-                         S.atom, ctx->n, d_forces, ab, part, max_items,
-                         rep_first, d_out, rb, B.count, nc, fresh, np,
-                         np_out);
-    else
-      hipLaunchKernelGGL(k_half_finish<true>, fg, dim3(1024), 0, s, ffix,
-                         S.atom, ctx->n, d_forces, ab, part, max_items,
-                         rep_first, d_out, rb, B.count, nc, fresh, np,
-                         np_out);
+    hipLaunchKernelGGL(k_pairs_finish,
+                       dim3((unsigned)(rb + blocks_for(ctx->nbin, 1024))),
+                       dim3(1024), 0, s, part, ctx->nslots, B.reps, B.rep_items,
+                       d_out, rb, B.count, ctx->nbin, fresh, B.npairs + 1,
+                       np_out);
     HIPCHK(hipGetLastError());
     if (own) ctx->counts_zero = true;
     return PMNB_OK;
@@ -1407,8 +1309,7 @@ int pmnb_set_topology(pmnb_ctx *ctx, int32_t n_atoms, const int32_t *type,
       const int lo = std::min(i, j), hi = std::max(i, j);
       const double *src = lj + 4 * ((size_t)lo * T + hi);
       for (int k = 0; k < 4; k++) ljd[4 * ((size_t)i * T + j) + k] = src[k];
-      ljf[(size_t)i * T + j] = make_float4((float)src[0], (float)src[1],
-                                           (float)src[2], (float)src[3]);
+      ljf[(size_t)i * T + j] = lj_record(src, ctx->prm.elec);
     }
   const size_t N = (size_t)std::max(n_atoms, 1);
   HIPCHK(ctx->d_type.ensure(N * sizeof(int)));
@@ -1416,7 +1317,8 @@ int pmnb_set_topology(pmnb_ctx *ctx, int32_t n_atoms, const int32_t *type,
   HIPCHK(ctx->d_mol.ensure(N * sizeof(int)));
   HIPCHK(ctx->d_xfull.ensure(N * sizeof(unsigned long long)));
   HIPCHK(ctx->d_xmod.ensure(N * sizeof(unsigned long long)));
-  HIPCHK(ctx->d_xown.ensure(N * 4 * sizeof(unsigned long long)));
+  // the masks (4 words an atom), then the codes (one)
+  HIPCHK(ctx->d_xown.ensure(N * 5 * sizeof(unsigned long long)));
   HIPCHK(ctx->d_lj.ensure(ljd.size() * sizeof(double)));
   HIPCHK(ctx->d_ljf.ensure(ljf.size() * sizeof(float4)));
   if (n_atoms > 0) {
@@ -1432,6 +1334,12 @@ int pmnb_set_topology(pmnb_ctx *ctx, int32_t n_atoms, const int32_t *type,
                      hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(ctx->d_xown.p, xown.data(), (size_t)n_atoms * 32,
                      hipMemcpyHostToDevice));
+    unsigned long long *x = ctx->d_xown.as<unsigned long long>();
+    hipLaunchKernelGGL(k_xcode, dim3(blocks_for(n_atoms)), dim3(kBlock), 0,
+                       (hipStream_t) nullptr, x, n_atoms,
+                       x + 4 * (size_t)n_atoms);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(nullptr));
   }
   HIPCHK(hipMemcpy(ctx->d_lj.p, ljd.data(), ljd.size() * sizeof(double),
                    hipMemcpyHostToDevice));
@@ -1622,6 +1530,8 @@ int pmnb_pairset(pmnb_ctx *ctx, const double *positions, int32_t *pairs,
   HIPCHK(hipMemcpyAsync(&np, ctx->d_npairs.p, sizeof np, hipMemcpyDeviceToHost,
                         s));
   HIPCHK(hipStreamSynchronize(s));
+  ctx->last_np = ctx->d_npairs.as<unsigned long long>();
+  ctx->last_np_per = 1;
   *n_pairs = (int64_t)np;
   if (!pairs) return PMNB_OK;
   if ((long long)np > cap)
@@ -1745,9 +1655,11 @@ int pmnb_kernel_timing(pmnb_ctx *ctx, int32_t enable, double *ms,
 int pmnb_pair_path(const pmnb_ctx *ctx, int32_t *path) {
   if (!ctx || !path) return PMNB_ERR_ARG;
   if (!ctx->have_box || !ctx->have_topo) return PMNB_ERR_STATE;
-  const bool list = ctx->use_list && ctx->n < (1 << kEntryAtomBits);
-  *path = ctx->use_tile ? PMNB_PATH_TILE : (list ? PMNB_PATH_LIST
-                                                 : PMNB_PATH_SCAN);
+  const bool list = ctx->ref_shell <= kMaxShell &&
+                    ctx->n < (1 << kEntryAtomBits);
+  *path = ctx->use_tile && ctx->tile_types ? PMNB_PATH_TILE
+          : list                           ? PMNB_PATH_LIST
+                                           : PMNB_PATH_SCAN;
   return PMNB_OK;
 }
 
@@ -1759,7 +1671,7 @@ int pmnb_last_pair_count(pmnb_ctx *ctx, int64_t *n_pairs) {
     HIPCHK(hipDeviceSynchronize());
     unsigned long long np = 0;
     HIPCHK(hipMemcpy(&np, ctx->last_np, sizeof np, hipMemcpyDeviceToHost));
-    ctx->last_pairs = (long long)np;
+    ctx->last_pairs = (long long)np / ctx->last_np_per;
   }
   *n_pairs = ctx->last_pairs;
   return PMNB_OK;
@@ -1774,19 +1686,18 @@ void pmnb_destroy(pmnb_ctx *ctx) {
   (void)hipSetDevice(ctx->prm.device);
   (void)hipStreamSynchronize(ctx->stream);
   DevBuf *bufs[] = {&ctx->d_type, &ctx->d_q, &ctx->d_mol, &ctx->d_xfull,
-                    &ctx->d_xmod, &ctx->d_xown, &ctx->d_lj, &ctx->d_ljf, &ctx->d_pos,
+                    &ctx->d_xmod, &ctx->d_xown, &ctx->d_lj,
+                    &ctx->d_ljf, &ctx->d_pos,
                     &ctx->d_force, &ctx->d_out, &ctx->d_com, &ctx->d_cell_of,
                     &ctx->d_count, &ctx->d_start, &ctx->d_fill, &ctx->d_sorted,
                     &ctx->d_sx, &ctx->d_sy, &ctx->d_sz, &ctx->d_loc,
                     &ctx->d_stype, &ctx->d_sq, &ctx->d_smol, &ctx->d_scell,
                     &ctx->d_srec, &ctx->d_shell, &ctx->d_partial, &ctx->d_npairs,
                     &ctx->d_pairs, &ctx->d_list, &ctx->d_ncount,
-                    &ctx->d_partial2, &ctx->d_shell_off, &ctx->d_box,
-                    &ctx->d_items,
-                    &ctx->d_nitems, &ctx->d_reps, &ctx->d_col_rep,
-                    &ctx->d_rep_first, &ctx->d_rep_of, &ctx->d_partial_lj,
-                    &ctx->d_ffix, &ctx->d_plog, &ctx->d_plog_count,
-                    &ctx->d_bucket, &ctx->d_colscan};
+                    &ctx->d_partial2, &ctx->d_shell_off, &ctx->d_items,
+                    &ctx->d_reps, &ctx->d_bin_rep, &ctx->d_rep_items,
+                    &ctx->d_rep_of, &ctx->d_partial_lj, &ctx->d_plog,
+                    &ctx->d_plog_count, &ctx->d_bucket, &ctx->d_ccount};
   for (DevBuf *b : bufs) b->release();
   for (hipEvent_t e : ctx->ev_pool) (void)hipEventDestroy(e);
   for (hipEvent_t e : ctx->h_ev)
@@ -1810,7 +1721,8 @@ int pmnb_set_parameters_device(pmnb_ctx *ctx, const double *d_lj,
     HIPCHK(hipMemcpyAsync(ctx->d_lj.p, d_lj, (size_t)nlj * 4 * sizeof(double),
                           hipMemcpyDeviceToDevice, s));
     hipLaunchKernelGGL(k_lj_to_f32, dim3(blocks_for(nlj)), dim3(kBlock), 0, s,
-                       ctx->d_lj.as<double>(), nlj, ctx->d_ljf.as<float4>());
+                       ctx->d_lj.as<double>(), nlj, ctx->prm.elec,
+                       ctx->d_ljf.as<float4>());
   }
   if (d_scaled_charge && ctx->n > 0)
     HIPCHK(hipMemcpyAsync(ctx->d_q.p, d_scaled_charge,
@@ -1828,7 +1740,7 @@ int pmnb_adjoint_device(pmnb_ctx *ctx, const double *d_positions,
   if (rc) return rc;
   if (!d_positions || !d_grad_forces)
     return fail(ctx, PMNB_ERR_ARG, "null device pointer");
-  if (!ctx->use_tile)
+  if (!ctx->use_tile || !ctx->tile_types)
     return fail(ctx, PMNB_ERR_UNSUPPORTED,
                 "the adjoint needs the tile path (algorithm cutoff >= "
                 "switching cutoff, at most 8 LJ types)");
@@ -1841,8 +1753,7 @@ int pmnb_adjoint_device(pmnb_ctx *ctx, const double *d_positions,
   hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
   rc = ensure_eval_buffers(ctx);
   if (rc) return rc;
-  const int ncol = ctx->ncol_total, nrep = (int)ctx->reps.size();
-  const int max_items = ctx->n / kTileAtoms + ncol + 1;
+  const int max_items = std::max(ctx->nslots, 1);
   HIPCHK(ctx->d_partial_lj.ensure((size_t)max_items * 10 * 4 *
                                   sizeof(double)));
   rc = build_cells(ctx, ctx_bufs(ctx), d_positions, s);
@@ -1851,13 +1762,14 @@ int pmnb_adjoint_device(pmnb_ctx *ctx, const double *d_positions,
   const Sorted S = make_sorted(ctx, ctx_bufs(ctx), nullptr);
   const TileRep *reps = ctx->d_reps.as<TileRep>();
   int4 *items = ctx->d_items.as<int4>();
-  int *nitems = ctx->d_nitems.as<int>();
-  // work items: built with the cell starts
+  int *nitems = ctx->d_rep_items.as<int>();
   if (ctx->n > 0) {
     const bool f64 = ctx->prm.precision == PMNB_PREC_FP64;
     const int el = ctx->prm.elec, T = ctx->ntypes;
     double *plj = ctx->d_partial_lj.as<double>();
     unsigned long long *np = ctx->d_npairs.as<unsigned long long>();
+    ctx->last_np = np;
+    ctx->last_np_per = 1;
 #define PMNB_ADJ(F, E)                                                        \
   launch_adj_t<F, E>(T, max_items, s, P, S, reps, items, nitems,              \
                      d_grad_forces, d_grad_positions, d_grad_charges, plj,    \
@@ -1980,35 +1892,41 @@ int batch_finalize(pmnb_batch *b) {
     return fail(ctx, PMNB_ERR_UNSUPPORTED, "a batch holds at most %d LJ types",
                 8);
   ctx->reps.clear();
-  ctx->col_rep.clear();
-  long long cells = 0;
-  int cols = 0;
+  ctx->bin_rep.clear();
+  long long cells = 0, bins = 0, slots = 0;
   std::vector<int4> shell;
-  for (int r = 0; r < R; r++) {
+  for (int r = 0, a = 0; r < R; r++) {
     TileRep rep{};
-    if (!make_tile_rep(b->boxes[r], rcp, tile_zfrac(ctx->prm), rep, shell))
-      return fail(ctx, PMNB_ERR_UNSUPPORTED, "replica %d grid too large", r);
+    int na = 0;
+    while (a + na < (int)b->rep_of.size() && b->rep_of[a + na] == r) na++;
+    make_tile_rep(b->boxes[r], rcp, na, rep, shell);
     rep.cell_off = (int)cells;
-    rep.col_off = cols;
+    rep.bin_off = (int)bins;
+    rep.atom_off = a;
+    rep.item_off = (int)slots;
+    a += na;
     cells += rep.grid.ncell;
-    cols += rep.ncol;
+    bins += rep.nbin;
+    slots += rep.item_max;
     if (cells >= (1ll << 28))
       return fail(ctx, PMNB_ERR_UNSUPPORTED, "batch cell grid too large");
-    for (int c = 0; c < rep.ncol; c++) ctx->col_rep.push_back(r);
+    ctx->bin_rep.insert(ctx->bin_rep.end(), rep.nbin, r);
     ctx->reps.push_back(rep);
   }
+  ctx->nbin = (int)bins;
+  ctx->nslots = (int)slots;
   ctx->use_tile = true;
+  ctx->tile_types = true;
   ctx->use_list = false;
   ctx->batch = true;
-  ctx->tile = ctx->reps[0].tg;
   ctx->box = ctx->reps[0].box;
   ctx->grid = Grid{};
   ctx->grid.ncell = (int)cells;
-  ctx->ncol_total = cols;
   ctx->shell.assign(1, make_int4(0, 0, 0, 0));
   ctx->shell_off.assign(1, make_float4(0.f, 0.f, 0.f, 0.f));
   ctx->shell_uploaded = 0;
   ctx->rep_uploaded = 0;
+  ctx->counts_zero = false;  // more bins may be counted than were cleared
   ctx->have_box = true;
   HIPCHK(hipSetDevice(ctx->prm.device));
   HIPCHK(ctx->d_rep_of.ensure(b->rep_of.size() * sizeof(int)));
@@ -2066,9 +1984,9 @@ int pmnb_batch_run_graph(pmnb_batch *b, const double *d_positions,
     drop_graph(b);
     if (ctx->timing)
       return fail(ctx, PMNB_ERR_STATE, "kernel timing is on: no capture");
-    // one step: clear forces and outputs, then the whole evaluation; the
-    // buffers are allocated by batch_finalize, so nothing allocates here
-    const long long n3 = 3ll * ctx->n, no = 20ll * (long long)ctx->reps.size();
+    // one step: the whole evaluation, forces and outputs written instead of
+    // added to; the buffers are allocated by batch_finalize, so nothing
+    // allocates here
     if (!b->cap_stream)
       HIPCHK(hipStreamCreateWithFlags(&b->cap_stream, hipStreamNonBlocking));
     hipStream_t cs = b->cap_stream;
@@ -2076,11 +1994,8 @@ int pmnb_batch_run_graph(pmnb_batch *b, const double *d_positions,
     // evaluation clears the cell counts itself
     ctx->counts_zero = false;
     HIPCHK(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    hipLaunchKernelGGL(k_zero_f64, dim3((unsigned)((n3 + kBlock - 1) / kBlock)),
-                       dim3(kBlock), 0, cs, d_forces, n3);
-    hipLaunchKernelGGL(k_zero_f64, dim3((unsigned)((no + kBlock - 1) / kBlock)),
-                       dim3(kBlock), 0, cs, d_out, no);
-    rc = run_device(ctx, d_positions, d_forces, d_out, nullptr, flags, cs);
+    rc = run_device(ctx, d_positions, d_forces, d_out, nullptr, flags, cs,
+                    true);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(cs, &g);
     ctx->counts_zero = false;  // the captured work has not run
@@ -2098,6 +2013,8 @@ int pmnb_batch_run_graph(pmnb_batch *b, const double *d_positions,
     b->gshape = ctx->shape;
     b->gcap = ctx->grid_cap;
   }
+  ctx->last_np = ctx->d_npairs.as<unsigned long long>() + 1;
+  ctx->last_np_per = 2;
   for (int k = 0; k < n_steps; k++) HIPCHK(hipGraphLaunch(b->gexec, s));
   return PMNB_OK;
 }
@@ -2265,6 +2182,7 @@ LfDev lf_dev(pmnb_leapfrog *lf, double *x, double *v, double *f,
   d.n_free = lf->nf;
   d.ngb = lf->ngb;
   d.n_cons = lf->n_cons;
+  d.z_force = lf->ctx->use_tile ? 0 : 1;
   d.n_out = lf->n_out + ((lf->n_bonds + lf->n_angles) > 0 ? 2 : 0);
   d.reps = lf->reps.as<LfRep>();
   d.blk_rep = lf->blk_rep.as<int>();
@@ -2335,7 +2253,7 @@ int lf_flush(pmnb_leapfrog *lf, LfKernel &k, const LfDev &d0, hipStream_t s) {
   if (zc) {
     // the evaluation before launched no finish kernel: clear its counts
     d.z_count = ctx->d_count.as<int>();
-    d.z_nc = ctx->grid.ncell;
+    d.z_nc = ctx->nbin;
   }
   const long long call = k.apply != kStNone ? lf->calls++ : -1;
   const long long sc_apply = lf->scalls[k.apply];
@@ -2395,8 +2313,8 @@ int lf_calc_forces(pmnb_leapfrog *lf, const double *d_pos, double *d_force,
   bool skipped = false;
   const uint32_t fl =
       energies ? flags : flags & ~(PMNB_FLAG_VIRIAL | PMNB_FLAG_MOLVIRIAL);
-  int rc = run_device(ctx, d_pos, d_force, d_out, nullptr, fl, s, false,
-                      assigned, energies ? nullptr : &skipped);
+  int rc = run_device(ctx, d_pos, d_force, d_out, nullptr, fl, s,
+                      ctx->use_tile, assigned, energies ? nullptr : &skipped);
   lf->zero_counts = skipped;
   if (rc) return rc;
   if (lf->pme) {
@@ -2701,7 +2619,7 @@ int pmnb_lf_run_device(pmnb_leapfrog *lf, double *d_positions,
     const EvalBufs B = ctx_bufs(ctx);
     da.c_reps = B.reps;
     da.c_rep_of = ctx->batch ? ctx->d_rep_of.as<int>() : nullptr;
-    da.c_cell_of = B.cell_of;
+    da.c_bin_of = B.cell_of;
     da.c_count = B.count;
     da.c_bucket = B.bucket;
     da.c_cap = B.cap;
@@ -2711,8 +2629,8 @@ int pmnb_lf_run_device(pmnb_leapfrog *lf, double *d_positions,
     if (assign && !ctx->counts_zero) {
       // (also what a clearing left to this kernel would have done: the
       // assignment's atomics must not race a clearing in the same kernel)
-      hipLaunchKernelGGL(k_clear, dim3(blocks_for(ctx->grid.ncell)),
-                         dim3(kBlock), 0, s, da.c_count, ctx->grid.ncell,
+      hipLaunchKernelGGL(k_clear, dim3(blocks_for(ctx->nbin)),
+                         dim3(kBlock), 0, s, da.c_count, ctx->nbin,
                          ctx->d_npairs.as<unsigned long long>());
       lf->zero_counts = false;
     }
@@ -2871,7 +2789,8 @@ int pmnb_lf_forces_device(pmnb_leapfrog *lf, const double *d_positions,
   HIPCHK(hipSetDevice(ctx->prm.device));
   hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
   if (lf->n == 0) return PMNB_OK;
-  launch_fill_i32(reinterpret_cast<int *>(d_forces), lf->n * 6, 0, s);
+  if (!ctx->use_tile)  // the tile path writes the forces
+    launch_fill_i32(reinterpret_cast<int *>(d_forces), lf->n * 6, 0, s);
   launch_fill_i32(reinterpret_cast<int *>(d_out),
                   2 * (lf->n_out + ((lf->n_bonds + lf->n_angles) > 0 ? 2 : 0)),
                   0, s);
@@ -2952,6 +2871,10 @@ int pmnb_lf_run_graph(pmnb_leapfrog *lf, double *d_positions,
     std::copy(ctx->box_key, ctx->box_key + 12, lf->gbox);
     lf->gshape = ctx->shape;
     lf->gcap = ctx->grid_cap;
+  }
+  if (ctx->use_tile) {
+    ctx->last_np = ctx->d_npairs.as<unsigned long long>() + 1;
+    ctx->last_np_per = 2;
   }
   for (int k = 0; k < n_replays; k++) HIPCHK(hipGraphLaunch(lf->gexec, s));
   return PMNB_OK;
@@ -3635,7 +3558,7 @@ int pmnb_lf_set_kspace(pmnb_leapfrog *lf, pmnb_pme *pme, pmnb_ewald *ewald) {
 // --------------------------------------------- evaluation without allocation
 // pmnb_evaluate_device_noalloc keeps every per-evaluation array of the tile
 // path (cell counts and starts, the sorted structure of arrays, work items,
-// partial sums, the fixed-point force array, the system's grid and box) in
+// partial sums, the system's grid and box) in
 // `scratch`, a file-scope device array of kScratchBytes that each GPU
 // holds for the life of the process.  Its device address on each GPU is
 // looked up once, by pmnb_create with that device current; host code uses
@@ -3679,23 +3602,20 @@ struct Carve {
 };
 
 // The tile path's arrays for one system of ctx, carved from `base`.
-EvalBufs carve_bufs(const pmnb_ctx *ctx, unsigned char *base, size_t &bytes,
-                    long long &nfix) {
+EvalBufs carve_bufs(const pmnb_ctx *ctx, unsigned char *base, size_t &bytes) {
   Carve c{base};
   const size_t N = (size_t)std::max(ctx->n, 1);
   const size_t nc = (size_t)std::max(ctx->grid.ncell, 1);
-  const int W = ctx->prm.precision == PMNB_PREC_FP64 ? FixWords<true>::W
-                                                      : FixWords<false>::W;
-  const size_t items = (size_t)(ctx->n / kTileAtoms + ctx->ncol_total + 1);
+  const size_t slots = (size_t)std::max(ctx->nslots, 1);
   EvalBufs B{};
-  B.ffix = c.take<long long>(N * W);
   B.cell_of = c.take<int>(N);
-  B.count = c.take<int>(nc);
+  B.count = c.take<int>((size_t)ctx->nbin);
   B.start = c.take<int>(nc);
+  B.ccount = c.take<int>(nc);
   B.rank = nullptr;  // the tile path fills bucket rows instead
   B.sorted = c.take<int>(N);
-  B.cap = tile_bucket_cap(ctx->n, (int)nc);
-  B.bucket = c.take<int>(nc * (size_t)B.cap);
+  B.cap = tile_bucket_cap(ctx->reps);
+  B.bucket = c.take<int>((size_t)ctx->nbin * B.cap);
   B.sx = c.take<double>(N);
   B.sy = c.take<double>(N);
   B.sz = c.take<double>(N);
@@ -3704,34 +3624,39 @@ EvalBufs carve_bufs(const pmnb_ctx *ctx, unsigned char *base, size_t &bytes,
   B.stype = c.take<int>(N);
   B.smol = c.take<int>(N);
   B.scell = c.take<int>(N);
-  B.srec = c.take<int2>(N);
-  B.partial = c.take<double>(items * ACC_N);
-  B.npairs = c.take<unsigned long long>(1);
-  B.items = c.take<int4>(items);
-  B.nitems = c.take<int>(1);
-  B.rep_first = c.take<int>(2);
+  B.srec = c.take<unsigned>(N);
+  B.partial = c.take<double>(slots * ACC_N);
+  B.npairs = c.take<unsigned long long>(2);
+  B.items = c.take<int4>(slots);
+  B.rep_items = c.take<int>(1);
   B.reps = c.take<TileRep>(1);
-  B.col_rep = c.take<int>((size_t)std::max(ctx->ncol_total, 1));
-  B.box = c.take<Box>(1);
   bytes = c.off;
-  nfix = (long long)(N * W);
   return B;
 }
 
-// Writes the system's grid and box into the scratch, marks every column as
-// replica 0 and clears the fixed-point force array (the previous call on
-// this GPU may have been another system's, or may have stopped early).
-__global__ void k_scratch_setup(TileRep rep, Box box, TileRep *d_rep,
-                                Box *d_box, int *col_rep, int ncol,
-                                long long *ffix, long long nfix) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long stride = (long long)gridDim.x * blockDim.x;
-  if (t == 0) {
-    *d_rep = rep;
-    *d_box = box;
-  }
-  for (long long k = t; k < ncol; k += stride) col_rep[k] = 0;
-  for (long long k = t; k < nfix; k += stride) ffix[k] = 0;
+// The bytes the documented limit counts for one system: 100 (FP64 124) per
+// atom, 128 per 16 atoms and column and, per cell of a grid of columns one
+// cutoff wide with z cells of a third (FP64 a quarter) of the cutoff, 8 and 4
+// per bucket slot, at least 4 times the mean occupancy.
+size_t scratch_limit_bytes(const pmnb_ctx *ctx) {
+  const bool mixed = ctx->prm.precision == PMNB_PREC_MIXED;
+  const double rcp = std::sqrt(make_params_for(ctx->prm, ctx->csf).cut2);
+  auto cells = [&](int k, double w) {
+    return std::max(1.0, std::floor(ctx->box.H[k] / w));
+  };
+  const double ncol = cells(0, rcp) * cells(1, rcp);
+  const double nc = ncol * cells(2, mixed ? rcp / 3.0 : 0.25 * rcp);
+  const double n = ctx->n;
+  double cap = 64;
+  while (cap < 4 * std::ceil(n / nc) && cap < 512) cap *= 2;
+  const double b = n * (mixed ? 100 : 124) + 128 * (n / 16 + ncol) +
+                   nc * (8 + 4 * cap);
+  return b < 1e18 ? (size_t)b : (size_t)1e18;
+}
+
+// Writes the system's grid and box into the scratch.
+__global__ void k_scratch_setup(TileRep rep, TileRep *d_rep) {
+  if (threadIdx.x == 0) *d_rep = rep;
 }
 
 }  // namespace
@@ -3744,7 +3669,8 @@ int pmnb_evaluate_device_noalloc(pmnb_ctx *ctx, const double *d_positions,
                                  void *stream) {
   int rc = check_ready(ctx);
   if (rc) return rc;
-  if (ctx->batch || !ctx->use_tile || ctx->reps.size() != 1)
+  if (ctx->batch || !ctx->use_tile || !ctx->tile_types ||
+      ctx->reps.size() != 1)
     return fail(ctx, PMNB_ERR_UNSUPPORTED,
                 "the allocation-free evaluation covers one system on the tile "
                 "path (algorithm cutoff >= switching cutoff, at most 8 LJ "
@@ -3769,23 +3695,18 @@ int pmnb_evaluate_device_noalloc(pmnb_ctx *ctx, const double *d_positions,
     return fail(ctx, PMNB_ERR_HIP, "no scratch address on device %d: %s", dev,
                 hipGetErrorString(serr));
   size_t need = 0;
-  long long nfix = 0;
-  carve_bufs(ctx, nullptr, need, nfix);
+  carve_bufs(ctx, nullptr, need);
+  need = std::max(need, scratch_limit_bytes(ctx));
   if (need > kScratchBytes)
     return fail(ctx, PMNB_ERR_CAPACITY,
                 "the evaluation needs %zu bytes of scratch; the static scratch "
                 "holds %zu (64 MiB)", need, kScratchBytes);
-  const EvalBufs B = carve_bufs(ctx, base, need, nfix);
+  const EvalBufs B = carve_bufs(ctx, base, need);
   HIPCHK(hipSetDevice(dev));
   hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
   if (ctx->n == 0) return PMNB_OK;
-  const long long work = std::max<long long>(nfix, ctx->ncol_total);
-  const unsigned grid = (unsigned)std::min<long long>(
-      std::max<long long>(1, (work + kBlock - 1) / kBlock), 4096);
-  hipLaunchKernelGGL(k_scratch_setup, dim3(grid), dim3(kBlock), 0, s,
-                     ctx->reps[0], ctx->box, const_cast<TileRep *>(B.reps),
-                     const_cast<Box *>(B.box), const_cast<int *>(B.col_rep),
-                     ctx->ncol_total, B.ffix, nfix);
+  hipLaunchKernelGGL(k_scratch_setup, dim3(1), dim3(64), 0, s, ctx->reps[0],
+                     const_cast<TileRep *>(B.reps));
   HIPCHK(hipGetLastError());
   return run_device_bufs(ctx, B, d_positions, d_forces, d_out, d_mol_com,
                          flags, s, false);

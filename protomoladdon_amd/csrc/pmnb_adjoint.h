@@ -25,7 +25,7 @@
 //
 // Work decomposition and candidate streaming are those of the tile-path
 // pair kernels (one wave per work item of 16 sorted atoms, candidates of the
-// 3 x 3 neighbour columns buffered in LDS after a bounding-box test); the
+// 5 x 5 neighbour columns buffered in LDS after a bounding-box test); the
 // test appends passing (atom, record) entries to an LDS pair queue at
 // ballot + mbcnt positions, which the wave consumes one pair per lane.  Each
 // atom's dL/dx and dL/dq~ are summed by its own
@@ -359,11 +359,10 @@ k_tq_adj(ForceParams P, AdjC<float> C32, AdjC<double> C64, Sorted S,
       return rem;
     };
 
-    for (int oc = 0; oc < 9; oc++) {
-      const int ox = oc / 3 - 1, oy = oc % 3 - 1;
-      // an axis with a single column takes it once
-      if (wx && ox != 0) continue;
-      if (wy && oy != 0) continue;
+    const int nox = wx ? G.nx : 5, noy = wy ? G.ny : 5;
+    for (int oc = 0; oc < nox * noy; oc++) {
+      // on an axis with a per-pair image every column once
+      const int ox = oc / noy - (wx ? 0 : 2), oy = oc % noy - (wy ? 0 : 2);
       const float gx = wx ? 0.f : fmaxf(0.f, fmaxf((float)ox * G.csx - bx1,
                                                   bx0 - (float)(ox + 1) * G.csx));
       const float gy = wy ? 0.f : fmaxf(0.f, fmaxf((float)oy * G.csy - by1,

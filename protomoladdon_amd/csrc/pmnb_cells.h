@@ -242,188 +242,4 @@ __global__ void k_gather(Box b, Grid g, const double *__restrict__ pos,
   scell[s] = cell_of[a];
 }
 
-// Replica-aware cell assignment and gather of the tile path: atom i belongs
-// to replica rep_of[i] (replica 0 when rep_of is null), whose box and
-// column grid place it; cells are numbered globally from the replica's
-// cell offset.  RepT provides box, grid and cell_off.
-// Cells of a block's atoms are few (consecutive atoms are neighbours): the
-// block counts its atoms per cell in an LDS table (open addressing on the
-// cell index), takes one global atomic add per distinct cell, all issued
-// together, and gives each atom the cell's base plus its rank in the block:
-// its arrival rank in the cell, at which it is written into the cell's row
-// of `bucket` (cap entries per cell; an atom ranked beyond cap is found
-// again from cell_of by k_sort_gather_r).  pos_copy as in k_assign.
-// Requires blockDim.x == kBlock.
-template <class RepT>
-__global__ void __launch_bounds__(kBlock)
-k_assign_r(const RepT *__restrict__ reps, const int *__restrict__ rep_of,
-           const double *__restrict__ pos, int n, int *__restrict__ cell_of,
-           int *__restrict__ count, int *__restrict__ bucket, int cap,
-           double *__restrict__ pos_copy) {
-  __shared__ int key[kBlock], lcount[kBlock], base[kBlock];
-  const int t = threadIdx.x;
-  const int i = blockIdx.x * kBlock + t;
-  key[t] = -1;
-  lcount[t] = 0;
-  __syncthreads();
-  int slot = -1, lrank = 0, c = 0;
-  if (i < n) {
-    const RepT &R = reps[rep_of ? rep_of[i] : 0];
-    int cx, cy, cz;
-    double vx, vy, vz;
-    const double px = pos[3 * i], py = pos[3 * i + 1], pz = pos[3 * i + 2];
-    if (pos_copy) {
-      pos_copy[3 * i] = px;
-      pos_copy[3 * i + 1] = py;
-      pos_copy[3 * i + 2] = pz;
-    }
-    cell_coords(R.box, R.grid, px, py, pz, cx, cy, cz, vx, vy, vz);
-    c = R.cell_off + (cx * R.grid.n[1] + cy) * R.grid.n[2] + cz;
-    cell_of[i] = c;
-    // at most kBlock distinct cells in kBlock slots: the probe ends
-    int h = c & (kBlock - 1);
-    while (true) {
-      const int old = atomicCAS(&key[h], -1, c);
-      if (old == -1 || old == c) break;
-      h = (h + 1) & (kBlock - 1);
-    }
-    slot = h;
-    lrank = atomicAdd(&lcount[h], 1);
-  }
-  __syncthreads();
-  if (key[t] >= 0) base[t] = atomicAdd(&count[key[t]], lcount[t]);
-  __syncthreads();
-  if (i < n) {
-    const int r = base[slot] + lrank;
-    if (r < cap) bucket[(size_t)c * cap + r] = i;
-  }
-}
-
-// Per-cell ordering and gather of the tile path in one pass: one wave per
-// cell takes the cell's atoms from its bucket row (or, for a cell of more
-// than cap atoms, from cell_of), puts them in ascending atom order (as
-// k_sort_cells) and writes, for each sorted slot, the atom index, its FP64
-// position, the FP32 offset from its cell's lower corner (computed in FP64)
-// with its charge, type, charge, molecule, cell and packed record.
-template <class RepT>
-__global__ void __launch_bounds__(kBlock)
-k_sort_gather_r(const RepT *__restrict__ reps, const int *__restrict__ rep_of,
-                const double *__restrict__ pos, const int *__restrict__ start,
-                const int *__restrict__ count, int ncell,
-                const int *__restrict__ bucket, int cap,
-                const int *__restrict__ cell_of, int n,
-                const int *__restrict__ type, const double *__restrict__ q,
-                const int *__restrict__ mol, int *__restrict__ sorted,
-                double *__restrict__ sx, double *__restrict__ sy,
-                double *__restrict__ sz, float4 *__restrict__ sloc,
-                int *__restrict__ stype, double *__restrict__ sq,
-                int *__restrict__ smol, int *__restrict__ scell,
-                int2 *__restrict__ srec) {
-  __shared__ int keys[kBlock / 64][kSortLds];
-  __shared__ int found[kBlock / 64];
-  const int w = threadIdx.x >> 6;
-  const int c = blockIdx.x * (kBlock / 64) + w;
-  const int lane = threadIdx.x & 63;
-  if (c >= ncell) return;
-  const int m = count[c];
-  if (m == 0) return;
-  const int s0 = start[c];
-  int *seg = sorted + s0;
-  const int *row = bucket + (size_t)c * cap;  // the first min(m, cap) atoms
-  // a cell of more than cap atoms: the wave finds them all in cell_of and
-  // appends them to dst (any order; sorted below)
-  auto collect = [&](int *dst) {
-    if (lane == 0) found[w] = 0;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int i = lane; i < n; i += 64)
-      if (cell_of[i] == c) dst[atomicAdd(&found[w], 1)] = i;
-  };
-  // slot s0 + k receives atom a
-  auto put = [&](int k, int a) {
-    const int s = s0 + k;
-    seg[k] = a;
-    const RepT &R = reps[rep_of ? rep_of[a] : 0];
-    const double x = pos[3 * a], y = pos[3 * a + 1], z = pos[3 * a + 2];
-    sx[s] = x;
-    sy[s] = y;
-    sz[s] = z;
-    int cx, cy, cz;
-    double vx, vy, vz;
-    cell_coords(R.box, R.grid, x, y, z, cx, cy, cz, vx, vy, vz);
-    float4 l;
-    l.x = (float)(vx - (double)cx * R.grid.cs[0]);
-    l.y = (float)(vy - (double)cy * R.grid.cs[1]);
-    l.z = (float)(vz - (double)cz * R.grid.cs[2]);
-    l.w = (float)q[a];
-    sloc[s] = l;
-    stype[s] = type[a];
-    sq[s] = q[a];
-    smol[s] = mol[a];
-    scell[s] = c;
-    srec[s] = make_int2(type[a] | (mol[a] << 8), a);
-  };
-  if (m <= 64) {  // cap >= 64: every atom is in the row
-    int v = lane < m ? row[lane] : 0x7fffffff;
-    for (int k = 2; k <= 64; k <<= 1) {
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        const int other = __shfl_xor(v, j, 64);
-        const bool up = (lane & k) == 0;
-        const bool lower = (lane & j) == 0;
-        v = (lower == up) ? min(v, other) : max(v, other);
-      }
-    }
-    if (lane < m) put(lane, v);
-  } else if (m <= kSortLds) {
-    if (m <= cap) {
-      for (int k = lane; k < m; k += 64) keys[w][k] = row[k];
-    } else {
-      collect(keys[w]);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int k = lane; k < m; k += 64) {
-      const int v = keys[w][k];
-      int rank = 0;
-      for (int j = 0; j < m; j++) rank += keys[w][j] < v;
-      put(rank, v);
-    }
-  } else {
-    // m > kSortLds >= cap
-    collect(seg);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    if (lane == 0) {
-      for (int i = 1; i < m; i++) {
-        int v = seg[i];
-        int j = i - 1;
-        while (j >= 0 && seg[j] > v) {
-          seg[j + 1] = seg[j];
-          j--;
-        }
-        seg[j + 1] = v;
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    for (int k = lane; k < m; k += 64) put(k, seg[k]);
-  }
-}
-
-// Sets n 64-bit integers to zero.
-__global__ void k_zero_i64(long long *p, long long n) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
-// Sets n doubles to zero (a kernel node, not a memset, inside graphs).
-__global__ void k_zero_f64(double *p, long long n) {
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0.0;
-}
-
 }  // namespace pmnb

@@ -58,6 +58,7 @@ struct F32Params {
   float cut2, band, Lx, Ly, Lz, iLx, iLy, iLz;
   float on2l, cut2l, s1l, s2l, s3l, on2e, cut2e, s1e, s2e, s3e;
   float alpha, tapi, csf;
+  float pal, ea2;   // 0.3275911 alpha, -alpha^2 log2(e)
   int same_switch;  // LJ and electrostatic switches are the same C2
 };
 

@@ -47,12 +47,13 @@
 // those blocks only and its sweep count, hint and iteration record are its
 // own, as when the replica runs alone.  A single system is one replica.
 //
-// Cells.  The kernel that clears the forces before an evaluation (ZERO) also
-// does the evaluation's cell assignment on the tile path when given the
-// cell arrays (as k_assign_r: cell of every atom, one global count atomic
-// per distinct cell of a block, bucket slot), from the positions it has
-// just written, which saves the evaluation that launch (single systems; a
-// batch measured faster with the evaluation's own launch).
+// Bins.  The last kernel before an evaluation (ZERO) clears the forces when
+// the evaluation adds to them (the tile path's pair kernel writes them) and
+// does the evaluation's bin assignment on the tile path when given the bin
+// arrays (as k_assign_bins: bin of every atom, one global count atomic per
+// distinct bin of a block, bucket slot), from the positions it has just
+// written, which saves the evaluation that launch (single systems; a batch
+// measured faster with the evaluation's own launch).
 #pragma once
 
 #include "pmnb_queue.h"
@@ -130,13 +131,15 @@ struct LfDev {
                             // ([call * n_reps + rep], optional)
   long long iters_cap;
   int *nonconv;             // [3] stage calls that hit max_iter
-  // cell assignment of the next evaluation (tile path; c_count null: none)
+  // bin assignment of the next evaluation (tile path; c_count null: none)
   const TileRep *c_reps;
   const int *c_rep_of;      // replica of each atom (null: one replica)
-  int *c_cell_of, *c_count, *c_bucket;
-  int c_cap;                // atom slots per cell of c_bucket
-  int *z_count;             // cell counts to clear (null: none)
+  int *c_bin_of, *c_count, *c_bucket;
+  int c_cap;                // atom slots per bin of c_bucket
+  int *z_count;             // bin counts to clear (null: none)
   int z_nc;
+  int z_force;              // the forces are cleared (the evaluation that
+                            // follows adds to them)
 };
 
 struct D3 {
@@ -608,11 +611,11 @@ __device__ __forceinline__ int lf_decide(const LfDev &d, long long scall,
   return lf_fallback<STAGE, SH>(d, L, R);
 }
 
-// Cell assignment of the atoms idx[0..NA) (negative: none) at positions x
-// (k_assign_r's scheme for a block of up to kLfBlock * NA atoms): the block
-// counts its atoms per cell in an LDS table, takes one global atomic add
-// per distinct cell and writes each atom into its cell's bucket row at the
-// cell's base plus its rank (below the row's capacity).  Block-wide (all
+// Bin assignment of the atoms idx[0..NA) (negative: none) at positions x
+// (k_assign_bins' scheme for a block of up to kLfBlock * NA atoms): the block
+// counts its atoms per bin in an LDS table, takes one global atomic add
+// per distinct bin and writes each atom into its bin's bucket row at the
+// bin's base plus its rank (below the row's capacity).  Block-wide (all
 // threads call it).
 constexpr int kLfCellSlots = 1024;
 // LDS of lf_assign_cells, one object per kernel whatever NA
@@ -646,9 +649,9 @@ __device__ __forceinline__ void lf_assign_cells(const LfDev &d,
     int cx, cy, cz;
     double vx, vy, vz;
     cell_coords(R.box, R.grid, x[a].x, x[a].y, x[a].z, cx, cy, cz, vx, vy, vz);
-    const int c = R.cell_off + (cx * R.grid.n[1] + cy) * R.grid.n[2] + cz;
-    d.c_cell_of[i] = c;
-    // at most NS distinct cells in NS slots: the probe ends
+    const int c = tile_bin(R, cx, cy, cz);
+    d.c_bin_of[i] = c;
+    // at most NS distinct bins in NS slots: the probe ends
     int h = c & (NS - 1);
     while (true) {
       const int old = atomicCAS(&key[h], -1, c);
@@ -672,7 +675,8 @@ __device__ __forceinline__ void lf_assign_cells(const LfDev &d,
 
 // One fused launch: apply stage APPLY (sweep count from its probe), then the
 // per-atom update PRE, store, then the first probe of stage PROBE; with
-// ZERO, clear the forces and the energy block for the next evaluation.
+// ZERO, what the next evaluation needs (energy block and, where it adds to
+// them, forces cleared; bins).
 // sc_apply / sc_probe: the per-stage call numbers; call: the global one.
 template <int APPLY, int PRE, int PROBE, bool ZERO, int SHAPE>
 __global__ __launch_bounds__(kLfBlock) void k_lf_step(LfDev d, long long sc_apply,
@@ -703,7 +707,7 @@ __global__ __launch_bounds__(kLfBlock) void k_lf_step(LfDev d, long long sc_appl
         st3(d.x, i, x);
         st3(d.v, i, v);
       }
-      if (ZERO) st3(d.f, i, D3{0, 0, 0});
+      if (ZERO && d.z_force) st3(d.f, i, D3{0, 0, 0});
       ia[0] = i;
       xa[0] = x;
     }
@@ -776,7 +780,7 @@ __global__ __launch_bounds__(kLfBlock) void k_lf_step(LfDev d, long long sc_appl
         st3(d.x, i, g.x[a]);
         st3(d.v, i, g.v[a]);
       }
-      if (ZERO) st3(d.f, i, D3{0, 0, 0});
+      if (ZERO && d.z_force) st3(d.f, i, D3{0, 0, 0});
     }
   }
   if constexpr (ZERO) {

@@ -25,19 +25,36 @@ struct Sorted {
   const double *q;
   const int *mol;
   const int *cell;               // linear cell of each sorted slot
-  const int2 *rec;               // {type | molecule << 8, original index}
-                                 // (tile path only; < 256 types and
-                                 // < 2^24 atoms there)
+  const unsigned *rec;           // original index << 8 | type (tile path
+                                 // only; at most 256 types and < 2^24
+                                 // atoms there)
   const int *cstart, *ccount;    // per-cell segment of the sorted order
   const int4 *delta;             // shell offsets, (0,0,0) first
   const unsigned long long *xfull, *xmod;  // exclusion masks (original idx)
   const unsigned long long *xown;  // per atom {forward FULL, forward MODIFIED,
                                    // reverse FULL, reverse MODIFIED}
+  const unsigned long long *xcode;  // per atom: two bits per partner at
+                                   // distance d = -15 .. 15 (bits 2 d + 30):
+                                   // its class, FULL for the atom itself
   const double *lj;              // T*T*4 {A, B, A14, B14}
   const float4 *ljf;             // same in FP32
   const double *com;             // molecule centres (molecular virial)
   const Box *box;                // device copy of the box (read on demand)
 };
+
+// FP32 record of an LJ table entry {A, B, A14, B14}.  The pair kernels' 1/r^2
+// comes from v_rsq_f32 squared (v_rcp_f32 without electrostatics), which are
+// low by 7.4e-9 (6.8e-9) on average (over all mantissas, measured); in the
+// sixth and seventh power, the same for every pair, that is 1e-7 of the
+// virial.  A and B carry the inverse of what r^-12 and r^-6 (6.5 and 3.5
+// factors 1/r^2, between the energy's and the force's) lose.
+__host__ __device__ __forceinline__ float4 lj_record(const double *v,
+                                                     int elec) {
+  const double b = elec != 0 ? 2.0 * 7.39e-9 : 6.75e-9;
+  const double a = 1.0 + 6.5 * b, c = 1.0 + 3.5 * b;
+  return make_float4((float)(v[0] * a), (float)(v[1] * c), (float)(v[2] * a),
+                     (float)(v[3] * c));
+}
 
 // Wave-then-block reduction of ACC_N doubles in a fixed order; block b
 // of NW waves writes partial[b * ACC_N + k].
@@ -214,6 +231,61 @@ __device__ __forceinline__ long long to_fixed(double v) {
   const double lim = 2147483647.0;
   v = fmin(fmax(v, -lim), lim);
   return (long long)__builtin_rint(v * kFixedScale);
+}
+
+// The same pair with fewer operations, for pairs whose 1-4 factor is already
+// in A, B and qq (tile path): with one switch for both terms (SAME) the
+// switched F/r is F S - E S~ of their sums.
+template <int ELEC, bool SAME>
+__device__ __forceinline__ void pair_mix(const F32Params &F, float r2, float A,
+                                         float B, float qq, float &ff,
+                                         float &e1, float &e2) {
+  const float rr = ELEC != 0 ? __builtin_amdgcn_rsqf(r2) : 0.f;
+  const float rd2 = ELEC != 0 ? rr * rr : __builtin_amdgcn_rcpf(r2);
+  const float r6 = rd2 * rd2 * rd2;
+  const float a6 = A * r6;
+  e1 = r6 * (a6 - B);
+  // 12 A / r^12 - 6 B / r^6 = 6 (A / r^12 + E)
+  float f1 = fmaf(r6, a6, e1) * (6.f * rd2);
+  float f2 = 0.f;
+  e2 = 0.f;
+  if (ELEC == 1) {
+    e2 = qq * rr;
+    f2 = e2 * rd2;
+  } else if (ELEC == 2) {
+    // Abramowitz & Stegun 7.1.26 (base/MathUtilities.cpp:39-49)
+    const float tt = __builtin_amdgcn_rcpf(fmaf(F.pal, r2 * rr, 1.f));
+    const float poly =
+        tt * fmaf(tt, fmaf(tt, fmaf(tt, fmaf(tt, 1.061405429f, -1.453152027f),
+                                    1.421413741f),
+                           -0.284496736f),
+                  0.254829592f);
+    const float e = qq * __builtin_amdgcn_exp2f(F.ea2 * r2);
+    e2 = poly * e * rr;
+    f2 = fmaf(F.tapi, e, e2) * rd2;
+  }
+  // with one switch the pair is within its cutoff
+  float c2 = SAME ? F.cut2l - r2 : fmaxf(F.cut2l - r2, 0.f);
+  float c4 = c2 * fmaf(2.f, r2, F.s2l);
+  const bool swl = r2 >= F.on2l;
+  const float sv = swl ? F.s1l * (c2 * c4) : 1.f;
+  const float sd = swl ? F.s3l * fmaf(c2, c2, -c4) : 0.f;
+  if (ELEC == 0 || SAME) {
+    ff = fmaf(f1 + f2, sv, -(e1 + e2) * sd);
+    e1 *= sv;
+    e2 *= sv;
+    return;
+  }
+  f1 = fmaf(f1, sv, -e1 * sd);
+  e1 = e1 * sv;
+  c2 = fmaxf(F.cut2e - r2, 0.f);
+  c4 = c2 * fmaf(2.f, r2, F.s2e);
+  const bool swe = r2 >= F.on2e;
+  const float se = swe ? F.s1e * (c2 * c4) : 1.f;
+  const float sde = swe ? F.s3e * fmaf(c2, c2, -c4) : 0.f;
+  f2 = fmaf(f2, se, -e2 * sde);
+  e2 = e2 * se;
+  ff = f1 + f2;
 }
 
 // FP32 pair of OneAtomPairTwo: returns the switched F/r (ff) and the two

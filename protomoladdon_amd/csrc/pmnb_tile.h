@@ -1,13 +1,14 @@
 // Column grid and wave helpers of the tile path (the pair kernels are in
-// pmnb_queue.h and pmnb_adjoint.h).
+// pmnb_cluster.h and pmnb_adjoint.h).
 //
-// Cell grid: x/y columns at least one cutoff wide (a neighbour's column
-// offset is -1, 0 or +1) and z cells of about a third (mixed) or a quarter
-// (FP64) of the cutoff; atoms are
-// sorted column by column, z cell by z cell, ascending atom index inside a
-// cell, so a column's z-range of cells is one contiguous run of the sorted
-// arrays (two when it wraps).  One wave handles 16 consecutive sorted atoms
-// of one column.
+// Cell grid: x/y columns at least half a cutoff wide (a neighbour's column
+// offset is -2 .. 2) and z cells of about an eighth of the cutoff; atoms are
+// sorted column by column and by z (then atom index) inside a column, so a
+// column's z-range of cells is one contiguous run of the sorted arrays (two
+// when it wraps).  A work item is 16 consecutive sorted atoms of one column:
+// with columns of half a cutoff its atoms fill a box of about 4.9 x 4.9 x 6 A
+// (96,000-atom water, 9 A cutoff), whose cutoff shell holds 750 candidates
+// of which a third are pairs; columns of a whole cutoff hold 980.
 #pragma once
 
 #include "pmnb_common.h"
@@ -20,6 +21,7 @@ constexpr int kTileAtoms = 16;   // atoms per wave
 struct TileGrid {
   int nx, ny, nz, rz;   // grid and z-cell reach of the cutoff
   float csx, csy, csz;  // cell sizes
+  float lox, loy, loz;  // ... and what rounding to FP32 left of them
 };
 
 __device__ __forceinline__ float wave_min(float v) {

@@ -1,0 +1,119 @@
+"""The tile path's cell build and pair kernel at the edges of their ranges,
+against the FP64 oracle, with the bars of test_gpu_parity: pair sets bit for
+bit, FP64 forces within 1e-11 of the largest component, mixed forces within
+1e-5 RMS."""
+import numpy as np
+import pytest
+
+from protomoladdon_amd import systems
+from protomoladdon_amd.batch import BatchedCutoffForce
+from protomoladdon_amd.topology import (EXCLUSION_FULL, EXCLUSION_MODIFIED,
+                                        PeriodicBoundaryConditions)
+from tests.test_gpu_batch import batch_eval
+from tests.test_gpu_parity import check_fp64, check_mixed, rms_rel, run_gpu
+
+pytestmark = pytest.mark.gpu
+
+
+def types(n):
+    """n LJ types: 8 fit the kernel's LDS table, 9 .. 256 are read from
+    memory, 257 take the general path."""
+    return systems.many_type_chains(n_chains=45, n_types=n)
+
+
+def stretched(sx, sy, sz, n_mol=500):
+    """Water in a box of sx, sy, sz times the cube's side (25 A at 500):
+    columns are 4.5 A wide, so an axis below 22.5 A has fewer than five and
+    takes the minimum image of every pair."""
+    w = systems.small_water(n_mol=n_mol)
+    L = float(w.topology.boundary_conditions.lengths()[0])
+    s = np.array([sx, sy, sz])
+    w.positions = w.positions * s
+    a, b, c = L * s
+    w.topology.boundary_conditions = PeriodicBoundaryConditions(
+        (a, 0, 0), (0, b, 0), (0, 0, c), (0.5 * a, 0.5 * b, 0.5 * c))
+    w.name = "water_%g_%g_%g" % (sx, sy, sz)
+    return w
+
+
+def gas(n_mol, L):
+    """A thin gas: wide columns and cells, items whose atoms spread beyond
+    the expanded distance test."""
+    return systems.water_workload("gas", n_mol, L, 5, 9.0, 7.5, "ewald", 0.32)
+
+
+def far_exclusions():
+    """FULL and MODIFIED pairs at index distances of 1 .. 64 (15 is the last
+    held in the code word, 64 the last in the masks)."""
+    w = systems.small_chains(n_chains=60)
+    n = w.n_atoms
+    w.topology.molecules[:] = np.arange(n) // 100
+    x = w.topology.exclusions
+    for k, d in enumerate((14, 15, 16, 31, 63, 64)):
+        a = np.arange(k, n - d, 7)
+        a = a[a // 100 == (a + d) // 100]
+        x.add_many(np.stack([a, a + d], 1),
+                   EXCLUSION_FULL if k % 2 else EXCLUSION_MODIFIED)
+    w.topology.touch()
+    return w
+
+
+CASES = {
+    "types1": lambda: types(1), "types8": lambda: types(8),
+    "types9": lambda: types(9), "types256": lambda: types(256),
+    "types257": lambda: types(257),
+    "four_columns_x": lambda: stretched(0.85, 1.2, 1.0),
+    "two_columns_y_flat_z": lambda: stretched(1.2, 0.73, 0.75),
+    "gas": lambda: gas(600, 120.0), "gas_no_pairs": lambda: gas(60, 90.0),
+    "gas_three_molecules": lambda: gas(3, 200.0),
+    "dense_column": lambda: stretched(0.8, 0.8, 12.0, n_mol=900),
+    "far_exclusions": far_exclusions,
+}
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_pairs_match_oracle(case):
+    ref = check_fp64(CASES[case](), flags=3)
+    if ref.n_pairs:
+        check_mixed(CASES[case](), flags=1)
+    else:
+        f, _, npairs, _ = run_gpu(CASES[case](), "mixed", 1, with_pairs=False)
+        assert npairs == 0 and not f.any()
+
+
+@pytest.mark.parametrize("precision,shapes", [("mixed", 3), ("fp64", 2)])
+def test_shapes_give_the_same_bits(precision, shapes):
+    """A wave per item or a block per item, mixed sizes in one batch."""
+    ws = [systems.config3_replica(0, 167), systems.config3_replica(1, 40),
+          systems.config3_replica(2, 700)]
+    bf = BatchedCutoffForce.from_workloads(ws, precision=precision)
+    res = []
+    for shape in range(shapes):
+        bf.set_shape(shape)
+        res.append(batch_eval(bf, ws)[1:])
+    bf.close()
+    for f, out in res[1:]:
+        np.testing.assert_array_equal(f, res[0][0])
+        np.testing.assert_array_equal(out, res[0][1])
+
+
+@pytest.mark.parametrize("precision", ["mixed", "fp64"])
+@pytest.mark.parametrize("bad", [np.nan, -np.nan, np.inf])
+def test_atoms_without_a_position_have_no_pairs(precision, bad):
+    """The other atoms' forces are those without them: the two atoms carry
+    no charge and the oxygens' type of a hydrogen, so at any position they
+    give no force."""
+    w = systems.small_water(n_mol=300)
+    t = w.topology
+    t.scaled_charges[[4, 5]] = 0.0
+    t.touch()
+    ref = run_gpu(w, "fp64", 0, with_pairs=False)
+    p = w.positions.copy()
+    p[4] = bad
+    p[5, 1] = bad
+    f, _, npairs, _ = run_gpu(w, precision, 0, positions=p, with_pairs=False)
+    rest = np.setdiff1d(np.arange(w.n_atoms), [4, 5])
+    assert npairs < ref[2]
+    assert np.isfinite(f).all()
+    assert rms_rel(f[rest], ref[0][rest]) <= (
+        1e-5 if precision == "mixed" else 1e-12)
