@@ -519,7 +519,7 @@ void pmnb_ewald_destroy(pmnb_ewald *ew);
    order (even, 2..8 here, each size >= order), cutoff rc (sets the default
    alpha), accuracy, alpha (<= 0: the reference's default, erfc(alpha rc) /
    rc = accuracy by bisection).  The charge grid is summed as 64-bit
-   fixed-point integers (2^-32), so results repeat bit for bit.  The
+   fixed-point integers (2^-40), so results repeat bit for bit.  The
    correction rows follow pmnb_ewald_create's rule.  Fixed at creation like
    pmnb_ewald (PMNB_ERR_STATE after a box or topology change). */
 

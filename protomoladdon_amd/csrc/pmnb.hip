@@ -3196,8 +3196,10 @@ struct pmnb_pme {
   int nx = 0, ny = 0, nz = 0;
   double alpha = 0, kc = 0, V = 0;
   double csf = 1.0, e_self = 0, e_charged = 0;
-  DevBuf q, qfix, qreal, qk, mod, ex, part, ew_part, xptr, xent, xrows;
-  int n_part = 0;
+  DevBuf q, count, bucket, over, qreal, qk, mod, ex, part, cpart, xptr, xent,
+      xrows;
+  int nb[3] = {0, 0, 0}, cap = 0;
+  int n_part = 0, n_cpart = 0;
   hipfftHandle fwd = 0, inv = 0;
   bool have_fwd = false, have_inv = false;
   double box_key[12] = {0};
@@ -3266,11 +3268,15 @@ PmeDev pme_dev(pmnb_pme *pm) {
     d.hr[a] = nn[a] / b.e[a];
     d.off[a] = -(pm->order - 1) / 2 + nn[a];
     d.Lr[a] = 1.0 / b.e[a];
+    d.nb[a] = pm->nb[a];
   }
   d.piVr = 1.0 / (M_PI * pm->V);
   d.fac = M_PI * M_PI / (pm->alpha * pm->alpha);
   d.q = pm->q.as<double>();
-  d.qfix = pm->qfix.as<long long>();
+  d.count = pm->count.as<int>();
+  d.bucket = pm->bucket.as<double4>();
+  d.over = pm->over.as<double4>();
+  d.cap = pm->cap;
   d.qreal = pm->qreal.as<double>();
   d.qk = pm->qk.as<double2>();
   const double *mod = pm->mod.as<double>(), *ex = pm->ex.as<double>();
@@ -3282,6 +3288,8 @@ PmeDev pme_dev(pmnb_pme *pm) {
   d.ex[2] = ex + pm->nx + pm->ny;
   d.part = pm->part.as<double>();
   d.n_part = pm->n_part;
+  d.cpart = pm->cpart.as<double>();
+  d.n_cpart = pm->n_cpart;
   return d;
 }
 
@@ -3291,7 +3299,6 @@ EwDev pme_corr_dev(pmnb_pme *pm) {
   e.n = pm->n;
   e.nk = 0;  // correction terms only
   e.q = pm->q.as<double>();
-  e.part = pm->ew_part.as<double>();
   e.xptr = pm->xptr.as<int>();
   e.xent = pm->xent.as<int>();
   e.xrows = pm->xrows.as<int>();
@@ -3308,19 +3315,18 @@ EwDev pme_corr_dev(pmnb_pme *pm) {
 template <int P>
 void pme_spread(pmnb_pme *pm, const PmeDev &d, const double *x,
                 hipStream_t s) {
-  hipLaunchKernelGGL(k_pme_spread<P>, dim3(blocks_for(pm->n, kPmeBlock)),
+  hipLaunchKernelGGL(k_pme_bin, dim3(blocks_for(pm->n, kPmeBlock)),
                      dim3(kPmeBlock), 0, s, d, x);
-  const long long total = (long long)pm->nx * pm->ny * pm->nz;
-  hipLaunchKernelGGL(k_pme_to_real,
-                     dim3((unsigned)((total + kPmeBlock - 1) / kPmeBlock)),
-                     dim3(kPmeBlock), 0, s, d, total);
+  const int tiles = blocks_for(pm->nx, kPmeTile) * blocks_for(pm->ny, kPmeTile) *
+                    blocks_for(pm->nz, kPmeTile);
+  hipLaunchKernelGGL(k_pme_spread<P>, dim3(tiles), dim3(kPmeBlock), 0, s, d);
 }
 
 template <int P>
 void pme_launch_gather(pmnb_pme *pm, const PmeDev &d, const EwDev &e,
                        const double *x, double *f, hipStream_t s) {
-  hipLaunchKernelGGL(k_pme_gather<P>, dim3(blocks_for(pm->n, kPmeBlock)),
-                     dim3(kPmeBlock), 0, s, d, e, x, f);
+  hipLaunchKernelGGL(k_pme_gather<P>, dim3(pm->n_cpart), dim3(kPmeBlock), 0, s, d,
+                     e, x, f);
 }
 
 }  // namespace
@@ -3423,7 +3429,13 @@ int pmnb_pme_create(pmnb_ctx *ctx, int32_t nx, int32_t ny, int32_t nz,
                  ent);
   const long long total = (long long)nx * ny * nz;
   const long long half = (long long)nx * ny * (nz / 2 + 1);
-  pm->n_part = (int)((half + kPmeBlock - 1) / kPmeBlock);
+  pm->n_part = std::min(kPmeScalarBlocks, blocks_for(nx * ny, kPmeBlock / 64));
+  pm->n_cpart = blocks_for(std::max(n_atoms, 1), kPmeBlock / kPmeLanes);
+  long long bins = 1;
+  for (int a = 0; a < 3; a++) bins *= pm->nb[a] = blocks_for(nn[a], kPmeBin);
+  // four times the mean occupancy and 8 more, at most 256 (the atoms beyond a
+  // full bucket go to the overflow list)
+  pm->cap = (int)std::min<long long>(256, 4 * (n_atoms / bins) + 8);
   auto up = [&](DevBuf &d, const void *src, size_t bytes) -> hipError_t {
     hipError_t e = d.ensure(std::max<size_t>(bytes, 16));
     if (e == hipSuccess && bytes && src)
@@ -3432,8 +3444,12 @@ int pmnb_pme_create(pmnb_ctx *ctx, int32_t nx, int32_t ny, int32_t nz,
   };
   hipError_t e = hipSetDevice(pm->device);
   if (e == hipSuccess) e = up(pm->q, scaled_charge, (size_t)n_atoms * sizeof(double));
-  if (e == hipSuccess) e = pm->qfix.ensure((size_t)total * sizeof(long long));
-  if (e == hipSuccess) e = hipMemset(pm->qfix.p, 0, (size_t)total * sizeof(long long));
+  if (e == hipSuccess) e = pm->count.ensure((size_t)(bins + 1) * sizeof(int));
+  if (e == hipSuccess) e = hipMemset(pm->count.p, 0, (size_t)(bins + 1) * sizeof(int));
+  if (e == hipSuccess)
+    e = pm->bucket.ensure((size_t)bins * pm->cap * sizeof(double4));
+  if (e == hipSuccess)
+    e = pm->over.ensure((size_t)std::max(n_atoms, 1) * sizeof(double4));
   if (e == hipSuccess) e = pm->qreal.ensure((size_t)total * sizeof(double));
   if (e == hipSuccess) e = pm->qk.ensure((size_t)half * sizeof(double2));
   if (e == hipSuccess) e = up(pm->mod, mod.data(), mod.size() * sizeof(double));
@@ -3441,7 +3457,7 @@ int pmnb_pme_create(pmnb_ctx *ctx, int32_t nx, int32_t ny, int32_t nz,
   if (e == hipSuccess)
     e = pm->part.ensure((size_t)pm->n_part * kPmeSums * sizeof(double));
   if (e == hipSuccess)
-    e = pm->ew_part.ensure((size_t)kEwFinBlocks * kEwFinSums * sizeof(double));
+    e = pm->cpart.ensure((size_t)pm->n_cpart * kPmeSums * sizeof(double));
   if (e == hipSuccess) e = up(pm->xptr, cnt.data(), (n_atoms + 1) * sizeof(int));
   if (e == hipSuccess) e = up(pm->xent, ent.data(), 2 * (size_t)n_excl * sizeof(int));
   if (e == hipSuccess) e = up(pm->xrows, rows.data(), rows.size() * sizeof(int));
@@ -3517,10 +3533,7 @@ int pmnb_pme_evaluate_device(pmnb_pme *pm, const double *d_positions,
     case 6: pme_launch_gather<6>(pm, d, e, d_positions, d_forces, s); break;
     default: pme_launch_gather<8>(pm, d, e, d_positions, d_forces, s); break;
   }
-  hipLaunchKernelGGL(k_pme_finish, dim3(1), dim3(64), 0, s, d, d_out, virial);
-  hipLaunchKernelGGL(k_ew_partials, dim3(kEwFinBlocks), dim3(kEwBlock), 0, s,
-                     e, d_positions);
-  hipLaunchKernelGGL(k_ew_finish, dim3(1), dim3(64), 0, s, e, d_out, virial,
+  hipLaunchKernelGGL(k_pme_finish, dim3(1), dim3(1024), 0, s, d, d_out, virial,
                      pm->e_self + pm->e_charged, pm->e_charged);
   HIPCHK(hipGetLastError());
   return PMNB_OK;
@@ -3532,8 +3545,9 @@ void pmnb_pme_destroy(pmnb_pme *pm) {
   (void)hipDeviceSynchronize();
   if (pm->have_fwd) (void)hipfftDestroy(pm->fwd);
   if (pm->have_inv) (void)hipfftDestroy(pm->inv);
-  DevBuf *bufs[] = {&pm->q, &pm->qfix, &pm->qreal, &pm->qk, &pm->mod, &pm->ex,
-                    &pm->part, &pm->ew_part, &pm->xptr, &pm->xent, &pm->xrows};
+  DevBuf *bufs[] = {&pm->q, &pm->count, &pm->bucket, &pm->over, &pm->qreal,
+                    &pm->qk, &pm->mod, &pm->ex, &pm->part, &pm->cpart,
+                    &pm->xptr, &pm->xent, &pm->xrows};
   for (DevBuf *b : bufs) b->release();
   delete pm;
 }

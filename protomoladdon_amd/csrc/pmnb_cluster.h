@@ -71,30 +71,6 @@ constexpr int kLjTypes = 8;                 // types held in LDS
 // What k_pairs forms beside the forces and the pair count.
 enum PairMode { kForces = 0, kEnergies = 1, kMolVirial = 2 };
 
-// Sum of each of eight values over the wave: lane l returns the sum of value
-// l % 8.  Three halving exchanges, then three full ones (fixed tree).
-__device__ __forceinline__ double wave_sum8(const double (&v)[8], int lane) {
-  double a[4], b[2];
-  const bool o0 = lane & 1, o1 = lane & 2, o2 = lane & 4;
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const double keep = o0 ? v[2 * k + 1] : v[2 * k];
-    const double send = o0 ? v[2 * k] : v[2 * k + 1];
-    a[k] = keep + __shfl_xor(send, 1, 64);
-  }
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const double keep = o1 ? a[2 * k + 1] : a[2 * k];
-    const double send = o1 ? a[2 * k] : a[2 * k + 1];
-    b[k] = keep + __shfl_xor(send, 2, 64);
-  }
-  double s = (o2 ? b[1] : b[0]) + __shfl_xor(o2 ? b[0] : b[1], 4, 64);
-  s += __shfl_xor(s, 8, 64);
-  s += __shfl_xor(s, 16, 64);
-  s += __shfl_xor(s, 32, 64);
-  return s;
-}
-
 // Index of the lowest set bit, -1 for 0 (v_ffbl_b32).
 __device__ __forceinline__ int ctz_or_none(unsigned m) {
   return m ? __builtin_ctz(m) : -1;

@@ -216,6 +216,30 @@ __device__ __forceinline__ int excl_class(const unsigned long long *full,
   return 0;
 }
 
+// Sum of each of eight values over the wave: lane l returns the sum of value
+// l % 8.  Three halving exchanges, then three full ones (fixed tree).
+__device__ __forceinline__ double wave_sum8(const double (&v)[8], int lane) {
+  double a[4], b[2];
+  const bool o0 = lane & 1, o1 = lane & 2, o2 = lane & 4;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const double keep = o0 ? v[2 * k + 1] : v[2 * k];
+    const double send = o0 ? v[2 * k] : v[2 * k + 1];
+    a[k] = keep + __shfl_xor(send, 1, 64);
+  }
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const double keep = o1 ? a[2 * k + 1] : a[2 * k];
+    const double send = o1 ? a[2 * k] : a[2 * k + 1];
+    b[k] = keep + __shfl_xor(send, 2, 64);
+  }
+  double s = (o2 ? b[1] : b[0]) + __shfl_xor(o2 ? b[0] : b[1], 4, 64);
+  s += __shfl_xor(s, 8, 64);
+  s += __shfl_xor(s, 16, 64);
+  s += __shfl_xor(s, 32, 64);
+  return s;
+}
+
 // Record of the pairs a force kernel evaluates (parity tests): when out is
 // not null every evaluated pair appends (i, j, class) with i < j original
 // indices; *count counts all of them, out holds the first cap.

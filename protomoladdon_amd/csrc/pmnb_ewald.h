@@ -87,14 +87,16 @@ __device__ __forceinline__ void ew_step(double s1, double c1, double &s,
   c = c2;
 }
 
-// Intramolecular correction force on atom i (:1105-1129): every excluded
-// pair of i, in row order, each pair evaluated by both of its atoms (no
-// atomics).
-__device__ __forceinline__ void ew_correction_force(const EwDev &d,
-                                                    const double *x, int i,
-                                                    double &gx, double &gy,
-                                                    double &gz) {
-  for (int e = d.xptr[i]; e < d.xptr[i + 1]; e++) {
+// Intramolecular correction of atom i (:1105-1129): the force of every
+// lanes-th excluded pair of i from `sub` on, each pair evaluated by both of
+// its atoms (no atomics), its energy and virial (acc: energy, xx, xy, xz, yy,
+// yz, zz) by the first.
+__device__ __forceinline__ void ew_correction(const EwDev &d, const double *x,
+                                              int i, int sub, int lanes,
+                                              double &gx, double &gy,
+                                              double &gz, double (&acc)[7]) {
+  const int e1 = d.xptr[i + 1];
+  for (int e = d.xptr[i] + sub; e < e1; e += lanes) {
     const int row = d.xent[e] >> 1, role = d.xent[e] & 1;
     const int a1 = d.xrows[3 * row], a2 = d.xrows[3 * row + 1],
               cls = d.xrows[3 * row + 2];
@@ -104,16 +106,24 @@ __device__ __forceinline__ void ew_correction_force(const EwDev &d,
     double qq = d.q[a1] * d.q[a2];
     if (cls == 1) qq *= 1 - d.csf;  // EXCLUSION_MODIFIED
     const double r = sqrt(r2), rr = 1 / r;
-    const double e1 = erf(d.alpha * r) * rr;
-    const double g = qq * (d.two_alpha_pi * exp(-d.alpha2 * r2) - e1) * rr * rr;
+    const double er = erf(d.alpha * r) * rr;
+    const double g = qq * (d.two_alpha_pi * exp(-d.alpha2 * r2) - er) * rr * rr;
+    const double fx = rx * g, fy = ry * g, fz = rz * g;
     if (role == 0) {
-      gx -= rx * g;
-      gy -= ry * g;
-      gz -= rz * g;
+      gx -= fx;
+      gy -= fy;
+      gz -= fz;
+      acc[0] -= qq * er;
+      acc[1] += fx * rx;
+      acc[2] += fx * ry;
+      acc[3] += fx * rz;
+      acc[4] += fy * ry;
+      acc[5] += fy * rz;
+      acc[6] += fz * rz;
     } else {
-      gx += rx * g;
-      gy += ry * g;
-      gz += rz * g;
+      gx += fx;
+      gy += fy;
+      gz += fz;
     }
   }
 }
@@ -302,7 +312,8 @@ __global__ __launch_bounds__(64 * kEwLanes) void k_ew_force(EwDev d,
     gy += part_f[w][part][1][lane];
     gz += part_f[w][part][2][lane];
   }
-  ew_correction_force(d, x, i, gx, gy, gz);
+  double unused[7] = {0, 0, 0, 0, 0, 0, 0};  // k_ew_partials adds those
+  ew_correction(d, x, i, 0, 1, gx, gy, gz, unused);
   f[3 * i] += gx;
   f[3 * i + 1] += gy;
   f[3 * i + 2] += gz;

@@ -6,31 +6,34 @@
 // kernels.
 //
 // One evaluation:
-//   k_pme_spread     one thread per atom: grid coordinates x = r n / L
+//   k_pme_bin        one thread per atom: grid coordinates x = r n / L
 //                    wrapped into [0, n) as Grid::anterpolateCharge does
-//                    (Grid.h:107-131), the B-spline weights of
-//                    BSpline::set (BSpline.cpp:58-95), and q Mx My Mz onto
-//                    the order^3 stencil as 64-bit fixed-point integers
-//                    (2^-40) with atomics: integer sums do not depend on
-//                    the order of the adds, so the grid is the same bits
-//                    on every run;
-//   k_pme_to_real    the integer grid to FP64, and cleared for the next run;
+//                    (Grid.h:107-131), written with the charge into the
+//                    bucket of the atom's bin (4^3 grid cells);
+//   k_pme_spread     one block per tile of 8^3 grid points: the atoms of the
+//                    bins that reach it, the B-spline weights of
+//                    BSpline::set (BSpline.cpp:58-95), and q Mx My Mz summed
+//                    over them in LDS as 64-bit fixed-point integers (2^-40):
+//                    integer sums do not depend on the order of the adds, so
+//                    the grid is the same bits on every run;
 //   hipFFT D2Z       the unnormalised transform of the real grid (nx, ny,
 //                    nz/2 + 1 half spectrum; the reference transforms the
 //                    full complex grid, whose other half is the conjugate);
-//   k_pme_scalar     one thread per spectrum point of the half spectrum,
+//   k_pme_scalar     one wave per row of the half spectrum,
 //                    the loop of Grid::scalarSum (Grid.h:237-341): theta(m)
 //                    = B(m) exp(-pi^2 m^2 / alpha^2) / (pi V m^2), energy
 //                    and virial terms (doubled where the reference doubles
 //                    them), the spectrum multiplied by theta; per-block sums
-//                    in a fixed tree;
+//                    in a fixed order; clears the bins for the next run;
 //   hipFFT Z2D       back to the real, convolved grid;
-//   k_pme_gather     one thread per atom: the force -q grad (the convolved
+//   k_pme_gather     two lanes per atom: the force -q grad (the convolved
 //                    grid) n / L, interpolateForce's loop (Grid.h:171-199),
-//                    plus the atom's correction pairs; no atomics;
-//   k_pme_finish     the blocks' energy and virial sums in block order,
-//                    half of them into the output (the reference returns
-//                    energy * 0.5 and adds virial * 0.5).
+//                    plus the atom's correction pairs, with their energy and
+//                    virial; no atomics;
+//   k_pme_finish     the blocks' energy and virial sums in a fixed order,
+//                    half of the grid's into the output (the reference
+//                    returns energy * 0.5 and adds virial * 0.5), and the
+//                    correction, self and charged-system terms.
 #pragma once
 
 #include "pmnb_ewald.h"
@@ -38,6 +41,13 @@
 namespace pmnb {
 
 constexpr int kPmeBlock = 256;
+constexpr int kPmeTile = 8;      // grid points of a spread tile, per axis
+constexpr int kPmeBin = 4;       // grid cells of an atom bin, per axis
+constexpr int kPmeList = 512;    // atoms of a tile listed in LDS
+constexpr int kPmeRow = kPmeTile + 1;  // LDS row and plane strides of a tile:
+constexpr int kPmePlane = kPmeTile * kPmeRow;  // an atom's planes on other banks
+constexpr int kPmeScalarBlocks = 4096;
+constexpr int kPmeLanes = 2;     // lanes per atom of the gather
 constexpr int kPmeSums = 7;  // energy, xx, xy, xz, yy, yz, zz
 // Charge grid resolution 2^-40: with order 8 on a 32^3 grid the rounding of
 // 2^-32 moves forces by 1e-9 of the largest, 2^-40 by 3e-12.  A grid value
@@ -56,13 +66,21 @@ struct PmeDev {
   double piVr;             // 1 / (pi V)
   double fac;              // pi^2 / alpha^2
   const double *q;         // scaled charges
-  long long *qfix;         // nx ny nz fixed-point grid (zero between runs)
+  int nb[3];               // atom bins per axis
+  int *count;              // atoms per bin, then of the overflow list (zero
+                           // between runs)
+  double4 *bucket;         // cap records {grid x, y, z, charge} per bin
+  double4 *over;           // records beyond a bin's bucket
+  int cap;
   double *qreal;           // nx ny nz real grid
   double2 *qk;             // nx ny nzh half spectrum
   const double *mod[3];    // B(m) per axis index (Grid::dftmod)
   const double *ex[3];     // exp(-fac m^2) per axis index (ex[2]: k <= nz/2)
-  double *part;            // kPmeSums per scalar-sum block
+  double *part;            // kPmeSums rows of n_part scalar-sum blocks
   int n_part;              // scalar-sum blocks
+  double *cpart;           // kPmeSums rows of n_cpart gather blocks: the
+                           // correction's energy and virial
+  int n_cpart;
 };
 
 // BSpline::set(w) (BSpline.cpp:58-95) with compile-time order P >= 2, in
@@ -117,124 +135,262 @@ __device__ __forceinline__ double pme_coord(double p, double hr, int n) {
   return x;
 }
 
-template <int P>
-__global__ __launch_bounds__(kPmeBlock) void k_pme_spread(PmeDev d,
-                                                          const double *x) {
+// Grid index b + u, b in [0, 2 n), u < n, brought below n.
+__device__ __forceinline__ int pme_wrap(int g, int n) {
+  g -= g >= 2 * n ? 2 * n : 0;
+  return g >= n ? g - n : g;
+}
+
+// Atoms beyond a bin's bucket go to the overflow list, which every tile reads
+// whole.  The order in a bucket varies from run to run; the integer sums of
+// the tiles do not.
+__global__ __launch_bounds__(kPmeBlock) void k_pme_bin(PmeDev d,
+                                                       const double *x) {
   const int i = blockIdx.x * kPmeBlock + threadIdx.x;
   if (i >= d.n) return;
-  const double q = d.q[i];
-  const int nn[3] = {d.nx, d.ny, d.nz};
-  int b[3];
-  double th[3][P], dth[3][P];
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    const double g = pme_coord(x[3 * i + a], d.hr[a], nn[a]);
-    const int ig = (int)g;
-    pme_bspline<P>(g - ig, th[a], dth[a]);
-    b[a] = ig + d.off[a];
+  const double4 r = make_double4(pme_coord(x[3 * i], d.hr[0], d.nx),
+                                 pme_coord(x[3 * i + 1], d.hr[1], d.ny),
+                                 pme_coord(x[3 * i + 2], d.hr[2], d.nz), d.q[i]);
+  const int b = (((int)r.x / kPmeBin) * d.nb[1] + (int)r.y / kPmeBin) * d.nb[2] +
+                (int)r.z / kPmeBin;
+  const int k = atomicAdd(d.count + b, 1);
+  if (k < d.cap) {
+    d.bucket[(size_t)b * d.cap + k] = r;
+  } else {
+    const int o = atomicAdd(d.count + (size_t)d.nb[0] * d.nb[1] * d.nb[2], 1);
+    d.over[o] = r;
   }
+}
+
+// Adds the contributions of stencil plane u of one atom that fall into the
+// tile at t0 of extent te.
+template <int P>
+__device__ __forceinline__ void pme_spread_plane(const PmeDev &d,
+                                                 const double4 &r, int u,
+                                                 const int (&t0)[3],
+                                                 const int (&te)[3],
+                                                 unsigned long long *tile) {
+  const int ix = (int)r.x, iy = (int)r.y, iz = (int)r.z;
+  const int lx = pme_wrap(ix + d.off[0] + u, d.nx) - t0[0];
+  if ((unsigned)lx >= (unsigned)te[0]) return;
+  double tx[P], ty[P], tz[P], dth[P];
+  pme_bspline<P>(r.x - ix, tx, dth);
+  pme_bspline<P>(r.y - iy, ty, dth);
+  pme_bspline<P>(r.z - iz, tz, dth);
+  double mx = tx[0];
 #pragma unroll
-  for (int u = 0; u < P; u++) {
-    const double av = q * th[0][u];
-    const int i1 = (u + b[0]) % d.nx;
+  for (int k = 1; k < P; k++) mx = u == k ? tx[k] : mx;
+  const double av = r.w * mx;
+  // |value| <= |charge| < 2048: adding 1.5 * 2^12 leaves the value rounded to
+  // 2^-40 in the low bits, the rounding of rint
+  const bool small = fabs(r.w) < 2048.0;
 #pragma unroll
-    for (int v = 0; v < P; v++) {
-      const double ab = av * th[1][v];
-      const int j1 = (v + b[1]) % d.ny;
-      long long *row = d.qfix + ((size_t)i1 * d.ny + j1) * d.nz;
+  for (int v = 0; v < P; v++) {
+    const int ly = pme_wrap(iy + d.off[1] + v, d.ny) - t0[1];
+    if ((unsigned)ly >= (unsigned)te[1]) continue;
+    const double ab = av * ty[v];
+    unsigned long long *row = tile + lx * kPmePlane + ly * kPmeRow;
 #pragma unroll
-      for (int w = 0; w < P; w++) {
-        const int k1 = (w + b[2]) % d.nz;
-        double val = ab * th[2][w];
+    for (int w = 0; w < P; w++) {
+      const int lz = pme_wrap(iz + d.off[2] + w, d.nz) - t0[2];
+      if ((unsigned)lz >= (unsigned)te[2]) continue;
+      double val = ab * tz[w];
+      unsigned long long fix;
+      if (small) {
+        fix = (unsigned long long)__double_as_longlong(val + 6144.0) -
+              0x40B8000000000000ull;
+      } else {
         val = fmin(fmax(val, -kPmeFixClamp), kPmeFixClamp);
-        atomicAdd(reinterpret_cast<unsigned long long *>(row + k1),
-                  (unsigned long long)(long long)__builtin_rint(val * kPmeFixScale));
+        fix = (unsigned long long)(long long)__builtin_rint(val * kPmeFixScale);
       }
+      __hip_atomic_fetch_add(row + lz, fix, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
     }
   }
 }
 
-__global__ __launch_bounds__(kPmeBlock) void k_pme_to_real(PmeDev d,
-                                                           long long total) {
-  const long long g = (long long)blockIdx.x * kPmeBlock + threadIdx.x;
-  if (g >= total) return;
-  d.qreal[g] = (double)d.qfix[g] * kPmeFixInv;
-  d.qfix[g] = 0;
-}
-
-__device__ __forceinline__ double pme_block_sum(double v, double *red) {
+// One block per tile of 8^3 grid points (fewer at the upper faces).  Its
+// points are written by it alone, so no global atomics: 6.1 million of them
+// took 156 us for 96,000 atoms of order 4 on a 96^3 grid, plus 8 us to convert
+// and clear the integer grid; this kernel takes 30 us and k_pme_bin 10 (bound by
+// its atomics' latency), this one by VALU issue, 38% of the lanes' stencil points
+// being in the tile.  Bins half a tile wide: 4 per axis reach a tile, 8 atoms
+// are read for one of the tile's own (27 with bins of a tile).  The listed atoms are spread over the
+// lanes by stencil plane, which evens out what the tile's edge cuts off.
+template <int P>
+__global__ __launch_bounds__(kPmeBlock) void k_pme_spread(PmeDev d) {
+  __shared__ unsigned long long tile[kPmeTile * kPmePlane];
+  __shared__ double4 list[kPmeList];
+  __shared__ int nlist;
   const int t = threadIdx.x;
-  red[t] = v;
-  __syncthreads();
-  for (int o = kPmeBlock / 2; o > 0; o >>= 1) {
-    if (t < o) red[t] += red[t + o];
+  const int nn[3] = {d.nx, d.ny, d.nz};
+  const int nty = (d.ny + kPmeTile - 1) / kPmeTile,
+            ntz = (d.nz + kPmeTile - 1) / kPmeTile;
+  const int b = blockIdx.x;
+  const int tc[3] = {b / (nty * ntz), b / ntz % nty, b % ntz};
+  int t0[3], te[3], first[3], cnt[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    t0[a] = tc[a] * kPmeTile;
+    te[a] = min(kPmeTile, nn[a] - t0[a]);
+    // cells of the atoms that reach the tile: t0 - P / 2 .. end + (P - 1) / 2;
+    // when they leave less than a bin of the axis, every bin once
+    const int lo = t0[a] - P / 2, hi = t0[a] + te[a] - 1 + (P - 1) / 2;
+    if (hi - lo + 1 > nn[a] - kPmeBin) {
+      first[a] = 0;
+      cnt[a] = d.nb[a];
+    } else {
+      first[a] = (lo < 0 ? lo + nn[a] : lo) / kPmeBin;
+      const int last = (hi >= nn[a] ? hi - nn[a] : hi) / kPmeBin;
+      cnt[a] = last - first[a] + (last < first[a] ? d.nb[a] : 0) + 1;
+    }
+  }
+  for (int k = t; k < kPmeTile * kPmePlane; k += kPmeBlock) tile[k] = 0;
+  const int nbin = cnt[0] * cnt[1] * cnt[2];
+  const int nover = d.count[(size_t)d.nb[0] * d.nb[1] * d.nb[2]];
+  auto reach = [&](double c, int a) -> bool {  // the atom's stencil meets it
+    int g = (int)c + d.off[a] - t0[a];  // first point, from the tile's
+    g = g < 0 ? g + nn[a] : g;
+    g = g >= 2 * nn[a] ? g - 2 * nn[a] : (g >= nn[a] ? g - nn[a] : g);
+    return g < te[a] || g + P > nn[a];
+  };
+  auto take = [&](const double4 &r) {
+    if (!(reach(r.x, 0) && reach(r.y, 1) && reach(r.z, 2))) return;
+    const int k = __hip_atomic_fetch_add(&nlist, 1, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (k < kPmeList) {
+      list[k] = r;
+    } else {  // a full list: this lane adds the atom itself
+      for (int u = 0; u < P; u++) pme_spread_plane<P>(d, r, u, t0, te, tile);
+    }
+  };
+  // four lanes per bin, 64 bins a turn; then the overflow list
+  const int turns = (nbin + 63) / 64;
+  for (int turn = 0; turn <= turns; turn++) {
+    if (turn == turns && nover == 0) break;
+    if (t == 0) nlist = 0;
+    __syncthreads();
+    if (turn < turns) {
+      const int k = turn * 64 + (t >> 2);
+      if (k < nbin) {
+        int bx = first[0] + k / (cnt[1] * cnt[2]),
+            by = first[1] + k / cnt[2] % cnt[1], bz = first[2] + k % cnt[2];
+        bx -= bx >= d.nb[0] ? d.nb[0] : 0;
+        by -= by >= d.nb[1] ? d.nb[1] : 0;
+        bz -= bz >= d.nb[2] ? d.nb[2] : 0;
+        const int bin = (bx * d.nb[1] + by) * d.nb[2] + bz;
+        const int n = min(d.count[bin], d.cap);
+        const double4 *rec = d.bucket + (size_t)bin * d.cap;
+        for (int s = t & 3; s < n; s += 4) take(rec[s]);
+      }
+    } else {
+      for (int s = t; s < nover; s += kPmeBlock) take(d.over[s]);
+    }
+    __syncthreads();
+    const int items = min(nlist, kPmeList) * P;
+    for (int k = t; k < items; k += kPmeBlock)
+      pme_spread_plane<P>(d, list[k / P], k % P, t0, te, tile);
     __syncthreads();
   }
-  const double r = red[0];
-  __syncthreads();
-  return r;
+  for (int k = t; k < kPmeTile * kPmeTile * kPmeTile; k += kPmeBlock) {
+    const int lx = k / (kPmeTile * kPmeTile), ly = k / kPmeTile % kPmeTile,
+              lz = k % kPmeTile;
+    if (lx < te[0] && ly < te[1] && lz < te[2])
+      d.qreal[((size_t)(t0[0] + lx) * d.ny + t0[1] + ly) * d.nz + t0[2] + lz] =
+          (double)(long long)tile[lx * kPmePlane + ly * kPmeRow + lz] * kPmeFixInv;
+  }
 }
 
+// Sums of kPmeSums values over the block: rows of part, column blockIdx.x, in
+// a fixed order (lanes by halving, then the waves in turn).
+__device__ __forceinline__ void pme_store_sums(double (&acc)[kPmeSums],
+                                               double *part, int n_part) {
+  __shared__ double red[kPmeBlock / 64][8];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const double v8[8] = {acc[0], acc[1], acc[2], acc[3],
+                        acc[4], acc[5], acc[6], 0.0};
+  const double s = wave_sum8(v8, lane);
+  if (lane < 8) red[wave][lane] = s;
+  __syncthreads();
+  if (threadIdx.x < kPmeSums) {
+    double v = 0.0;
+#pragma unroll
+    for (int w = 0; w < kPmeBlock / 64; w++) v += red[w][threadIdx.x];
+    part[(size_t)threadIdx.x * n_part + blockIdx.x] = v;
+  }
+}
+
+// One wave per (x, y) row of the spectrum, lanes over z: the row's factors
+// are wave-uniform.  Bound by the read and write of the spectrum, 14 MB for
+// 96^3, and its latency: 8.4 us (11 with one thread per point, 64-bit
+// index divisions and a barrier tree per sum).
 __global__ __launch_bounds__(kPmeBlock) void k_pme_scalar(PmeDev d,
                                                           int virial) {
-  __shared__ double red[kPmeBlock];
-  const long long idx = (long long)blockIdx.x * kPmeBlock + threadIdx.x;
-  const long long total = (long long)d.nx * d.ny * d.nzh;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(
+      (int)(blockIdx.x * (kPmeBlock / 64) + (threadIdx.x >> 6)));
+  // the spread of this run is done: clear its bins for the next
+  const long long nclear = (long long)d.nb[0] * d.nb[1] * d.nb[2] + 1;
+  for (long long k = (long long)blockIdx.x * kPmeBlock + threadIdx.x; k < nclear;
+       k += (long long)gridDim.x * kPmeBlock)
+    d.count[k] = 0;
   double acc[kPmeSums];
 #pragma unroll
   for (int c = 0; c < kPmeSums; c++) acc[c] = 0.0;
-  if (idx < total) {
-    const int k = (int)(idx % d.nzh);
-    const int j = (int)((idx / d.nzh) % d.ny);
-    const int i = (int)(idx / ((long long)d.nzh * d.ny));
-    double2 s = d.qk[idx];
-    if (i == 0 && j == 0 && k == 0) {
-      s = make_double2(0.0, 0.0);
-    } else {
-      const int i0 = i <= d.nx / 2 ? i : i - d.nx;
-      const int j0 = j <= d.ny / 2 ? j : j - d.ny;
-      const int k0 = k <= d.nz / 2 ? k : k - d.nz;
-      const double mi = i0 * d.Lr[0], mj = j0 * d.Lr[1], mk = k0 * d.Lr[2];
-      const double exv = d.ex[0][i] * d.piVr;
-      const double modxy = d.mod[0][i] * d.mod[1][j];
-      const double mij = mi * mi + mj * mj;
-      const double exy = exv * d.ex[1][j];
+  const int rows = d.nx * d.ny, nw = gridDim.x * (kPmeBlock / 64);
+  for (int row = wave; row < rows; row += nw) {
+    const int i = row / d.ny, j = row - i * d.ny;
+    const int i0 = i <= d.nx / 2 ? i : i - d.nx;
+    const int j0 = j <= d.ny / 2 ? j : j - d.ny;
+    const double mi = i0 * d.Lr[0], mj = j0 * d.Lr[1];
+    const double modxy = d.mod[0][i] * d.mod[1][j];
+    const double mij = mi * mi + mj * mj;
+    const double exy = d.ex[0][i] * d.piVr * d.ex[1][j];
+    double2 *qk = d.qk + (size_t)row * d.nzh;
+    for (int k = lane; k < d.nzh; k += 64) {
+      double2 s = qk[k];
+      const double mk = k * d.Lr[2];
       const double m2 = mij + mk * mk;
-      const double theta = modxy * d.mod[2][k] * exy * d.ex[2][k] / m2;
+      const double im2 = 1.0 / m2;
+      const bool zero = row == 0 && k == 0;
+      const double theta =
+          zero ? 0.0 : modxy * d.mod[2][k] * exy * d.ex[2][k] * im2;
       const double qq = s.x * s.x + s.y * s.y;
       double e = qq * theta;
-      const double v = 2.0 * (1.0 / m2 + d.fac);
       if (k > 0 && ((k != d.nz / 2) || (d.nz & 1))) e *= 2.0;
-      acc[0] = e;
-      if (virial) {
-        acc[1] = e * (1.0 - v * mi * mi);
-        acc[2] = -(e * (v * mi * mj));
-        acc[3] = -(e * (v * mi * mk));
-        acc[4] = e * (1.0 - v * mj * mj);
-        acc[5] = -(e * (v * mj * mk));
-        acc[6] = e * (1.0 - v * mk * mk);
+      acc[0] += e;
+      if (virial && !zero) {
+        const double v = 2.0 * (im2 + d.fac);
+        acc[1] += e * (1.0 - v * mi * mi);
+        acc[2] -= e * (v * mi * mj);
+        acc[3] -= e * (v * mi * mk);
+        acc[4] += e * (1.0 - v * mj * mj);
+        acc[5] -= e * (v * mj * mk);
+        acc[6] += e * (1.0 - v * mk * mk);
       }
-      s.x *= theta;
-      s.y *= theta;
+      s.x = zero ? 0.0 : s.x * theta;
+      s.y = zero ? 0.0 : s.y * theta;
+      qk[k] = s;
     }
-    d.qk[idx] = s;
   }
-  double *out = d.part + (size_t)blockIdx.x * kPmeSums;
-#pragma unroll
-  for (int c = 0; c < kPmeSums; c++) {
-    const double t = pme_block_sum(acc[c], red);
-    if (threadIdx.x == 0) out[c] = t;
-  }
+  pme_store_sums(acc, d.part, d.n_part);
 }
 
-// Force of the reciprocal term on each atom and the correction forces of
-// its excluded pairs (ew_correction_force), added to f in a fixed order.
+// Force of the reciprocal term on each atom and the correction of its
+// excluded pairs (ew_correction), added to f in a fixed order.  kPmeLanes lanes
+// take the stencil planes and the excluded pairs of an atom in turn: one lane
+// per atom leaves 1.5 waves a SIMD on 96,000 atoms, with 64 grid values and two
+// erf in one chain each: 16 us, and 15 us more for a pass over the excluded
+// pairs' energies.  Two lanes take 15 us for both; four take 24, the weights
+// and the erf of a wave with idle lanes being computed twice as often.
 template <int P>
 __global__ __launch_bounds__(kPmeBlock) void k_pme_gather(PmeDev d, EwDev e,
                                                           const double *x,
                                                           double *f) {
-  const int i = blockIdx.x * kPmeBlock + threadIdx.x;
-  if (i >= d.n) return;
+  const int at = blockIdx.x * (kPmeBlock / kPmeLanes) + threadIdx.x / kPmeLanes;
+  const int sub = threadIdx.x % kPmeLanes;
+  const bool in = at < d.n;
+  const int i = in ? at : d.n - 1;  // past the end: a real atom, not written
   const int nn[3] = {d.nx, d.ny, d.nz};
   int b[3];
   double th[3][P], dth[3][P];
@@ -245,53 +401,100 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_gather(PmeDev d, EwDev e,
     pme_bspline<P>(g - ig, th[a], dth[a]);
     b[a] = ig + d.off[a];
   }
+  int zk[P];
+#pragma unroll
+  for (int w = 0; w < P; w++) zk[w] = pme_wrap(b[2] + w, d.nz);
   double fx = 0.0, fy = 0.0, fz = 0.0;
 #pragma unroll
-  for (int u = 0; u < P; u++) {
-    const int i1 = (u + b[0]) % d.nx;
+  for (int u0 = 0; u0 < P; u0 += kPmeLanes) {
+    const int u = u0 + sub;
+    if (u >= P) break;
+    double tx = 0.0, dx = 0.0;
+#pragma unroll
+    for (int k = u0; k < P && k < u0 + kPmeLanes; k++) {
+      tx = u == k ? th[0][k] : tx;
+      dx = u == k ? dth[0][k] : dx;
+    }
+    const double *plane = d.qreal + (size_t)pme_wrap(b[0] + u, d.nx) * d.ny * d.nz;
+    double sx = 0.0, sy = 0.0, sz = 0.0;
 #pragma unroll
     for (int v = 0; v < P; v++) {
-      const int j1 = (v + b[1]) % d.ny;
-      const double xij = dth[0][u] * th[1][v];
-      const double yij = th[0][u] * dth[1][v];
-      const double zij = th[0][u] * th[1][v];
-      const double *row = d.qreal + ((size_t)i1 * d.ny + j1) * d.nz;
+      const double *row = plane + (size_t)pme_wrap(b[1] + v, d.ny) * d.nz;
+      double s0 = 0.0, s1 = 0.0;
 #pragma unroll
       for (int w = 0; w < P; w++) {
-        const double term = row[(w + b[2]) % d.nz];
-        fx -= term * xij * th[2][w];
-        fy -= term * yij * th[2][w];
-        fz -= term * zij * dth[2][w];
+        const double term = row[zk[w]];
+        s0 = fma(term, th[2][w], s0);
+        s1 = fma(term, dth[2][w], s1);
       }
+      sx = fma(th[1][v], s0, sx);
+      sy = fma(dth[1][v], s0, sy);
+      sz = fma(th[1][v], s1, sz);
     }
+    fx = fma(-dx, sx, fx);
+    fy = fma(-tx, sy, fy);
+    fz = fma(-tx, sz, fz);
   }
   const double q = d.q[i];
   double gx = fx * d.hr[0] * q, gy = fy * d.hr[1] * q, gz = fz * d.hr[2] * q;
-  ew_correction_force(e, x, i, gx, gy, gz);
-  f[3 * i] += gx;
-  f[3 * i + 1] += gy;
-  f[3 * i + 2] += gz;
+  double acc[kPmeSums];
+#pragma unroll
+  for (int c = 0; c < kPmeSums; c++) acc[c] = 0.0;
+  if (in) ew_correction(e, x, i, sub, kPmeLanes, gx, gy, gz, acc);
+#pragma unroll
+  for (int o = 1; o < kPmeLanes; o <<= 1) {
+    gx += __shfl_xor(gx, o);
+    gy += __shfl_xor(gy, o);
+    gz += __shfl_xor(gz, o);
+  }
+  if (in && sub == 0) {
+    f[3 * i] += gx;
+    f[3 * i + 1] += gy;
+    f[3 * i + 2] += gz;
+  }
+  pme_store_sums(acc, d.cpart, d.n_cpart);
 }
 
-// One wave: lane c < kPmeSums adds sum c of every block in block order;
-// out[1] += energy / 2, and with the virial flag the virial slots XX..ZZ
-// += the virial sums / 2 (Grid.h:316-326).
-__global__ __launch_bounds__(64) void k_pme_finish(PmeDev d, double *out,
-                                                   int virial) {
-  __shared__ double tot[kPmeSums];
-  const int t = threadIdx.x;
-  if (t < kPmeSums) {
-    double v = 0.0;
-    for (int b = 0; b < d.n_part; b++) v += d.part[(size_t)b * kPmeSums + t];
-    tot[t] = v;
+// Wave w < 14 adds one of the sums over the blocks (lanes by stride, then by
+// halving: a fixed order; one lane per sum took 235 us over 1,764 blocks).
+// out[1] += energy / 2 + correction + constant energies, and with the virial
+// flag the virial slots XX..ZZ += the virial sums / 2 (Grid.h:316-326), the
+// correction's and the charged-system diagonal.
+__global__ __launch_bounds__(1024) void k_pme_finish(PmeDev d, double *out,
+                                                     int virial, double e_const,
+                                                     double e_charged) {
+  __shared__ double tot[2 * kPmeSums];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (w < 2 * kPmeSums) {
+    const bool corr = w >= kPmeSums;
+    const int n = corr ? d.n_cpart : d.n_part;
+    const double *p = (corr ? d.cpart : d.part) +
+                      (size_t)(corr ? w - kPmeSums : w) * n;
+    double v0 = 0.0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
+    int b = lane;
+    for (; b + 192 < n; b += 256) {
+      v0 += p[b];
+      v1 += p[b + 64];
+      v2 += p[b + 128];
+      v3 += p[b + 192];
+    }
+    for (; b < n; b += 64) v0 += p[b];
+    const double v = ew_wave_sum((v0 + v1) + (v2 + v3));
+    if (lane == 0) tot[w] = v;
   }
   __syncthreads();
-  if (t == 0) {
-    out[1] += tot[0] * 0.5;
+  if (threadIdx.x == 0) {
+    const double *c = tot + kPmeSums;
+    out[1] += tot[0] * 0.5 + c[0] + e_const;
     if (virial) {
-      out[2] += tot[1] * 0.5; out[3] += tot[2] * 0.5; out[4] += tot[3] * 0.5;
-      out[5] += tot[2] * 0.5; out[6] += tot[4] * 0.5; out[7] += tot[5] * 0.5;
-      out[8] += tot[3] * 0.5; out[9] += tot[5] * 0.5; out[10] += tot[6] * 0.5;
+      const double xx = tot[1] * 0.5 + c[1] + e_charged;
+      const double xy = tot[2] * 0.5 + c[2], xz = tot[3] * 0.5 + c[3];
+      const double yy = tot[4] * 0.5 + c[4] + e_charged;
+      const double yz = tot[5] * 0.5 + c[5];
+      const double zz = tot[6] * 0.5 + c[6] + e_charged;
+      out[2] += xx; out[3] += xy; out[4] += xz;
+      out[5] += xy; out[6] += yy; out[7] += yz;
+      out[8] += xz; out[9] += yz; out[10] += zz;
     }
   }
 }
