@@ -2957,13 +2957,105 @@ void correction_csr(int n_atoms, int n_excl, const int32_t *excl,
 
 }  // namespace
 
+namespace {
+
+// Tiles of the k-space matrix products over the runs (contiguous k of one h,
+// h ascending).  A tile's columns and steps end at the largest |l| of its k,
+// so the cut-off sphere costs no more than its edge.
+void ew_tiles(const std::vector<EwRun> &runs, int &n_pass, std::vector<EwH> &hs,
+              std::vector<EwTile> &tiles, std::vector<EwFTile> &ftiles,
+              std::vector<int2> &fsteps) {
+  auto top = [](const EwRun &r) {
+    return std::max(std::abs(r.l_lo), std::abs(r.l_hi)) + 1;  // orders 0 .. |l|
+  };
+  n_pass = 1;
+  for (const EwRun &r : runs)
+    n_pass = std::max(n_pass, (top(r) + kEwOrders - 1) / kEwOrders);
+  std::vector<std::vector<int>> forders(n_pass);  // per pass and force tile
+  for (size_t r0 = 0; r0 < runs.size();) {
+    size_t r1 = r0;
+    while (r1 < runs.size() && runs[r1].h == runs[r0].h) r1++;
+    const int h = runs[r0].h, kmin = runs[r0].k, kmax = runs[r1 - 1].k;
+    hs.resize(h + 1, EwH{0, -1, 0, 0});
+    hs[h] = EwH{kmin, kmax, (int)ftiles.size(), (int)r0};
+    const int ka = std::max(std::abs(kmin), std::abs(kmax));
+    std::vector<int> orders(ka + 4, 0);  // by |k|
+    for (size_t r = r0; r < r1; r++) {
+      int &o = orders[std::abs(runs[r].k)];
+      o = std::max(o, top(runs[r]));
+    }
+    for (int k0 = 0; k0 <= ka; k0 += 4) {
+      const int o = *std::max_element(&orders[k0], &orders[k0] + 4);
+      for (int m0 = 0; m0 < o; m0 += kEwOrders)
+        tiles.push_back(
+            EwTile{h, k0, m0, (std::min(o - m0, kEwOrders) + 7) / 8});
+    }
+    for (int k0 = kmin; k0 <= kmax; k0 += 4) {
+      ftiles.push_back(EwFTile{h, k0});
+      int o = 0;
+      for (int k = k0; k <= std::min(k0 + 3, kmax); k++)
+        o = std::max(o, top(runs[r0 + (k - kmin)]));
+      for (int p = 0; p < n_pass; p++)
+        forders[p].push_back(
+            std::max(0, std::min(o - p * kEwOrders, (int)kEwOrders)));
+    }
+    r0 = r1;
+  }
+  int at = 0;
+  for (int p = 0; p < n_pass; p++)
+    for (int o : forders[p]) {
+      const int steps = (o + 3) / 4 * 2;  // 2 o columns, an even number of fours
+      fsteps.push_back(make_int2(at, steps));
+      at += steps;
+    }
+  // tiles of one pass and similar width share a block
+  std::sort(tiles.begin(), tiles.end(), [](const EwTile &a, const EwTile &b) {
+    if (a.m0 != b.m0) return a.m0 < b.m0;
+    if (a.nc != b.nc) return a.nc > b.nc;
+    return a.h != b.h ? a.h < b.h : a.k0 < b.k0;
+  });
+  std::vector<EwTile> padded;
+  for (size_t i = 0; i < tiles.size(); i++) {
+    if (i && tiles[i].m0 != tiles[i - 1].m0)
+      while (padded.size() % kEwTiles) padded.push_back(EwTile{0, 0, tiles[i - 1].m0, 0});
+    padded.push_back(tiles[i]);
+  }
+  while (padded.size() % kEwTiles)
+    padded.push_back(EwTile{0, 0, padded.back().m0, 0});
+  tiles.swap(padded);
+}
+
+// First force tile of each split, and the end: about equal matrix steps (and
+// three for a tile's own work), at least one tile each (n_split <= n_ft).
+std::vector<int> ew_splits(const std::vector<int2> &fsteps, int n_ft, int n_pass,
+                           int n_split) {
+  std::vector<long long> upto(n_ft + 1, 0);
+  for (int f = 0; f < n_ft; f++) {
+    upto[f + 1] = upto[f] + 3;
+    for (int p = 0; p < n_pass; p++)
+      upto[f + 1] += fsteps[(size_t)p * n_ft + f].y;
+  }
+  std::vector<int> first(n_split + 1, 0);
+  for (int s = 1; s <= n_split; s++) {
+    int f = first[s - 1] + 1;
+    while (f < n_ft && upto[f] * n_split < upto[n_ft] * s) f++;
+    first[s] = std::min(f, n_ft - (n_split - s));
+  }
+  first[n_split] = n_ft;
+  return first;
+}
+
+}  // namespace
+
 struct pmnb_ewald {
   pmnb_ctx *ctx = nullptr;
   int device = 0, n = 0, nk = 0, H = 0, n_excl = 0;
   double alpha = 0, alpha2 = 0, rc = 0, kc = 0, fac = 0, V = 0, Vr = 0;
   double csf = 1.0, e_self = 0, e_charged = 0;
-  int n_runs = 0, n_chunks = 0;
-  DevBuf kv, q, tab, sk, kf, part, xptr, xent, xrows, runs, chunks;
+  int n_tiles = 0, n_chunks = 0, chunk = 0;
+  int n_ft = 0, n_split = 0, n_pass = 0, n_cpart = 0;
+  DevBuf kv, q, tab, C, P, pf, part, cpart, xptr, xent, xrows, runs, hs, tiles,
+      ftiles, fsteps, fsplit;
   // the box and topology the k-vectors, charges and rows were built for
   double box_key[12] = {0};
   unsigned long long topo_gen = 0;
@@ -3045,26 +3137,35 @@ int pmnb_ewald_create(pmnb_ctx *ctx, double alpha, double accuracy,
     }
   }
   ew->nk = (int)kv.size();
-  // runs of equal (h, k) (contiguous l) and their chunks of l values
+  // runs of equal (h, k) (contiguous l)
   std::vector<EwRun> runs;
-  std::vector<EwChunk> chunks;
   for (int i = 0; i < ew->nk; i++) {
     if (runs.empty() || runs.back().h != hkl[i].x || runs.back().k != hkl[i].y)
       runs.push_back(EwRun{hkl[i].x, hkl[i].y, hkl[i].z, hkl[i].z, i});
     else
       runs.back().l_hi = hkl[i].z;
   }
-  // chunks of |l| values, both signs of l in one chunk: |l| runs over
-  // [m_lo, m_hi], the |l| of the run's l interval
-  for (int r = 0; r < (int)runs.size(); r++) {
-    const int lo = runs[r].l_lo, hi = runs[r].l_hi;
-    const int m_hi = std::max(std::abs(lo), std::abs(hi));
-    const int m_lo = (lo <= 0 && hi >= 0) ? 0 : std::min(std::abs(lo), std::abs(hi));
-    for (int m0 = m_lo; m0 <= m_hi; m0 += kEwChunk)
-      chunks.push_back(EwChunk{r, m0, std::min(m0 + kEwChunk - 1, m_hi)});
-  }
-  ew->n_runs = (int)runs.size();
-  ew->n_chunks = (int)chunks.size();
+  std::vector<EwH> hs;
+  std::vector<EwTile> tiles;
+  std::vector<EwFTile> ftiles;
+  std::vector<int2> fsteps;
+  std::vector<int> fsplit;
+  ew_tiles(runs, ew->n_pass, hs, tiles, ftiles, fsteps);
+  ew->n_tiles = (int)tiles.size();
+  ew->n_ft = (int)ftiles.size();
+  // 1,536 blocks of k_ew_sk (two of three resident a CU), at least 64 atoms each; 8,192 waves of
+  // k_ew_force
+  const int nblk = std::max(1, ew->n_tiles / kEwTiles);
+  ew->n_chunks = std::max(1, std::min(blocks_for(1536, nblk),
+                                      blocks_for(n_atoms, 64)));
+  ew->chunk = kEwStage * std::max(1, blocks_for(n_atoms, ew->n_chunks * kEwStage));
+  ew->n_chunks = std::max(1, blocks_for(n_atoms, ew->chunk));
+  const int nwave = 4 * std::max(1, blocks_for(n_atoms, 4 * kEwAtoms));
+  ew->n_split = std::min(std::min(blocks_for(8192, nwave), 64), ew->n_ft);
+  fsplit = ew_splits(fsteps, ew->n_ft, ew->n_pass, ew->n_split);
+  const int total_steps =
+      fsteps.empty() ? 0 : fsteps.back().x + fsteps.back().y;
+  ew->n_cpart = blocks_for(std::max(n_atoms, 1), 256 / kEwFinalLanes);
   double q2 = 0.0, qs = 0.0;
   for (int i = 0; i < n_atoms; i++) q2 += scaled_charge[i] * scaled_charge[i];
   for (int i = 0; i < n_atoms; i++) qs += scaled_charge[i];
@@ -3086,14 +3187,31 @@ int pmnb_ewald_create(pmnb_ctx *ctx, double alpha, double accuracy,
   if (e == hipSuccess) e = up(ew->q, scaled_charge, (size_t)n_atoms * sizeof(double));
   if (e == hipSuccess)
     e = ew->tab.ensure((size_t)3 * ew->H * 2 * std::max(n_atoms, 1) * sizeof(double));
-  if (e == hipSuccess) e = ew->sk.ensure((size_t)std::max(ew->nk, 1) * sizeof(double2));
-  if (e == hipSuccess) e = ew->kf.ensure((size_t)std::max(ew->nk, 1) * sizeof(EwKF));
-  if (e == hipSuccess) e = ew->part.ensure((size_t)kEwFinBlocks * kEwFinSums * sizeof(double));
+  if (e == hipSuccess)
+    e = ew->C.ensure((size_t)ew->n_chunks * ew->n_tiles * 16 * kEwCols *
+                     sizeof(double));
+  // entries of no k-vector stay zero; four steps are read past the end
+  const size_t pbytes = (size_t)(total_steps + 6) * 64 * sizeof(double);
+  if (e == hipSuccess) e = ew->P.ensure(pbytes);
+  if (e == hipSuccess) e = hipMemset(ew->P.p, 0, pbytes);
+  if (e == hipSuccess)
+    e = ew->pf.ensure((size_t)ew->n_split * n_atoms * 3 * sizeof(double));
+  if (e == hipSuccess)
+    e = ew->part.ensure((size_t)ew->n_tiles * kEwSums * sizeof(double));
+  if (e == hipSuccess)
+    e = ew->cpart.ensure((size_t)ew->n_cpart * kEwSums * sizeof(double));
   if (e == hipSuccess) e = up(ew->xptr, cnt.data(), (n_atoms + 1) * sizeof(int));
   if (e == hipSuccess) e = up(ew->xent, ent.data(), 2 * (size_t)n_excl * sizeof(int));
   if (e == hipSuccess) e = up(ew->xrows, excl, 3 * (size_t)n_excl * sizeof(int));
   if (e == hipSuccess) e = up(ew->runs, runs.data(), runs.size() * sizeof(EwRun));
-  if (e == hipSuccess) e = up(ew->chunks, chunks.data(), chunks.size() * sizeof(EwChunk));
+  if (e == hipSuccess) e = up(ew->hs, hs.data(), hs.size() * sizeof(EwH));
+  if (e == hipSuccess) e = up(ew->tiles, tiles.data(), tiles.size() * sizeof(EwTile));
+  if (e == hipSuccess)
+    e = up(ew->ftiles, ftiles.data(), ftiles.size() * sizeof(EwFTile));
+  if (e == hipSuccess)
+    e = up(ew->fsteps, fsteps.data(), fsteps.size() * sizeof(int2));
+  if (e == hipSuccess)
+    e = up(ew->fsplit, fsplit.data(), fsplit.size() * sizeof(int));
   if (e != hipSuccess) {
     pmnb_ewald_destroy(ew);
     return fail(ctx, PMNB_ERR_HIP, "Ewald set-up failed: %s", hipGetErrorString(e));
@@ -3139,14 +3257,26 @@ int pmnb_ewald_evaluate_device(pmnb_ewald *ew, const double *d_positions,
   d.H = ew->H;
   d.kv = ew->kv.as<double4>();
   d.runs = ew->runs.as<EwRun>();
-  d.chunks = ew->chunks.as<EwChunk>();
-  d.n_runs = ew->n_runs;
+  d.hs = ew->hs.as<EwH>();
+  d.tiles = ew->tiles.as<EwTile>();
+  d.n_tiles = ew->n_tiles;
   d.n_chunks = ew->n_chunks;
+  d.chunk = ew->chunk;
+  d.ftiles = ew->ftiles.as<EwFTile>();
+  d.fsteps = ew->fsteps.as<int2>();
+  d.fsplit = ew->fsplit.as<int>();
+  d.n_ft = ew->n_ft;
+  d.n_split = ew->n_split;
+  d.n_pass = ew->n_pass;
   d.q = ew->q.as<double>();
   d.tab = ew->tab.as<double>();
-  d.sk = ew->sk.as<double2>();
-  d.kf = ew->kf.as<EwKF>();
+  d.C = ew->C.as<double>();
+  d.P = ew->P.as<double>();
+  d.pf = ew->pf.as<double>();
   d.part = ew->part.as<double>();
+  d.cpart = ew->cpart.as<double>();
+  d.n_cpart = ew->n_cpart;
+  for (int a = 0; a < 3; a++) d.kunit[a] = 2.0 * M_PI * ctx->box.er[a];
   d.xptr = ew->xptr.as<int>();
   d.xent = ew->xent.as<int>();
   d.xrows = ew->xrows.as<int>();
@@ -3157,20 +3287,20 @@ int pmnb_ewald_evaluate_device(pmnb_ewald *ew, const double *d_positions,
   d.csf = ew->csf;
   d.Vr = ew->Vr;
   d.fac = ew->fac;
-  const int nb = blocks_for(ew->n, kEwBlock);
-  hipLaunchKernelGGL(k_ew_tables, dim3(nb), dim3(kEwBlock), 0, s, d, d_positions);
-  if (ew->n_chunks > 0)
-    hipLaunchKernelGGL(k_ew_sk, dim3(ew->n_chunks), dim3(kEwBlock), 0, s, d);
-  const int nbf = blocks_for(ew->n, 64 * kEwAtomsLarge);
-  if (nbf >= 256)
-    hipLaunchKernelGGL((k_ew_force<kEwLanesLarge, kEwAtomsLarge>), dim3(nbf),
-                       dim3(64 * kEwLanesLarge), 0, s, d, d_positions, d_forces);
-  else
-    hipLaunchKernelGGL((k_ew_force<kEwLanesSmall, 2>), dim3(blocks_for(ew->n, 128)),
-                       dim3(64 * kEwLanesSmall), 0, s, d, d_positions, d_forces);
-  hipLaunchKernelGGL(k_ew_partials, dim3(kEwFinBlocks), dim3(kEwBlock), 0, s, d,
-                     d_positions);
-  hipLaunchKernelGGL(k_ew_finish, dim3(1), dim3(64), 0, s, d, d_out,
+  if (ew->nk > 0) {
+    hipLaunchKernelGGL(k_ew_tables, dim3(blocks_for(ew->n, 64)), dim3(192), 0, s,
+                       d, d_positions);
+    hipLaunchKernelGGL(k_ew_sk, dim3(ew->n_chunks, ew->n_tiles / kEwTiles),
+                       dim3(256), 0, s, d);
+    hipLaunchKernelGGL(k_ew_coef, dim3(ew->n_tiles), dim3(kEwCoefBlock), 0, s, d);
+    hipLaunchKernelGGL(k_ew_force,
+                       dim3(blocks_for(ew->n, 4 * kEwAtoms), ew->n_split),
+                       dim3(256), 0, s, d);
+  }
+  hipLaunchKernelGGL(k_ew_final, dim3(ew->n_cpart), dim3(256), 0, s, d,
+                     d_positions, d_forces);
+  hipLaunchKernelGGL(k_ew_finish, dim3(1), dim3(1024), 0, s, d.part, d.n_tiles,
+                     d.cpart, d.n_cpart, 4.0 * M_PI * d.Vr, d_out,
                      (int)((flags & PMNB_FLAG_VIRIAL) != 0),
                      ew->e_self + ew->e_charged, ew->e_charged);
   HIPCHK(hipGetLastError());
@@ -3181,8 +3311,10 @@ void pmnb_ewald_destroy(pmnb_ewald *ew) {
   if (!ew) return;
   (void)hipSetDevice(ew->device);
   (void)hipDeviceSynchronize();
-  DevBuf *bufs[] = {&ew->kv, &ew->q, &ew->tab, &ew->sk, &ew->kf, &ew->part,
-                    &ew->xptr, &ew->xent, &ew->xrows, &ew->runs, &ew->chunks};
+  DevBuf *bufs[] = {&ew->kv, &ew->q, &ew->tab, &ew->C, &ew->P, &ew->pf,
+                    &ew->part, &ew->cpart, &ew->xptr, &ew->xent, &ew->xrows,
+                    &ew->runs, &ew->hs, &ew->tiles, &ew->ftiles, &ew->fsteps,
+                    &ew->fsplit};
   for (DevBuf *b : bufs) b->release();
   delete ew;
 }
@@ -3455,9 +3587,9 @@ int pmnb_pme_create(pmnb_ctx *ctx, int32_t nx, int32_t ny, int32_t nz,
   if (e == hipSuccess) e = up(pm->mod, mod.data(), mod.size() * sizeof(double));
   if (e == hipSuccess) e = up(pm->ex, ex.data(), ex.size() * sizeof(double));
   if (e == hipSuccess)
-    e = pm->part.ensure((size_t)pm->n_part * kPmeSums * sizeof(double));
+    e = pm->part.ensure((size_t)pm->n_part * kEwSums * sizeof(double));
   if (e == hipSuccess)
-    e = pm->cpart.ensure((size_t)pm->n_cpart * kPmeSums * sizeof(double));
+    e = pm->cpart.ensure((size_t)pm->n_cpart * kEwSums * sizeof(double));
   if (e == hipSuccess) e = up(pm->xptr, cnt.data(), (n_atoms + 1) * sizeof(int));
   if (e == hipSuccess) e = up(pm->xent, ent.data(), 2 * (size_t)n_excl * sizeof(int));
   if (e == hipSuccess) e = up(pm->xrows, rows.data(), rows.size() * sizeof(int));
@@ -3533,7 +3665,8 @@ int pmnb_pme_evaluate_device(pmnb_pme *pm, const double *d_positions,
     case 6: pme_launch_gather<6>(pm, d, e, d_positions, d_forces, s); break;
     default: pme_launch_gather<8>(pm, d, e, d_positions, d_forces, s); break;
   }
-  hipLaunchKernelGGL(k_pme_finish, dim3(1), dim3(1024), 0, s, d, d_out, virial,
+  hipLaunchKernelGGL(k_ew_finish, dim3(1), dim3(1024), 0, s, d.part, d.n_part,
+                     d.cpart, d.n_cpart, 0.5, d_out, virial,
                      pm->e_self + pm->e_charged, pm->e_charged);
   HIPCHK(hipGetLastError());
   return PMNB_OK;

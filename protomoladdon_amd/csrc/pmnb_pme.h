@@ -30,9 +30,9 @@
 //                    grid) n / L, interpolateForce's loop (Grid.h:171-199),
 //                    plus the atom's correction pairs, with their energy and
 //                    virial; no atomics;
-//   k_pme_finish     the blocks' energy and virial sums in a fixed order,
-//                    half of the grid's into the output (the reference
-//                    returns energy * 0.5 and adds virial * 0.5), and the
+//   k_ew_finish      the blocks' energy and virial sums, half of the grid's
+//                    into the output (the reference returns energy * 0.5
+//                    and adds virial * 0.5, Grid.h:316-326), and the
 //                    correction, self and charged-system terms.
 #pragma once
 
@@ -48,7 +48,6 @@ constexpr int kPmeRow = kPmeTile + 1;  // LDS row and plane strides of a tile:
 constexpr int kPmePlane = kPmeTile * kPmeRow;  // an atom's planes on other banks
 constexpr int kPmeScalarBlocks = 4096;
 constexpr int kPmeLanes = 2;     // lanes per atom of the gather
-constexpr int kPmeSums = 7;  // energy, xx, xy, xz, yy, yz, zz
 // Charge grid resolution 2^-40: with order 8 on a 32^3 grid the rounding of
 // 2^-32 moves forces by 1e-9 of the largest, 2^-40 by 3e-12.  A grid value
 // must stay below 2^23 (8.4e6, about 4.6e5 elementary charges on one grid
@@ -76,9 +75,9 @@ struct PmeDev {
   double2 *qk;             // nx ny nzh half spectrum
   const double *mod[3];    // B(m) per axis index (Grid::dftmod)
   const double *ex[3];     // exp(-fac m^2) per axis index (ex[2]: k <= nz/2)
-  double *part;            // kPmeSums rows of n_part scalar-sum blocks
+  double *part;            // kEwSums rows of n_part scalar-sum blocks
   int n_part;              // scalar-sum blocks
-  double *cpart;           // kPmeSums rows of n_cpart gather blocks: the
+  double *cpart;           // kEwSums rows of n_cpart gather blocks: the
                            // correction's energy and virial
   int n_cpart;
 };
@@ -301,25 +300,6 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_spread(PmeDev d) {
   }
 }
 
-// Sums of kPmeSums values over the block: rows of part, column blockIdx.x, in
-// a fixed order (lanes by halving, then the waves in turn).
-__device__ __forceinline__ void pme_store_sums(double (&acc)[kPmeSums],
-                                               double *part, int n_part) {
-  __shared__ double red[kPmeBlock / 64][8];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const double v8[8] = {acc[0], acc[1], acc[2], acc[3],
-                        acc[4], acc[5], acc[6], 0.0};
-  const double s = wave_sum8(v8, lane);
-  if (lane < 8) red[wave][lane] = s;
-  __syncthreads();
-  if (threadIdx.x < kPmeSums) {
-    double v = 0.0;
-#pragma unroll
-    for (int w = 0; w < kPmeBlock / 64; w++) v += red[w][threadIdx.x];
-    part[(size_t)threadIdx.x * n_part + blockIdx.x] = v;
-  }
-}
-
 // One wave per (x, y) row of the spectrum, lanes over z: the row's factors
 // are wave-uniform.  Bound by the read and write of the spectrum, 14 MB for
 // 96^3, and its latency: 8.4 us (11 with one thread per point, 64-bit
@@ -334,9 +314,9 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_scalar(PmeDev d,
   for (long long k = (long long)blockIdx.x * kPmeBlock + threadIdx.x; k < nclear;
        k += (long long)gridDim.x * kPmeBlock)
     d.count[k] = 0;
-  double acc[kPmeSums];
+  double acc[kEwSums];
 #pragma unroll
-  for (int c = 0; c < kPmeSums; c++) acc[c] = 0.0;
+  for (int c = 0; c < kEwSums; c++) acc[c] = 0.0;
   const int rows = d.nx * d.ny, nw = gridDim.x * (kPmeBlock / 64);
   for (int row = wave; row < rows; row += nw) {
     const int i = row / d.ny, j = row - i * d.ny;
@@ -373,7 +353,7 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_scalar(PmeDev d,
       qk[k] = s;
     }
   }
-  pme_store_sums(acc, d.part, d.n_part);
+  ew_store_sums<kPmeBlock / 64>(acc, d.part, d.n_part);
 }
 
 // Force of the reciprocal term on each atom and the correction of its
@@ -437,9 +417,9 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_gather(PmeDev d, EwDev e,
   }
   const double q = d.q[i];
   double gx = fx * d.hr[0] * q, gy = fy * d.hr[1] * q, gz = fz * d.hr[2] * q;
-  double acc[kPmeSums];
+  double acc[kEwSums];
 #pragma unroll
-  for (int c = 0; c < kPmeSums; c++) acc[c] = 0.0;
+  for (int c = 0; c < kEwSums; c++) acc[c] = 0.0;
   if (in) ew_correction(e, x, i, sub, kPmeLanes, gx, gy, gz, acc);
 #pragma unroll
   for (int o = 1; o < kPmeLanes; o <<= 1) {
@@ -452,51 +432,7 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_gather(PmeDev d, EwDev e,
     f[3 * i + 1] += gy;
     f[3 * i + 2] += gz;
   }
-  pme_store_sums(acc, d.cpart, d.n_cpart);
-}
-
-// Wave w < 14 adds one of the sums over the blocks (lanes by stride, then by
-// halving: a fixed order; one lane per sum took 235 us over 1,764 blocks).
-// out[1] += energy / 2 + correction + constant energies, and with the virial
-// flag the virial slots XX..ZZ += the virial sums / 2 (Grid.h:316-326), the
-// correction's and the charged-system diagonal.
-__global__ __launch_bounds__(1024) void k_pme_finish(PmeDev d, double *out,
-                                                     int virial, double e_const,
-                                                     double e_charged) {
-  __shared__ double tot[2 * kPmeSums];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  if (w < 2 * kPmeSums) {
-    const bool corr = w >= kPmeSums;
-    const int n = corr ? d.n_cpart : d.n_part;
-    const double *p = (corr ? d.cpart : d.part) +
-                      (size_t)(corr ? w - kPmeSums : w) * n;
-    double v0 = 0.0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
-    int b = lane;
-    for (; b + 192 < n; b += 256) {
-      v0 += p[b];
-      v1 += p[b + 64];
-      v2 += p[b + 128];
-      v3 += p[b + 192];
-    }
-    for (; b < n; b += 64) v0 += p[b];
-    const double v = ew_wave_sum((v0 + v1) + (v2 + v3));
-    if (lane == 0) tot[w] = v;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const double *c = tot + kPmeSums;
-    out[1] += tot[0] * 0.5 + c[0] + e_const;
-    if (virial) {
-      const double xx = tot[1] * 0.5 + c[1] + e_charged;
-      const double xy = tot[2] * 0.5 + c[2], xz = tot[3] * 0.5 + c[3];
-      const double yy = tot[4] * 0.5 + c[4] + e_charged;
-      const double yz = tot[5] * 0.5 + c[5];
-      const double zz = tot[6] * 0.5 + c[6] + e_charged;
-      out[2] += xx; out[3] += xy; out[4] += xz;
-      out[5] += xy; out[6] += yy; out[7] += yz;
-      out[8] += xz; out[9] += yz; out[10] += zz;
-    }
-  }
+  ew_store_sums<kPmeBlock / 64>(acc, d.cpart, d.n_cpart);
 }
 
 }  // namespace pmnb
