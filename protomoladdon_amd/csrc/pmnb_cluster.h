@@ -205,7 +205,9 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
       const int k = lane >> 1, part = lane & 1;
       const int kx = k / 5, ky = k - 5 * kx;
       const int ox = wx ? kx - cx : kx - 2, oy = wy ? ky - cy : ky - 2;
-      bool ok = k < 25 && !(wx && kx >= G.nx) && !(wy && ky >= G.ny);
+      // (no run without a live atom: the box is empty and so are the z ranges)
+      bool ok = k < 25 && bz0 <= bz1 && !(wx && kx >= G.nx) &&
+                !(wy && ky >= G.ny);
       int tx = cx + ox, ty = cy + oy;
       tx = tx < 0 ? tx + G.nx : (tx >= G.nx ? tx - G.nx : tx);
       ty = ty < 0 ? ty + G.ny : (ty >= G.ny ? ty - G.ny : ty);

@@ -117,3 +117,14 @@ def test_atoms_without_a_position_have_no_pairs(precision, bad):
     assert np.isfinite(f).all()
     assert rms_rel(f[rest], ref[0][rest]) <= (
         1e-5 if precision == "mixed" else 1e-12)
+
+
+@pytest.mark.parametrize("precision", ["mixed", "fp64"])
+@pytest.mark.parametrize("n_mol", [60, 500])
+def test_no_atom_has_a_position(precision, n_mol):
+    """Work items without one finite position, in a box that wraps per pair
+    (60 waters) and one that does not."""
+    w = systems.small_water(n_mol=n_mol)
+    p = np.full_like(w.positions, np.nan)
+    f, _, npairs, _ = run_gpu(w, precision, 0, positions=p, with_pairs=False)
+    assert npairs == 0 and not f.any()
