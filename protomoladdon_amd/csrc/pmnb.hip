@@ -766,10 +766,8 @@ void launch_pairs_mode(const PairArgs &a) {
 
 template <bool F64, int EL, int SW>
 void launch_pairs_types(const PairArgs &a) {
-  // the FP64 kernel always reads the table from memory
-  if constexpr (F64) launch_pairs_mode<true, EL, SW, false>(a);
-  else if (a.big_types) launch_pairs_mode<false, EL, SW, true>(a);
-  else launch_pairs_mode<false, EL, SW, false>(a);
+  if (a.big_types) launch_pairs_mode<F64, EL, SW, true>(a);
+  else launch_pairs_mode<F64, EL, SW, false>(a);
 }
 
 // Pair kernel of the tile path for the force's precision and functors.

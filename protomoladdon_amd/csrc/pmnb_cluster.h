@@ -48,7 +48,7 @@
 // pair where columns of one cutoff left 4.4.  Measured against that layout
 // with its z-level loop (3 x 3 columns, one z cell of the columns a time):
 //   96,000 atoms   160 -> 137 us forces only, 205 -> 157 with energies
-//   the same, FP64 540 -> 508
+//   the same, FP64 540 -> 412 (508 with IEEE quotients, roots and exp)
 //   522,000 atoms in 128 boxes  751 -> 603, 1,076 -> 690 (half shell before)
 //   3,000 atoms, 10 A Coulomb   104 -> 35 (a block an item)
 //   30,000 atoms of 12 types    1,293 (neighbour list) -> 83
@@ -99,8 +99,9 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
         double *__restrict__ forces, double *__restrict__ partial, int pstride,
         unsigned long long *__restrict__ npairs, PairLog plog) {
   using Real = typename std::conditional<F64, double, float>::type;
-  constexpr int BUF = F64 ? 192 : 256;   // records buffered per wave
+  constexpr int BUF = F64 ? 176 : 256;   // records buffered per wave
   constexpr bool kLjLds = !F64 && !BIGT;
+  constexpr bool kLjLds64 = F64 && !BIGT;
   __shared__ float4 recA[kTmWaves][BUF];    // x, y, z, |x|^2
   __shared__ float2 recB[kTmWaves][BUF];    // charge, atom << 8 | type
   __shared__ int recT[kTmWaves][BUF];       // sorted slot
@@ -111,6 +112,8 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
   __shared__ float2 segL[F64 ? 1 : kTmWaves][F64 ? 1 : kSegs];
   __shared__ float2 ljA[kLjLds ? kLjTypes * kLjRow : 1];  // A, B
   __shared__ float2 ljM[kLjLds ? kLjTypes * kLjRow : 1];  // A14, B14
+  // FP64: A, B (the 1-4 values are read from memory)
+  __shared__ double2 ljD[kLjLds64 ? kLjTypes * kLjTypes : 1];
   __shared__ double combE[MODE ? kTmWaves : 1][MODE == kMolVirial ? 16 : 8];
   __shared__ long long combF[kTmWaves][3 * kTileAtoms];
   const int wave = uni((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
@@ -123,6 +126,12 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
       ljA[at] = make_float2(v.x, v.y);
       ljM[at] = make_float2(v.z, v.w);
     }
+    __syncthreads();
+  }
+  if (kLjLds64) {
+    const int T = P.n_types;
+    for (int k = threadIdx.x; k < T * T; k += kBlock)
+      ljD[(k / T) * kLjTypes + k % T] = make_double2(S.lj[4 * k], S.lj[4 * k + 1]);
     __syncthreads();
   }
   const float hi = F.cut2 + F.band, lo = F.cut2 - F.band;
@@ -362,6 +371,13 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
           auto eval = [&](const float4 &A, const float2 &B, int k, bool valid,
                           auto WR, auto SAME) __attribute__((always_inline)) {
             const unsigned w = __float_as_uint(B.y);
+            double2 abd = make_double2(0.0, 0.0);
+            if constexpr (kLjLds64) {
+              abd = ljD[ti * kLjTypes + (w & 255u)];
+            } else if constexpr (F64) {
+              const double *lp = ljrow64 + 4 * (w & 255u);
+              abd = make_double2(lp[0], lp[1]);
+            }
             float2 ab = make_float2(0.f, 0.f);
             float4 ab4 = make_float4(0.f, 0.f, 0.f, 0.f);
             if constexpr (kLjLds) ab = ljr[w & 255u];
@@ -417,10 +433,14 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
               log_pair(plog, ai, (int)(w >> 8), cls);
             Real ff, e1, e2, ddx, ddy, ddz;
             if constexpr (F64) {
-              const double *lp = ljrow64 + 4 * (w & 255u);
-              pair_f64<ELEC, ELSW>(P, e2d, cls != 1 ? lp[0] : lp[2],
-                                   cls != 1 ? lp[1] : lp[3],
-                                   qi * recD[wave][k].w, cls, ff, e1, e2);
+              double q2 = qi * recD[wave][k].w;
+              if (cls == 1) {
+                const double *lp = ljrow64 + 4 * (w & 255u);
+                abd = make_double2(lp[2], lp[3]);
+                q2 *= P.csf;
+              }
+              pair_fma64<ELEC, ELSW, decltype(SAME)::value>(P, e2d, abd.x, abd.y,
+                                                            q2, ff, e1, e2);
               ddx = exd;
               ddy = eyd;
               ddz = ezd;
@@ -530,7 +550,7 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
             }
           };
           if (wrapped) run(std::true_type{}, std::false_type{});
-          else if (F64 || F.same_switch)
+          else if (F.same_switch)
             run(std::false_type{}, std::true_type{});
           else run(std::false_type{}, std::false_type{});
           if constexpr (F64) {
