@@ -227,7 +227,7 @@ struct pmnb_ctx {
   bool batch = false;
   DevBuf d_rep_of;
   int rep_uploaded = 0;           // reps and bin_rep are on the device
-  DevBuf d_partial_lj;            // adjoint: LJ-parameter partials per item
+  DevBuf d_partial_lj;            // adjoint: LJ-parameter gradients per atom
   DevBuf d_bucket, d_ccount;
   // d_count holds zeros at the start of the next evaluation on the tile path
   // (the finish kernel clears it after the pair kernel): no clearing launch
@@ -751,7 +751,7 @@ void launch_pairs_as(const PairArgs &a) {
   hipLaunchKernelGGL((k_pairs<F64, EL, SW, MODE, BIGT, LOG>), dim3(nb),
                      dim3(kBlock), 0, a.s, *a.P, *a.S, a.reps, a.items,
                      a.nslots, (int)split, a.forces, a.partial, a.nslots,
-                     a.npairs, a.log);
+                     a.npairs, a.log, AdjArgs{});
 }
 
 template <bool F64, int EL, int SW, bool BIGT>
@@ -826,37 +826,13 @@ AdjC<R> make_adj_consts(const ForceParams &P) {
   return C;
 }
 
-template <bool F64, int EL, int MK>
-void launch_adj(int max_items, hipStream_t s, const ForceParams &P,
-                const Sorted &S, const TileRep *reps, const int4 *items,
-                const int *nitems, const double *gf, double *gx, double *gq,
-                double *plj, unsigned long long *np) {
-  constexpr int NW = 1, BUF = 128;
-  const int nb = std::max(1, blocks_for(max_items, NW));
-  hipLaunchKernelGGL((k_tq_adj<F64, EL, NW, BUF, MK>), dim3(nb),
-                     dim3(64 * NW), 0, s, P, make_adj_consts<float>(P),
-                     make_adj_consts<double>(P), S, reps, items, nitems, gf,
-                     gx, gq, plj, max_items, np);
-}
-
 template <bool F64, int EL>
-void launch_adj_t(int T, int max_items, hipStream_t s, const ForceParams &P,
-                  const Sorted &S, const TileRep *reps, const int4 *items,
-                  const int *nitems, const double *gf, double *gx, double *gq,
-                  double *plj, double *glj, unsigned long long *np) {
-  if (T <= 2) {
-    launch_adj<F64, EL, 3>(max_items, s, P, S, reps, items, nitems, gf, gx,
-                           gq, plj, np);
-    if (glj)
-      hipLaunchKernelGGL(k_adj_lj_finish<3>, dim3(3 * 4), dim3(1024), 0, s,
-                         plj, max_items, nitems, T, glj);
-  } else {
-    launch_adj<F64, EL, 10>(max_items, s, P, S, reps, items, nitems, gf, gx,
-                            gq, plj, np);
-    if (glj)
-      hipLaunchKernelGGL(k_adj_lj_finish<10>, dim3(10 * 4), dim3(1024), 0, s,
-                         plj, max_items, nitems, T, glj);
-  }
+void launch_adj(const PairArgs &a, const AdjArgs &adj) {
+  const int nb = 8 * std::max(1, blocks_for(blocks_for(a.nslots, kTmWaves), 8));
+  hipLaunchKernelGGL((k_pairs<F64, EL, 0, kAdjoint, false, false>), dim3(nb),
+                     dim3(kBlock), 0, a.s, *a.P, *a.S, a.reps, a.items,
+                     a.nslots, 0, (double *)nullptr, (double *)nullptr, a.nslots,
+                     a.npairs, a.log, adj);
 }
 
 // The per-evaluation device arrays of run_device: the context's own
@@ -1751,37 +1727,47 @@ int pmnb_adjoint_device(pmnb_ctx *ctx, const double *d_positions,
   hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
   rc = ensure_eval_buffers(ctx);
   if (rc) return rc;
-  const int max_items = std::max(ctx->nslots, 1);
-  HIPCHK(ctx->d_partial_lj.ensure((size_t)max_items * 10 * 4 *
-                                  sizeof(double)));
+  const size_t rows = (size_t)kAdjRows * std::max(ctx->n, 1);
+  HIPCHK(ctx->d_partial_lj.ensure(
+      (rows + (size_t)kAdjChunks * kAdjRows * kAdjTypes) * sizeof(double)));
   rc = build_cells(ctx, ctx_bufs(ctx), d_positions, s);
   if (rc) return rc;
   const ForceParams P = make_params(ctx, 0);
   const Sorted S = make_sorted(ctx, ctx_bufs(ctx), nullptr);
-  const TileRep *reps = ctx->d_reps.as<TileRep>();
-  int4 *items = ctx->d_items.as<int4>();
-  int *nitems = ctx->d_rep_items.as<int>();
   if (ctx->n > 0) {
     const bool f64 = ctx->prm.precision == PMNB_PREC_FP64;
-    const int el = ctx->prm.elec, T = ctx->ntypes;
+    const int el = ctx->prm.elec;
     double *plj = ctx->d_partial_lj.as<double>();
-    unsigned long long *np = ctx->d_npairs.as<unsigned long long>();
+    unsigned long long *np = ctx->d_npairs.as<unsigned long long>() + 1;
     ctx->last_np = np;
-    ctx->last_np_per = 1;
-#define PMNB_ADJ(F, E)                                                        \
-  launch_adj_t<F, E>(T, max_items, s, P, S, reps, items, nitems,              \
-                     d_grad_forces, d_grad_positions, d_grad_charges, plj,    \
-                     d_grad_lj, np)
+    ctx->last_np_per = 2;
+    PairArgs a{};
+    a.s = s;
+    a.P = &P;
+    a.S = &S;
+    a.reps = ctx->d_reps.as<TileRep>();
+    a.items = ctx->d_items.as<int4>();
+    a.nslots = ctx->nslots;
+    a.npairs = np;
+    const AdjArgs adj{d_grad_forces, d_grad_positions, d_grad_charges,
+                      d_grad_lj ? plj : nullptr, make_adj_consts<float>(P),
+                      make_adj_consts<double>(P)};
     if (f64) {
-      if (el == PMNB_ELEC_NONE) PMNB_ADJ(true, 0);
-      else if (el == PMNB_ELEC_COULOMB) PMNB_ADJ(true, 1);
-      else PMNB_ADJ(true, 2);
+      if (el == PMNB_ELEC_NONE) launch_adj<true, 0>(a, adj);
+      else if (el == PMNB_ELEC_COULOMB) launch_adj<true, 1>(a, adj);
+      else launch_adj<true, 2>(a, adj);
     } else {
-      if (el == PMNB_ELEC_NONE) PMNB_ADJ(false, 0);
-      else if (el == PMNB_ELEC_COULOMB) PMNB_ADJ(false, 1);
-      else PMNB_ADJ(false, 2);
+      if (el == PMNB_ELEC_NONE) launch_adj<false, 0>(a, adj);
+      else if (el == PMNB_ELEC_COULOMB) launch_adj<false, 1>(a, adj);
+      else launch_adj<false, 2>(a, adj);
     }
-#undef PMNB_ADJ
+    if (d_grad_lj) {
+      double *part = plj + rows;
+      hipLaunchKernelGGL(k_adj_lj_part, dim3(kAdjChunks, kAdjRows), dim3(kBlock),
+                         0, s, plj, S.type, ctx->n, part);
+      hipLaunchKernelGGL(k_adj_lj_finish, dim3(1), dim3(64), 0, s, part,
+                         ctx->ntypes, d_grad_lj);
+    }
   }
   HIPCHK(hipGetLastError());
   return PMNB_OK;

@@ -52,10 +52,13 @@
 //   522,000 atoms in 128 boxes  751 -> 603, 1,076 -> 690 (half shell before)
 //   3,000 atoms, 10 A Coulomb   104 -> 35 (a block an item)
 //   30,000 atoms of 12 types    1,293 (neighbour list) -> 83
+//   adjoint, 250,000 atoms      2,004 -> 780 (a queue of pairs and LDS slots
+//                               per atom left two waves a SIMD)
 #pragma once
 
 #include <type_traits>
 
+#include "pmnb_adjoint.h"
 #include "pmnb_bins.h"
 #include "pmnb_list.h"
 
@@ -68,8 +71,9 @@ constexpr int kSegs = 64;                   // runs of candidates per item
 constexpr int kLjRow = 16;                  // LDS row stride of the LJ table
 constexpr int kLjTypes = 8;                 // types held in LDS
 
-// What k_pairs forms beside the forces and the pair count.
-enum PairMode { kForces = 0, kEnergies = 1, kMolVirial = 2 };
+// What k_pairs forms beside the forces and the pair count; kAdjoint forms the
+// adjoint of the forces instead.
+enum PairMode { kForces = 0, kEnergies = 1, kMolVirial = 2, kAdjoint = 3 };
 
 // Index of the lowest set bit, -1 for 0 (v_ffbl_b32).
 __device__ __forceinline__ int ctz_or_none(unsigned m) {
@@ -93,19 +97,28 @@ __device__ __forceinline__ float slot_max(float v) {
 // block takes one item (a wave one stream); otherwise a wave takes an item.
 template <bool F64, int ELEC, int ELSW, int MODE, bool BIGT, bool LOG>
 __global__ void __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(F64 ? 3 : (MODE == kMolVirial ? 3 : 4))))
+__attribute__((amdgpu_waves_per_eu(
+    F64 ? (MODE == kAdjoint ? 2 : 3) : (MODE >= kMolVirial ? 3 : 4))))
 k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
         const int4 *__restrict__ items, int nslots, int split,
         double *__restrict__ forces, double *__restrict__ partial, int pstride,
-        unsigned long long *__restrict__ npairs, PairLog plog) {
+        unsigned long long *__restrict__ npairs, PairLog plog, AdjArgs adj) {
   using Real = typename std::conditional<F64, double, float>::type;
-  constexpr int BUF = F64 ? 176 : 256;   // records buffered per wave
+  constexpr bool kEn = MODE == kEnergies || MODE == kMolVirial;
+  constexpr bool kAdj = MODE == kAdjoint;
+  // records buffered per wave
+  constexpr int BUF = F64 ? (kAdj ? 128 : 176) : (kAdj ? 192 : 256);
   constexpr bool kLjLds = !F64 && !BIGT;
   constexpr bool kLjLds64 = F64 && !BIGT;
   __shared__ float4 recA[kTmWaves][BUF];    // x, y, z, |x|^2
   __shared__ float2 recB[kTmWaves][BUF];    // charge, atom << 8 | type
   __shared__ int recT[kTmWaves][BUF];       // sorted slot
   __shared__ double4 recD[F64 ? kTmWaves : 1][F64 ? BUF : 1];  // FP64 x, y, z, q
+  // adjoint: dL/dF of the record's atom, FP32 or FP64 as the pairs are
+  __shared__ float4 recG[kAdj && !F64 ? kTmWaves : 1][kAdj && !F64 ? BUF : 1];
+  __shared__ double4 recH[kAdj && F64 ? kTmWaves : 1][kAdj && F64 ? BUF : 1];
+  // ... and the lanes' LJ gradients of 1-4 pairs (few, so not in registers)
+  __shared__ Real ljm[kAdj ? kTmWaves : 1][kAdj ? 2 * kAdjTypes : 1][64];
   __shared__ int segE[kTmWaves][kSegs];     // end position of each run
   __shared__ int4 segI[kTmWaves][kSegs];    // x, y offset, cell and slot bases
   // what FP32 left of the offsets (FP64 pairs take the sorted positions)
@@ -114,7 +127,7 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
   __shared__ float2 ljM[kLjLds ? kLjTypes * kLjRow : 1];  // A14, B14
   // FP64: A, B (the 1-4 values are read from memory)
   __shared__ double2 ljD[kLjLds64 ? kLjTypes * kLjTypes : 1];
-  __shared__ double combE[MODE ? kTmWaves : 1][MODE == kMolVirial ? 16 : 8];
+  __shared__ double combE[kEn ? kTmWaves : 1][MODE == kMolVirial ? 16 : 8];
   __shared__ long long combF[kTmWaves][3 * kTileAtoms];
   const int wave = uni((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
   const F32Params &F = P.f;
@@ -183,6 +196,26 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
     const double xd = F64 && live ? S.x[ii] : 0.0,
                  yd = F64 && live ? S.y[ii] : 0.0,
                  zd = F64 && live ? S.z[ii] : 0.0;
+    // adjoint: the lane's dL/dF, in FP32 with its remainder
+    Real gi0 = 0, gi1 = 0, gi2 = 0, gl0 = 0, gl1 = 0, gl2 = 0;
+    if constexpr (kAdj) {
+      const double *g = adj.grad_f + 3 * (size_t)ai;
+      gi0 = (Real)g[0];
+      gi1 = (Real)g[1];
+      gi2 = (Real)g[2];
+      gl0 = (Real)(g[0] - (double)gi0);
+      gl1 = (Real)(g[1] - (double)gi1);
+      gl2 = (Real)(g[2] - (double)gi2);
+    }
+    // dL/d{A, B} / 2 by the partner's type
+    Real lj[kAdj ? kAdjTypes : 1][2];
+    if constexpr (kAdj)
+#pragma unroll
+      for (int c = 0; c < kAdjTypes; c++) {
+        lj[c][0] = lj[c][1] = Real(0);
+        ljm[wave][2 * c][lane] = ljm[wave][2 * c + 1][lane] = Real(0);
+      }
+    double fq64 = 0.0;
     const float2 *ljr = &ljA[kLjLds ? ti * kLjRow : 0];
     const float4 *ljrow = S.ljf + ti * P.n_types;
     const double *ljrow64 = S.lj + 4 * (ti * P.n_types);
@@ -359,7 +392,7 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
             m1 = J > 32 ? word(32, J - 32, test) : 0u;
           }
           cnt += __builtin_popcount(m0) + __builtin_popcount(m1);
-          Real px = 0, py = 0, pz = 0, pelj = 0, peel = 0;
+          Real px = 0, py = 0, pz = 0, pq = 0, pelj = 0, peel = 0;
           Real v0 = 0, v1 = 0, v2 = 0, v3 = 0, v4 = 0, v5 = 0;
           double mv[8];
           if (MODE == kMolVirial)
@@ -393,7 +426,7 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
               if (wz) fold(dz, L2, R.Llo[2], iL2);
             }
             const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-            float qq = li.w * B.x;
+            float qj = B.x;
             bool keep = valid;
             int cls = 0;
             if (valid && w - wlo < wrange) {
@@ -405,7 +438,7 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
                 cnt--;
               }
               if (!F64 && cls == 1) {
-                qq *= F.csf;
+                qj *= F.csf;
                 if constexpr (kLjLds) ab = ljM[ti * kLjRow + (w & 255u)];
                 else ab4 = make_float4(ab4.z, ab4.w, 0.f, 0.f);
               }
@@ -431,6 +464,57 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
             }
             if (LOG && keep && i < recT[wave][k])
               log_pair(plog, ai, (int)(w >> 8), cls);
+            if constexpr (kAdj) {
+              Real ff, ffp, h, dA, dB, q2, ddx, ddy, ddz, w0, w1, w2;
+              if constexpr (F64) {
+                if (cls == 1) {
+                  const double *lp = ljrow64 + 4 * (w & 255u);
+                  abd = make_double2(lp[2], lp[3]);
+                }
+                q2 = recD[wave][k].w * (cls == 1 ? P.csf : 1.0);
+                pair_adj<Real, ELEC, decltype(SAME)::value>(
+                    adj.c64, e2d, abd.x, abd.y, qi * q2, ff, ffp, h, dA, dB);
+                ddx = exd;
+                ddy = eyd;
+                ddz = ezd;
+                const double4 g = recH[wave][k];
+                w0 = g.x - gi0;
+                w1 = g.y - gi1;
+                w2 = g.z - gi2;
+              } else {
+                q2 = qj;
+                pair_adj<Real, ELEC, decltype(SAME)::value>(
+                    adj.c32, r2, ab.x, ab.y, li.w * qj, ff, ffp, h, dA, dB);
+                ddx = dx;
+                ddy = dy;
+                ddz = dz;
+                const float4 g = recG[wave][k];
+                w0 = (g.x - gi0) - gl0;
+                w1 = (g.y - gi1) - gl1;
+                w2 = (g.z - gi2) - gl2;
+              }
+              const Real wd = adj_fma(w0, ddx, adj_fma(w1, ddy, w2 * ddz));
+              const Real c2 = Real(2) * ffp * wd;
+              px -= keep ? adj_fma(ff, w0, c2 * ddx) : Real(0);
+              py -= keep ? adj_fma(ff, w1, c2 * ddy) : Real(0);
+              pz -= keep ? adj_fma(ff, w2, c2 * ddz) : Real(0);
+              pq += keep ? wd * q2 * h : Real(0);
+              const Real hA = keep ? Real(0.5) * wd * dA : Real(0);
+              const Real hB = keep ? Real(0.5) * wd * dB : Real(0);
+              const int tj = (int)(w & 255u);
+              if (cls == 1) {
+                ljm[wave][2 * tj][lane] += hA;
+                ljm[wave][2 * tj + 1][lane] += hB;
+              } else {
+#pragma unroll
+                for (int c = 0; c < kAdjTypes; c++) {
+                  lj[c][0] += tj == c ? hA : Real(0);
+                  lj[c][1] += tj == c ? hB : Real(0);
+                }
+              }
+              return;
+            }
+            const float qq = li.w * qj;
             Real ff, e1, e2, ddx, ddy, ddz;
             if constexpr (F64) {
               double q2 = qi * recD[wave][k].w;
@@ -553,7 +637,12 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
           else if (F.same_switch)
             run(std::false_type{}, std::true_type{});
           else run(std::false_type{}, std::false_type{});
-          if constexpr (F64) {
+          if constexpr (kAdj) {
+            fx64 += px;
+            fy64 += py;
+            fz64 += pz;
+            fq64 += pq;
+          } else if constexpr (F64) {
             sx64 += px;
             sy64 += py;
             sz64 += pz;
@@ -562,7 +651,7 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
             Fy += to_fixed_f32(py);
             Fz += to_fixed_f32(pz);
           }
-          if constexpr (MODE != kForces) {
+          if constexpr (kEn) {
             const double e[8] = {(double)pelj, (double)peel, (double)v0,
                                  (double)v1,   (double)v2,   (double)v3,
                                  (double)v4,   (double)v5};
@@ -579,10 +668,19 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
           recT[wave][pos] = t;
           if (F64)
             recD[wave][pos] = make_double4(S.x[t], S.y[t], S.z[t], S.q[t]);
+          if constexpr (kAdj) {
+            const double *g =
+                adj.grad_f + 3 * (size_t)(__float_as_uint(rb.y) >> 8);
+            if constexpr (F64)
+              recH[wave][pos] = make_double4(g[0], g[1], g[2], 0.0);
+            else
+              recG[wave][pos] =
+                  make_float4((float)g[0], (float)g[1], (float)g[2], 0.f);
+          }
         }
         nbuf += nb;
       }
-      if constexpr (F64) {
+      if constexpr (F64 && !kAdj) {
         // the four lanes of an atom, then the streams in order
         sx64 += __shfl_xor(sx64, 32, 64);
         sy64 += __shfl_xor(sy64, 32, 64);
@@ -596,6 +694,37 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
       }
       etot += erow;
       mtot += mrow;
+    }
+    if constexpr (kAdj) {  // never split
+      auto quad = [](double v) {
+        v += __shfl_xor(v, 32, 64);
+        return v + __shfl_xor(v, 16, 64);
+      };
+      fx64 = quad(fx64);
+      fy64 = quad(fy64);
+      fz64 = quad(fz64);
+      fq64 = quad(fq64);
+      if (active && sp == 0) {
+        if (adj.grad_x) {
+          double *f = adj.grad_x + 3 * (size_t)ai;
+          f[0] += fx64;
+          f[1] += fy64;
+          f[2] += fz64;
+        }
+        if (adj.grad_q) adj.grad_q[ai] += fq64;
+      }
+      if (adj.lj) {
+#pragma unroll
+        for (int c = 0; c < kAdjTypes; c++)
+#pragma unroll
+          for (int m = 0; m < 4; m++) {
+            double v = (double)(m < 2 ? lj[c][m] : ljm[wave][2 * c + m - 2][lane]);
+            v = quad(v);
+            if (active && sp == m)
+              adj.lj[(size_t)(4 * c + m) * P.n_atoms + i] = v;
+          }
+      }
+      continue;
     }
     if (!F64) {
       Fx += __shfl_xor(Fx, 32, 64);
@@ -613,7 +742,7 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
         combF[wave][slot + 2 * kTileAtoms] =
             F64 ? __double_as_longlong(fz64) : Fz;
       }
-      if constexpr (MODE != kForces) {
+      if constexpr (kEn) {
         if (lane < 8) {
           combE[wave][lane] = etot;
           if constexpr (MODE == kMolVirial) combE[wave][8 + lane] = mtot;
@@ -637,7 +766,7 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
             Fz += c;
           }
         }
-        if constexpr (MODE != kForces) {
+        if constexpr (kEn) {
           etot = mtot = 0.0;
 #pragma unroll
           for (int k = 0; k < kStreams; k++) {
@@ -663,7 +792,7 @@ k_pairs(ForceParams P, Sorted S, const TileRep *__restrict__ reps,
           f[2] += oz;
         }
       }
-      if constexpr (MODE != kForces) {
+      if constexpr (kEn) {
         // each pair is seen from both atoms: half of its energy and virial
         if (lane < 8) {
           partial[(size_t)lane * pstride + it] = 0.5 * etot;

@@ -1,6 +1,5 @@
-// Pieces the tile-path pair kernel (pmnb_cluster.h) and the adjoint
-// (pmnb_adjoint.h) share: the geometry of one replica (TileRep), the
-// per-replica reduction of the items' partial rows in a fixed order
+// Pieces the tile path's kernels share: the geometry of one replica (TileRep),
+// the per-replica reduction of the items' partial rows in a fixed order
 // (finish_rep_block), fixed-point conversion and scalar-register helpers.
 //
 // Each replica has its own column grid (TileRep): x/y columns at least half
@@ -9,9 +8,6 @@
 // is taken once with the minimum image of every pair along it (as z is when
 // the cutoff reaches all z cells), so small boxes keep the reference's
 // one-image pair set.
-//
-// The adjoint's records carry {sorted index | type << 24, molecule}; the LJ
-// table is held in LDS (at most kQLj entries).
 #pragma once
 
 #include <type_traits>
@@ -22,10 +18,8 @@
 
 namespace pmnb {
 
-constexpr int kQCap = 2048;   // adjoint pair-queue entries per wave
 constexpr int kQLj = 64;      // LJ table entries held in LDS
-constexpr int kQTypeShift = 24;
-constexpr int kQIndexMask = (1 << kQTypeShift) - 1;
+constexpr int kQTypeShift = 24;  // bits of an atom index beside its type
 
 // Geometry of one replica on the tile path.  Its atoms occupy the sorted
 // slots atom_off ..; they are sorted in bins (a bin: fz z cells of one

@@ -24,15 +24,6 @@ struct TileGrid {
   float lox, loy, loz;  // ... and what rounding to FP32 left of them
 };
 
-__device__ __forceinline__ float wave_min(float v) {
-  for (int m = 32; m > 0; m >>= 1) v = fminf(v, __shfl_xor(v, m, 64));
-  return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-  for (int m = 32; m > 0; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, 64));
-  return v;
-}
-
 __device__ __forceinline__ void wave_sync_lds() {
   // LDS written by some lanes of this wave is read by other lanes next.
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
