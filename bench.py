@@ -650,7 +650,7 @@ def main():
     # HBM bytes per launch of the pair kernel, from the committed rocprofv3
     # FETCH_SIZE / WRITE_SIZE passes (scaled by a copy kernel of known size)
     traffic = traffic_fo = None
-    tpath = os.path.join(ROOT, "profiles", "k_tile_water96k_traffic.json")
+    tpath = os.path.join(ROOT, "profiles", "pair_water96k_traffic.json")
     if os.path.exists(tpath):
         with open(tpath) as fh:
             tj = json.load(fh)
@@ -719,7 +719,7 @@ def main():
                      "traffic_unit": "bytes per launch (HBM, rocprofv3)",
                      "peak_without_packed_fp32": PEAK_FP64_TFLOPS,
                      "frac_without_packed_fp32": achieved / PEAK_FP64_TFLOPS,
-                     "kernel": "k_tile<mixed, Ewald-real, C2>",
+                     "kernel": "k_pairs<mixed, Ewald-real, C2>",
                      "kernel_ms": mx["kernel_ms"],
                      "cell_build_ms": mx["build_ms"],
                      "achieved_incl_cell_build": P * FLOP_PER_PAIR / (
@@ -728,7 +728,7 @@ def main():
                      # the dynamics' pair kernel (every evaluation of a
                      # run but its last): forces only, 73 of the 90 FLOP
                      "md_kernel": {
-                         "kernel": "k_tile<mixed, Ewald-real, C2, forces only>",
+                         "kernel": "k_pairs<mixed, Ewald-real, C2, forces only>",
                          "kernel_ms": md_mx["pair_kernel_ms_forces_only"],
                          "flop_per_pair": FLOP_PER_PAIR_FORCES,
                          "achieved": md_achieved,
