@@ -212,8 +212,8 @@ __device__ __forceinline__ void pme_spread_plane(const PmeDev &d,
 // points are written by it alone, so no global atomics: 6.1 million of them
 // took 156 us for 96,000 atoms of order 4 on a 96^3 grid, plus 8 us to convert
 // and clear the integer grid; this kernel takes 30 us and k_pme_bin 10 (bound by
-// its atomics' latency), this one by VALU issue, 38% of the lanes' stencil points
-// being in the tile.  Bins half a tile wide: 4 per axis reach a tile, 8 atoms
+// its atomics' latency), this one by its LDS atomics (a tile with margins, which
+// needs no test per point but adds 1.9 times as many, took 51).  Bins half a tile wide: 4 per axis reach a tile, 8 atoms
 // are read for one of the tile's own (27 with bins of a tile).  The listed atoms are spread over the
 // lanes by stencil plane, which evens out what the tile's edge cuts off.
 template <int P>
