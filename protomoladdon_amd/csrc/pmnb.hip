@@ -3631,14 +3631,30 @@ int pmnb_pme_evaluate_device(pmnb_pme *pm, const double *d_positions,
     case 6: pme_spread<6>(pm, d, d_positions, s); break;
     default: pme_spread<8>(pm, d, d_positions, s); break;
   }
-  HIPCHK(hipGetLastError());
+  // An evaluation that stops before k_pme_scalar clears the bins itself: the
+  // next one counts from zero.
+  auto clear_bins = [&]() {
+    const int nbin = pm->nb[0] * pm->nb[1] * pm->nb[2];
+    launch_fill_i32(d.count, nbin + 1, 0, s);
+  };
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) {
+    clear_bins();
+    HIPCHK(err);
+  }
   if (hipfftSetStream(pm->fwd, s) != HIPFFT_SUCCESS ||
       hipfftExecD2Z(pm->fwd, d.qreal, (hipfftDoubleComplex *)d.qk) !=
-          HIPFFT_SUCCESS)
+          HIPFFT_SUCCESS) {
+    clear_bins();
     return fail(ctx, PMNB_ERR_HIP, "hipFFT D2Z failed");
+  }
   hipLaunchKernelGGL(k_pme_scalar, dim3(pm->n_part), dim3(kPmeBlock), 0, s, d,
                      virial);
-  HIPCHK(hipGetLastError());
+  err = hipGetLastError();
+  if (err != hipSuccess) {
+    clear_bins();
+    HIPCHK(err);
+  }
   if (hipfftSetStream(pm->inv, s) != HIPFFT_SUCCESS ||
       hipfftExecZ2D(pm->inv, (hipfftDoubleComplex *)d.qk, d.qreal) !=
           HIPFFT_SUCCESS)

@@ -156,8 +156,10 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_bin(PmeDev d,
   if (k < d.cap) {
     d.bucket[(size_t)b * d.cap + k] = r;
   } else {
+    // (bounded whatever the counts held on entry: two evaluations of one
+    // object that overlap give wrong sums, not a write past the list)
     const int o = atomicAdd(d.count + (size_t)d.nb[0] * d.nb[1] * d.nb[2], 1);
-    d.over[o] = r;
+    if (o < d.n) d.over[o] = r;
   }
 }
 
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_spread(PmeDev d) {
   }
   for (int k = t; k < kPmeTile * kPmePlane; k += kPmeBlock) tile[k] = 0;
   const int nbin = cnt[0] * cnt[1] * cnt[2];
-  const int nover = d.count[(size_t)d.nb[0] * d.nb[1] * d.nb[2]];
+  const int nover = min(d.count[(size_t)d.nb[0] * d.nb[1] * d.nb[2]], d.n);
   auto reach = [&](double c, int a) -> bool {  // the atom's stencil meets it
     int g = (int)c + d.off[a] - t0[a];  // first point, from the tile's
     g = g < 0 ? g + nn[a] : g;
