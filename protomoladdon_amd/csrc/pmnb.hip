@@ -344,28 +344,41 @@ ForceParams make_params_for(const pmnb_params &prm, double csf) {
 }
 
 // Column grid of the tile path for box b, pair cutoff rcp and n atoms: x/y
-// columns at least rcp / 2 wide, z cells of about rcp / 8.  A thin gas gets
-// wider columns and z cells (16 atoms per column, one per z cell on average),
-// so that a work item still holds several atoms.  An axis with fewer than
-// five columns is marked for the per-pair minimum image.  A column's z cells
-// are split into bins of at most 256 cells and about 256 atoms.  shell
-// receives the distinct cell offsets within reach ((0,0,0) first), which the
-// pair-set extraction walks.
-void make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
+// columns at least rcp / 2 wide, z cells of about rcp / 8.  A box whose columns
+// would hold fewer than 16 atoms on average gets columns of up to rcp and z
+// cells of up to rcp / 3, so that a work item still holds several atoms; never
+// wider, whatever the mean density: the atoms may be a dense part of a large
+// box (a droplet of 32,000 atoms in an 830 A box: 8,180 us with columns of
+// 16 atoms on average, 19 A wide, 372 with these), and coordinates are
+// FP32 offsets from the corner of a cell (columns of 300 A leave them an error
+// beyond `band`, and so another pair set).  False: more than 2^26 columns of
+// rcp by cells of rcp, which the reference's grid takes.
+// An axis with fewer than five columns is marked for the per-pair minimum
+// image.  A column's z cells are split into bins of at most 256 cells and about
+// 256 atoms.  shell receives the distinct cell offsets within reach ((0,0,0)
+// first), which the pair-set extraction walks.
+bool make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
                    std::vector<int4> &shell) {
-  auto cells = [](double len, double w) {
-    return (int)std::max(1.0, std::min(std::floor(len / w), 1e5));
+  auto cells = [&](int axis, double w) {
+    return std::max(1.0, std::floor(b.H[axis] / w));
   };
-  int tx = cells(b.H[0], 0.5 * rcp), ty = cells(b.H[1], 0.5 * rcp);
-  const double most = std::max(1.0, n / 16.0);
-  while ((double)tx * ty > most && (tx > 5 || ty > 5)) {
-    int &k = tx >= ty ? tx : ty;
-    k = std::max(5, std::min(k - 1, (int)(k * 0.9)));
+  if (!(cells(0, rcp) * cells(1, rcp) * cells(2, rcp) < 67108864.0))
+    return false;
+  int tx = (int)cells(0, 0.5 * rcp), ty = (int)cells(1, 0.5 * rcp);
+  // the fewest columns of an axis: rcp wide, five where there are five
+  const int mx = std::max((int)cells(0, rcp), std::min(tx, 5)),
+            my = std::max((int)cells(1, rcp), std::min(ty, 5));
+  const double most = n / 16.0;
+  while ((double)tx * ty > most && (tx > mx || ty > my)) {
+    const bool x = ty <= my || (tx > mx && tx >= ty);
+    int &k = x ? tx : ty;
+    k = std::max(x ? mx : my, std::min(k - 1, (int)(k * 0.9)));
   }
   const int ncol = tx * ty;
   const int col_atoms = (n + ncol - 1) / ncol;
-  const int tz = std::min(cells(b.H[2], 0.125 * rcp),
-                          std::max(col_atoms, std::min(cells(b.H[2], rcp), 64)));
+  int tz = (int)std::min(cells(2, 0.125 * rcp),
+                         std::max((double)col_atoms, cells(2, rcp / 3.0)));
+  if ((double)ncol * tz >= 67108864.0) tz = (int)cells(2, rcp);
   rep = TileRep{};
   const double csz = b.H[2] / tz;
   const int rz = (int)std::floor(rcp / csz) + 1;
@@ -421,6 +434,7 @@ void make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
     for (int dy : oy)
       for (int dz : oz)
         if (dx || dy || dz) shell.push_back(make_int4(dx, dy, dz, 0));
+  return true;
 }
 
 // Box + grid + shell offsets exactly as PeriodicBoundaryConditions::set,
@@ -551,12 +565,12 @@ int build_box(pmnb_ctx *ctx, const double *e1, const double *e2,
     const ForceParams P0 = make_params_for(ctx->prm, ctx->csf);
     const double rcp = std::sqrt(P0.cut2);
     const bool packs = ctx->ntypes <= 256 && ctx->n < (1 << kQTypeShift);
-    ctx->use_tile = ctx->prm.algorithm_cutoff >= rcp && packs;
+    std::vector<int4> tshell;
+    TileRep rep{};
+    ctx->use_tile = ctx->prm.algorithm_cutoff >= rcp && packs &&
+                    make_tile_rep(b, rcp, ctx->n, rep, tshell);
     ctx->tile_types = ctx->ntypes * ctx->ntypes <= kQLj;
     if (ctx->use_tile) {
-      std::vector<int4> tshell;
-      TileRep rep{};
-      make_tile_rep(b, rcp, ctx->n, rep, tshell);
       g = rep.grid;
       ctx->shell = tshell;  // pair-set extraction walks it
       ctx->reps.assign(1, rep);
@@ -1883,7 +1897,8 @@ int batch_finalize(pmnb_batch *b) {
     TileRep rep{};
     int na = 0;
     while (a + na < (int)b->rep_of.size() && b->rep_of[a + na] == r) na++;
-    make_tile_rep(b->boxes[r], rcp, na, rep, shell);
+    if (!make_tile_rep(b->boxes[r], rcp, na, rep, shell))
+      return fail(ctx, PMNB_ERR_UNSUPPORTED, "replica %d grid too large", r);
     rep.cell_off = (int)cells;
     rep.bin_off = (int)bins;
     rep.atom_off = a;
