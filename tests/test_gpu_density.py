@@ -3,10 +3,13 @@ with the bars of test_gpu_parity (pair sets bit for bit, FP64 forces within
 1e-11 of the largest component, mixed forces within 1e-5 RMS): the cell grid
 is laid out from the box and the number of atoms alone, the atoms may be
 anywhere in it."""
+import time
+
 import numpy as np
 import pytest
 
 from protomoladdon_amd import systems
+from protomoladdon_amd.topology import PeriodicBoundaryConditions
 from tests.test_gpu_parity import check_fp64, check_mixed
 
 pytestmark = pytest.mark.gpu
@@ -38,3 +41,46 @@ def test_dimers_in_a_wide_box():
     offsets in a cell lose the pairs near the cutoff."""
     check_fp64(dimers(300, 2400.0))
     check_mixed(dimers(300, 2400.0))
+
+
+def dense_in_wide_box(n_mol, L, squeeze):
+    """A cube of water, squeezed by `squeeze` per axis, in a corner of a box
+    of L."""
+    w = systems.small_water(n_mol=n_mol)
+    w.positions = w.positions * squeeze
+    w.topology.boundary_conditions = PeriodicBoundaryConditions(
+        (L, 0, 0), (0, L, 0), (0, 0, L), (0.5 * L,) * 3)
+    return w
+
+
+@pytest.mark.parametrize("n_mol,L,squeeze", [
+    (700, 60.0, 0.62),    # no bin beyond what a block sorts in LDS
+    (2500, 150.0, 0.5),   # bins of over 1,024 atoms
+    (1500, 150.0, 0.12),  # z cells of over 256 atoms
+])
+def test_dense_part_of_a_box(n_mol, L, squeeze):
+    check_fp64(dense_in_wide_box(n_mol, L, squeeze))
+
+
+@pytest.mark.parametrize("precision", ["mixed", "fp64"])
+def test_no_finite_position_takes_no_time(precision):
+    """All atoms in one z cell of one bin: sorted in linear time (a sort by
+    comparison of all pairs of 30,000 atoms takes seconds)."""
+    import torch
+    w = systems.small_water(n_mol=10000)
+    f = w.make_force(precision)
+    x = torch.full((w.n_atoms, 3), float("nan"), dtype=torch.float64,
+                   device="cuda")
+    frc = torch.zeros_like(x)
+    out = torch.zeros(20, dtype=torch.float64, device="cuda")
+    f.evaluate_device(w.topology, x, frc, out, 0)
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    f.evaluate_device(w.topology, x, frc, out, 0)
+    torch.cuda.synchronize()
+    ms = 1e3 * (time.perf_counter() - t0)
+    n = f.last_pair_count()
+    f.close()
+    print("%d atoms %.2f ms" % (w.n_atoms, ms), flush=True)
+    assert n == 0 and not frc.abs().max().item()
+    assert ms < 100.0
