@@ -651,15 +651,15 @@ void launch_fill_i32(int *p, int n, int v, hipStream_t s) {
                        n, v);
 }
 
-// Atom slots per bin of the tile path's buckets: twice the mean occupancy of
-// the fullest replica's bins and 64 more, a power of two up to kBinSort (a
-// fuller bin is read back from the bin index of every atom instead).
-int tile_bucket_cap(const std::vector<TileRep> &reps) {
-  long long mean = 0;
-  for (const TileRep &r : reps)
-    mean = std::max<long long>(mean, (r.natom + r.nbin - 1) / r.nbin);
-  int cap = 64;
-  while (cap < 2 * mean + 64 && cap < kBinSort) cap *= 2;
+// Atom slots per bin of the tile path's buckets: what a block sorts in LDS,
+// whatever the mean, since the atoms may fill only a part of the box; fewer
+// where the rows of all bins would pass 256 MB (the block of a bin with more
+// atoms than its row holds reads the bin index of every atom of the replica).
+// 277,000 atoms filling a third of their box along x, 660 a column: 673 us with
+// rows of twice the mean, 386 with these.
+int tile_bucket_cap(long long nbin) {
+  int cap = kBinSort;
+  while (cap > 64 && nbin * cap > (1ll << 26)) cap /= 2;
   return cap;
 }
 
@@ -687,7 +687,7 @@ int ensure_eval_buffers(pmnb_ctx *ctx) {
   if (ctx->use_tile) {
     HIPCHK(ctx->d_srec.ensure(N * sizeof(unsigned)));
     HIPCHK(ctx->d_ccount.ensure((size_t)nc * sizeof(int)));
-    ctx->bucket_cap = tile_bucket_cap(ctx->reps);
+    ctx->bucket_cap = tile_bucket_cap(ctx->nbin);
     HIPCHK(ctx->d_bucket.ensure((size_t)ctx->nbin * ctx->bucket_cap *
                                 sizeof(int)));
   }
@@ -3763,8 +3763,10 @@ struct Carve {
   }
 };
 
-// The tile path's arrays for one system of ctx, carved from `base`.
-EvalBufs carve_bufs(const pmnb_ctx *ctx, unsigned char *base, size_t &bytes) {
+// The tile path's arrays for one system of ctx, carved from `base`, with
+// bucket rows of cap atoms.
+EvalBufs carve_bufs(const pmnb_ctx *ctx, unsigned char *base, int cap,
+                    size_t &bytes) {
   Carve c{base};
   const size_t N = (size_t)std::max(ctx->n, 1);
   const size_t nc = (size_t)std::max(ctx->grid.ncell, 1);
@@ -3776,7 +3778,7 @@ EvalBufs carve_bufs(const pmnb_ctx *ctx, unsigned char *base, size_t &bytes) {
   B.ccount = c.take<int>(nc);
   B.rank = nullptr;  // the tile path fills bucket rows instead
   B.sorted = c.take<int>(N);
-  B.cap = tile_bucket_cap(ctx->reps);
+  B.cap = cap;
   B.bucket = c.take<int>((size_t)ctx->nbin * B.cap);
   B.sx = c.take<double>(N);
   B.sy = c.take<double>(N);
@@ -3857,13 +3859,17 @@ int pmnb_evaluate_device_noalloc(pmnb_ctx *ctx, const double *d_positions,
     return fail(ctx, PMNB_ERR_HIP, "no scratch address on device %d: %s", dev,
                 hipGetErrorString(serr));
   size_t need = 0;
-  carve_bufs(ctx, nullptr, need);
+  // the longest bucket rows that fit (a shorter row gives the same results)
+  int cap = tile_bucket_cap(ctx->nbin);
+  carve_bufs(ctx, nullptr, cap, need);
+  while (need > kScratchBytes && cap > 64)
+    carve_bufs(ctx, nullptr, cap /= 2, need);
   need = std::max(need, scratch_limit_bytes(ctx));
   if (need > kScratchBytes)
     return fail(ctx, PMNB_ERR_CAPACITY,
                 "the evaluation needs %zu bytes of scratch; the static scratch "
                 "holds %zu (64 MiB)", need, kScratchBytes);
-  const EvalBufs B = carve_bufs(ctx, base, need);
+  const EvalBufs B = carve_bufs(ctx, base, cap, need);
   HIPCHK(hipSetDevice(dev));
   hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
   if (ctx->n == 0) return PMNB_OK;

@@ -57,9 +57,11 @@ def dense_in_wide_box(n_mol, L, squeeze):
     (700, 60.0, 0.62),    # no bin beyond what a block sorts in LDS
     (2500, 150.0, 0.5),   # bins of over 1,024 atoms
     (1500, 150.0, 0.12),  # z cells of over 256 atoms
+    (2000, 2400.0, 1.0),  # bucket rows shorter than the bins' atoms
 ])
 def test_dense_part_of_a_box(n_mol, L, squeeze):
-    check_fp64(dense_in_wide_box(n_mol, L, squeeze))
+    w = dense_in_wide_box(n_mol, L, squeeze)
+    check_fp64(systems.with_algorithm(w, 9.0, max(4.5, L / 48)))
 
 
 @pytest.mark.parametrize("precision", ["mixed", "fp64"])
