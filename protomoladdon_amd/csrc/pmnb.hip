@@ -229,6 +229,8 @@ struct pmnb_ctx {
   int rep_uploaded = 0;           // reps and bin_rep are on the device
   DevBuf d_partial_lj;            // adjoint: LJ-parameter gradients per atom
   DevBuf d_bucket, d_ccount;
+  DevBuf d_group;                 // sums of groups of bins
+  int ngroup = 0;
   // d_count holds zeros at the start of the next evaluation on the tile path
   // (the finish kernel clears it after the pair kernel): no clearing launch
   bool counts_zero = false;
@@ -414,6 +416,7 @@ bool make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
   rep.fz = std::max(1, (tz + want - 1) / want);
   rep.ns = (tz + rep.fz - 1) / rep.fz;
   rep.nbin = ncol * rep.ns;
+  rep.grp_off = rep.nbin > kGroupBins ? 0 : -1;
   rep.natom = n;
   rep.item_max = n / kTileAtoms + std::min(n, rep.nbin);
   // distinct offsets per axis
@@ -435,6 +438,10 @@ bool make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
       for (int dz : oz)
         if (dx || dy || dz) shell.push_back(make_int4(dx, dy, dz, 0));
   return true;
+}
+
+int bin_groups(const TileRep &rep) {
+  return rep.grp_off < 0 ? 0 : blocks_for(rep.nbin, kBinGroup);
 }
 
 // Box + grid + shell offsets exactly as PeriodicBoundaryConditions::set,
@@ -576,6 +583,7 @@ int build_box(pmnb_ctx *ctx, const double *e1, const double *e2,
       ctx->reps.assign(1, rep);
       ctx->bin_rep.clear();
       ctx->nbin = rep.nbin;
+      ctx->ngroup = bin_groups(rep);
       ctx->nslots = rep.item_max;
     }
   }
@@ -687,6 +695,7 @@ int ensure_eval_buffers(pmnb_ctx *ctx) {
   if (ctx->use_tile) {
     HIPCHK(ctx->d_srec.ensure(N * sizeof(unsigned)));
     HIPCHK(ctx->d_ccount.ensure((size_t)nc * sizeof(int)));
+    HIPCHK(ctx->d_group.ensure((size_t)std::max(ctx->ngroup, 1) * sizeof(int2)));
     ctx->bucket_cap = tile_bucket_cap(ctx->nbin);
     HIPCHK(ctx->d_bucket.ensure((size_t)ctx->nbin * ctx->bucket_cap *
                                 sizeof(int)));
@@ -868,6 +877,7 @@ struct EvalBufs {
   unsigned long long *npairs;  // [0] pairs, [1] visits of the tile path
   int4 *items;
   int *rep_items;
+  int2 *group;            // sums of groups of bins
   const TileRep *reps;
 };
 
@@ -894,6 +904,7 @@ EvalBufs ctx_bufs(const pmnb_ctx *ctx) {
   B.npairs = ctx->d_npairs.as<unsigned long long>();
   B.items = ctx->d_items.as<int4>();
   B.rep_items = ctx->d_rep_items.as<int>();
+  B.group = ctx->d_group.as<int2>();
   B.reps = ctx->d_reps.as<TileRep>();
   return B;
 }
@@ -930,7 +941,12 @@ int build_cells(pmnb_ctx *ctx, const EvalBufs &B, const double *d_pos,
     }
     BinOut O{B.sorted, B.sx,   B.sy,    B.sz,     B.sq,    B.loc,
              B.stype,  B.smol, B.scell, B.srec,   B.start, B.ccount,
-             B.items,  B.rep_items,     B.npairs + 1};
+             B.items,  B.rep_items,     B.npairs + 1,      B.group};
+    for (size_t r = 0; r < ctx->reps.size(); r++)
+      if (ctx->reps[r].grp_off >= 0)
+        hipLaunchKernelGGL(k_bin_groups, dim3(bin_groups(ctx->reps[r])),
+                           dim3(kBinGroup), 0, s, B.reps, (int)r, B.count,
+                           B.group, B.items);
     const int *bin_rep = ctx->batch ? ctx->d_bin_rep.as<int>() : nullptr;
     hipLaunchKernelGGL(k_sort_bins, dim3(ctx->nbin), dim3(kBlock), 0, s, B.reps,
                        bin_rep, d_pos, B.count, B.bucket, B.cap, B.cell_of,
@@ -1685,7 +1701,8 @@ void pmnb_destroy(pmnb_ctx *ctx) {
                     &ctx->d_partial2, &ctx->d_shell_off, &ctx->d_items,
                     &ctx->d_reps, &ctx->d_bin_rep, &ctx->d_rep_items,
                     &ctx->d_rep_of, &ctx->d_partial_lj, &ctx->d_plog,
-                    &ctx->d_plog_count, &ctx->d_bucket, &ctx->d_ccount};
+                    &ctx->d_plog_count, &ctx->d_bucket, &ctx->d_ccount,
+                    &ctx->d_group};
   for (DevBuf *b : bufs) b->release();
   for (hipEvent_t e : ctx->ev_pool) (void)hipEventDestroy(e);
   for (hipEvent_t e : ctx->h_ev)
@@ -1892,6 +1909,7 @@ int batch_finalize(pmnb_batch *b) {
   ctx->reps.clear();
   ctx->bin_rep.clear();
   long long cells = 0, bins = 0, slots = 0;
+  int groups = 0;
   std::vector<int4> shell;
   for (int r = 0, a = 0; r < R; r++) {
     TileRep rep{};
@@ -1901,6 +1919,8 @@ int batch_finalize(pmnb_batch *b) {
       return fail(ctx, PMNB_ERR_UNSUPPORTED, "replica %d grid too large", r);
     rep.cell_off = (int)cells;
     rep.bin_off = (int)bins;
+    if (rep.grp_off >= 0) rep.grp_off = groups;
+    groups += bin_groups(rep);
     rep.atom_off = a;
     rep.item_off = (int)slots;
     a += na;
@@ -1913,6 +1933,7 @@ int batch_finalize(pmnb_batch *b) {
     ctx->reps.push_back(rep);
   }
   ctx->nbin = (int)bins;
+  ctx->ngroup = groups;
   ctx->nslots = (int)slots;
   ctx->use_tile = true;
   ctx->tile_types = true;
@@ -3793,6 +3814,7 @@ EvalBufs carve_bufs(const pmnb_ctx *ctx, unsigned char *base, int cap,
   B.npairs = c.take<unsigned long long>(2);
   B.items = c.take<int4>(slots);
   B.rep_items = c.take<int>(1);
+  B.group = c.take<int2>((size_t)std::max(ctx->ngroup, 1));
   B.reps = c.take<TileRep>(1);
   bytes = c.off;
   return B;

@@ -6,8 +6,9 @@
 // Bins, not z cells, are counted: 400 instead of 3,200 on the 96,000-atom
 // water, so that every block finds its first slot and first item by adding
 // the counts of its replica's earlier bins itself, with no scan launch
-// between the two kernels.  A replica's atoms and item slots start at offsets
-// fixed on the host.
+// between the two kernels (a replica of thousands of bins gets sums of groups
+// of bins in a launch of its own).  A replica's atoms and item slots start at
+// offsets fixed on the host.
 #pragma once
 
 #include "pmnb_queue.h"
@@ -16,6 +17,12 @@ namespace pmnb {
 
 constexpr int kBinSort = 1024;  // atoms a block sorts in LDS
 constexpr int kBinCells = 256;  // most z cells of a bin
+constexpr int kBinGroup = kBlock;  // bins of a sum of k_bin_groups
+// Replicas of more bins than this get their counts added by groups first (a
+// launch of 4 us).  An evaluation without / with the groups: 4,608 bins 1,263 /
+// 1,261 us (1,029,000 atoms), 17,000 bins 369 / 331 (32,000 atoms), 35,000 bins
+// 251 / 83 (900 atoms), 98,000 bins 2,513 / 1,019 (999,000 atoms).
+constexpr int kGroupBins = 4096;
 
 // Bin of every atom.  Bins of a block's atoms are few (consecutive atoms are
 // neighbours): the block counts its atoms per bin in an LDS table (open
@@ -70,6 +77,40 @@ k_assign_bins(const TileRep *__restrict__ reps, const int *__restrict__ rep_of,
   }
 }
 
+// Atoms and items of each group of kBinGroup bins of replica r, so that a
+// block of k_sort_bins adds groups instead of all earlier bins; the item slots
+// are emptied here for those replicas.  One block per group.
+__global__ void __launch_bounds__(kBinGroup)
+k_bin_groups(const TileRep *__restrict__ reps, int r,
+             const int *__restrict__ count, int2 *__restrict__ group,
+             int4 *__restrict__ items) {
+  __shared__ int red[2][kBinGroup / 64];
+  const TileRep &R = reps[r];
+  const int t = threadIdx.x, k = blockIdx.x * kBinGroup + t;
+  const int c = k < R.nbin ? count[R.bin_off + k] : 0;
+  int sa = c, si = (c + kTileAtoms - 1) / kTileAtoms;
+  for (int o = 32; o > 0; o >>= 1) {
+    sa += __shfl_down(sa, o, 64);
+    si += __shfl_down(si, o, 64);
+  }
+  if ((t & 63) == 0) {
+    red[0][t >> 6] = sa;
+    red[1][t >> 6] = si;
+  }
+  for (int j = k; j < R.item_max; j += gridDim.x * kBinGroup)
+    items[R.item_off + j] = make_int4(0, 0, 0, 0);
+  __syncthreads();
+  if (t == 0) {
+    sa = si = 0;
+#pragma unroll
+    for (int w = 0; w < kBinGroup / 64; w++) {
+      sa += red[0][w];
+      si += red[1][w];
+    }
+    group[R.grp_off + blockIdx.x] = make_int2(sa, si);
+  }
+}
+
 // A double as an integer of the same order (a total order, NaN included).
 __device__ __forceinline__ long long order_key(double v) {
   const long long b = __double_as_longlong(v);
@@ -88,6 +129,7 @@ struct BinOut {
   int4 *items;              // {first slot, end slot, local column, replica}
   int *rep_items;           // items of each replica
   unsigned long long *npairs;  // pair counter, cleared here
+  const int2 *group;        // sums of k_bin_groups
 };
 
 // One block per bin.  The atoms (from the bin's bucket row or, beyond its
@@ -124,7 +166,14 @@ k_sort_bins(const TileRep *__restrict__ reps, const int *__restrict__ bin_rep,
   if (t == 0) found = 0;
   // first slot and first item: the replica's earlier bins
   int sa = 0, si = 0;
-  for (int k = t; k < lb; k += kBlock) {
+  const bool grouped = R.grp_off >= 0;
+  const int g0 = grouped ? lb / kBinGroup : 0;
+  for (int k = t; k < g0; k += kBlock) {
+    const int2 g = O.group[R.grp_off + k];
+    sa += g.x;
+    si += g.y;
+  }
+  for (int k = g0 * kBinGroup + t; k < lb; k += kBlock) {
     const int c = count[R.bin_off + k];
     sa += c;
     si += (c + kTileAtoms - 1) / kTileAtoms;
@@ -152,7 +201,7 @@ k_sort_bins(const TileRep *__restrict__ reps, const int *__restrict__ bin_rep,
   if (lb == R.nbin - 1) {
     // the replica's unused item slots are empty
     if (t == 0) O.rep_items[r] = si + ni;
-    for (int k = si + ni + t; k < R.item_max; k += kBlock)
+    for (int k = si + ni + t; k < R.item_max && !grouped; k += kBlock)
       O.items[R.item_off + k] = make_int4(0, 0, 0, 0);
   }
   // z cell (in the bin) and order key of atom a

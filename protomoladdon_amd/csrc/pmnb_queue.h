@@ -35,6 +35,7 @@ struct TileRep {
   int cell_off;       // first global cell of the replica
   int bin_off, nbin;  // its bins: (column) * ns + z cell / fz
   int ns, fz;         // bins per column, z cells per bin
+  int grp_off;        // its sums of kBinGroup bins start here (-1: none)
   int atom_off, natom;  // first sorted slot (= first atom), atoms
   int item_off, item_max;  // its item slots
 };

@@ -8,9 +8,12 @@ import time
 import numpy as np
 import pytest
 
+from oracle import oracle as O
 from protomoladdon_amd import systems
+from protomoladdon_amd.batch import BatchedCutoffForce
 from protomoladdon_amd.topology import PeriodicBoundaryConditions
-from tests.test_gpu_parity import check_fp64, check_mixed
+from tests.test_gpu_batch import batch_eval, single_eval
+from tests.test_gpu_parity import check_fp64, check_mixed, rms_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -62,6 +65,32 @@ def dense_in_wide_box(n_mol, L, squeeze):
 def test_dense_part_of_a_box(n_mol, L, squeeze):
     w = dense_in_wide_box(n_mol, L, squeeze)
     check_fp64(systems.with_algorithm(w, 9.0, max(4.5, L / 48)))
+
+
+@pytest.mark.parametrize("precision", ["mixed", "fp64"])
+def test_replicas_of_many_bins(precision):
+    """Replicas whose bins are counted by groups between others, each as it
+    gives alone."""
+    ws = [systems.config3_replica(i, n) for i, n in enumerate((40, 300, 700, 90))]
+    for w, L in ((ws[1], 640.0), (ws[2], 620.0)):
+        w.topology.boundary_conditions = PeriodicBoundaryConditions(
+            (L, 0, 0), (0, L, 0), (0, 0, 1.5 * L), (0.5 * L,) * 3)
+    bf = BatchedCutoffForce.from_workloads(ws, precision=precision)
+    frc, out = batch_eval(bf, ws)[1:]
+    n = bf.pair_count()
+    total = 0
+    for r, w in enumerate(ws):
+        f1, o1, n1 = single_eval(w, precision)
+        ref = O.evaluate(O.System.from_workload(w, flags=1))
+        total += n1
+        assert n1 == ref.n_pairs
+        a, b = bf.offsets[r], bf.offsets[r + 1]
+        np.testing.assert_array_equal(frc[a:b], f1)
+        np.testing.assert_array_equal(out[r], o1)
+        assert rms_rel(f1, ref.forces) <= (1e-5 if precision == "mixed" else
+                                           1e-12)
+    bf.close()
+    assert n == total
 
 
 @pytest.mark.parametrize("precision", ["mixed", "fp64"])
