@@ -3348,7 +3348,7 @@ struct pmnb_pme {
   int nx = 0, ny = 0, nz = 0;
   double alpha = 0, kc = 0, V = 0;
   double csf = 1.0, e_self = 0, e_charged = 0;
-  DevBuf q, count, bucket, over, qreal, qk, mod, ex, part, cpart, xptr, xent,
+  DevBuf q, count, bucket, qfix, qreal, qk, mod, ex, part, cpart, xptr, xent,
       xrows;
   int nb[3] = {0, 0, 0}, cap = 0;
   int n_part = 0, n_cpart = 0;
@@ -3427,7 +3427,7 @@ PmeDev pme_dev(pmnb_pme *pm) {
   d.q = pm->q.as<double>();
   d.count = pm->count.as<int>();
   d.bucket = pm->bucket.as<double4>();
-  d.over = pm->over.as<double4>();
+  d.qfix = pm->qfix.as<unsigned long long>();
   d.cap = pm->cap;
   d.qreal = pm->qreal.as<double>();
   d.qk = pm->qk.as<double2>();
@@ -3467,7 +3467,7 @@ EwDev pme_corr_dev(pmnb_pme *pm) {
 template <int P>
 void pme_spread(pmnb_pme *pm, const PmeDev &d, const double *x,
                 hipStream_t s) {
-  hipLaunchKernelGGL(k_pme_bin, dim3(blocks_for(pm->n, kPmeBlock)),
+  hipLaunchKernelGGL(k_pme_bin<P>, dim3(blocks_for(pm->n, kPmeBlock)),
                      dim3(kPmeBlock), 0, s, d, x);
   const int tiles = blocks_for(pm->nx, kPmeTile) * blocks_for(pm->ny, kPmeTile) *
                     blocks_for(pm->nz, kPmeTile);
@@ -3585,9 +3585,9 @@ int pmnb_pme_create(pmnb_ctx *ctx, int32_t nx, int32_t ny, int32_t nz,
   pm->n_cpart = blocks_for(std::max(n_atoms, 1), kPmeBlock / kPmeLanes);
   long long bins = 1;
   for (int a = 0; a < 3; a++) bins *= pm->nb[a] = blocks_for(nn[a], kPmeBin);
-  // four times the mean occupancy and 8 more, at most 256 (the atoms beyond a
-  // full bucket go to the overflow list)
-  pm->cap = (int)std::min<long long>(256, 4 * (n_atoms / bins) + 8);
+  // four times the mean occupancy and 8 more, between 32 and 256
+  pm->cap = (int)std::max<long long>(
+      32, std::min<long long>(256, 4 * (n_atoms / bins) + 8));
   auto up = [&](DevBuf &d, const void *src, size_t bytes) -> hipError_t {
     hipError_t e = d.ensure(std::max<size_t>(bytes, 16));
     if (e == hipSuccess && bytes && src)
@@ -3600,8 +3600,8 @@ int pmnb_pme_create(pmnb_ctx *ctx, int32_t nx, int32_t ny, int32_t nz,
   if (e == hipSuccess) e = hipMemset(pm->count.p, 0, (size_t)(bins + 1) * sizeof(int));
   if (e == hipSuccess)
     e = pm->bucket.ensure((size_t)bins * pm->cap * sizeof(double4));
-  if (e == hipSuccess)
-    e = pm->over.ensure((size_t)std::max(n_atoms, 1) * sizeof(double4));
+  if (e == hipSuccess) e = pm->qfix.ensure((size_t)total * sizeof(long long));
+  if (e == hipSuccess) e = hipMemset(pm->qfix.p, 0, (size_t)total * sizeof(long long));
   if (e == hipSuccess) e = pm->qreal.ensure((size_t)total * sizeof(double));
   if (e == hipSuccess) e = pm->qk.ensure((size_t)half * sizeof(double2));
   if (e == hipSuccess) e = up(pm->mod, mod.data(), mod.size() * sizeof(double));
@@ -3667,11 +3667,16 @@ int pmnb_pme_evaluate_device(pmnb_pme *pm, const double *d_positions,
     case 6: pme_spread<6>(pm, d, d_positions, s); break;
     default: pme_spread<8>(pm, d, d_positions, s); break;
   }
-  // An evaluation that stops before k_pme_scalar clears the bins itself: the
-  // next one counts from zero.
+  // An evaluation that stops before k_pme_scalar clears the bins itself (and
+  // the integer grid, which k_pme_spread may not have read): the next one
+  // counts from zero.
   auto clear_bins = [&]() {
     const int nbin = pm->nb[0] * pm->nb[1] * pm->nb[2];
     launch_fill_i32(d.count, nbin + 1, 0, s);
+    const long long total = (long long)pm->nx * pm->ny * pm->nz;
+    hipLaunchKernelGGL(k_zero_u64,
+                       dim3((unsigned)((total + kPmeBlock - 1) / kPmeBlock)),
+                       dim3(kPmeBlock), 0, s, d.qfix, total);
   };
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) {
@@ -3714,7 +3719,7 @@ void pmnb_pme_destroy(pmnb_pme *pm) {
   (void)hipDeviceSynchronize();
   if (pm->have_fwd) (void)hipfftDestroy(pm->fwd);
   if (pm->have_inv) (void)hipfftDestroy(pm->inv);
-  DevBuf *bufs[] = {&pm->q, &pm->count, &pm->bucket, &pm->over, &pm->qreal,
+  DevBuf *bufs[] = {&pm->q, &pm->count, &pm->bucket, &pm->qfix, &pm->qreal,
                     &pm->qk, &pm->mod, &pm->ex, &pm->part, &pm->cpart,
                     &pm->xptr, &pm->xent, &pm->xrows};
   for (DevBuf *b : bufs) b->release();

@@ -20,8 +20,8 @@ __global__ void k_fill_i32(int *p, int n, int v) {
   if (i < n) p[i] = v;
 }
 
-__global__ void k_fill_u64(unsigned long long *p, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_zero_u64(unsigned long long *p, long long n) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0ull;
 }
 

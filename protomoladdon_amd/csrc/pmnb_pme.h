@@ -9,11 +9,14 @@
 //   k_pme_bin        one thread per atom: grid coordinates x = r n / L
 //                    wrapped into [0, n) as Grid::anterpolateCharge does
 //                    (Grid.h:107-131), written with the charge into the
-//                    bucket of the atom's bin (4^3 grid cells);
+//                    bucket of the atom's bin (4^3 grid cells); an atom
+//                    beyond the bucket is spread at once, by atomic adds
+//                    into an integer grid that is zero otherwise;
 //   k_pme_spread     one block per tile of 8^3 grid points: the atoms of the
 //                    bins that reach it, the B-spline weights of
 //                    BSpline::set (BSpline.cpp:58-95), and q Mx My Mz summed
-//                    over them in LDS as 64-bit fixed-point integers (2^-40):
+//                    over them in LDS as 64-bit fixed-point integers (2^-40),
+//                    on top of what k_pme_bin spread:
 //                    integer sums do not depend on the order of the adds, so
 //                    the grid is the same bits on every run;
 //   hipFFT D2Z       the unnormalised transform of the real grid (nx, ny,
@@ -66,11 +69,12 @@ struct PmeDev {
   double fac;              // pi^2 / alpha^2
   const double *q;         // scaled charges
   int nb[3];               // atom bins per axis
-  int *count;              // atoms per bin, then of the overflow list (zero
-                           // between runs)
+  int *count;              // atoms per bin, then all beyond their buckets
+                           // (zero between runs)
   double4 *bucket;         // cap records {grid x, y, z, charge} per bin
-  double4 *over;           // records beyond a bin's bucket
   int cap;
+  unsigned long long *qfix;  // nx ny nz: charges of the atoms beyond their
+                           // buckets, 2^-40 (zero between runs)
   double *qreal;           // nx ny nz real grid
   double2 *qk;             // nx ny nzh half spectrum
   const double *mod[3];    // B(m) per axis index (Grid::dftmod)
@@ -140,9 +144,52 @@ __device__ __forceinline__ int pme_wrap(int g, int n) {
   return g >= n ? g - n : g;
 }
 
-// Atoms beyond a bin's bucket go to the overflow list, which every tile reads
-// whole.  The order in a bucket varies from run to run; the integer sums of
-// the tiles do not.
+// A contribution in units of 2^-40.  small: |value| <= |charge| < 2048, where
+// adding 1.5 * 2^12 leaves the value rounded to 2^-40 in the low bits, the
+// rounding of rint.
+__device__ __forceinline__ unsigned long long pme_fixed(double val, bool small) {
+  if (small)
+    return (unsigned long long)__double_as_longlong(val + 6144.0) -
+           0x40B8000000000000ull;
+  val = fmin(fmax(val, -kPmeFixClamp), kPmeFixClamp);
+  return (unsigned long long)(long long)__builtin_rint(val * kPmeFixScale);
+}
+
+// Spreads one atom into the integer grid in memory.
+template <int P>
+__device__ __forceinline__ void pme_spread_global(const PmeDev &d,
+                                                  const double4 &r) {
+  const int ix = (int)r.x, iy = (int)r.y, iz = (int)r.z;
+  double tx[P], ty[P], tz[P], dth[P];
+  pme_bspline<P>(r.x - ix, tx, dth);
+  pme_bspline<P>(r.y - iy, ty, dth);
+  pme_bspline<P>(r.z - iz, tz, dth);
+  const bool small = fabs(r.w) < 2048.0;
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    const size_t plane = (size_t)pme_wrap(ix + d.off[0] + u, d.nx) * d.ny;
+    const double av = r.w * tx[u];
+#pragma unroll
+    for (int v = 0; v < P; v++) {
+      unsigned long long *row =
+          d.qfix + (plane + pme_wrap(iy + d.off[1] + v, d.ny)) * d.nz;
+      const double ab = av * ty[v];
+#pragma unroll
+      for (int w = 0; w < P; w++)
+        atomicAdd(row + pme_wrap(iz + d.off[2] + w, d.nz),
+                  pme_fixed(ab * tz[w], small));
+    }
+  }
+}
+
+// The order in a bucket varies from run to run, and so does which atoms are
+// beyond it; the integer sums do not.  A bucket holds four times the mean and
+// at least 32 atoms (three times what a bin of water holds on a grid of 1.2 A),
+// so that atoms are beyond it only on coarse grids, where they are much denser
+// than on average.  32,000 atoms in a 68 A cube, 256^3 grid, with a list of
+// those atoms that every tile reads / with their charges added in memory: box
+// of 300 A 783 / 582 us (none beyond its bucket), of 830 A 1,472 / 693.
+template <int P>
 __global__ __launch_bounds__(kPmeBlock) void k_pme_bin(PmeDev d,
                                                        const double *x) {
   const int i = blockIdx.x * kPmeBlock + threadIdx.x;
@@ -156,10 +203,8 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_bin(PmeDev d,
   if (k < d.cap) {
     d.bucket[(size_t)b * d.cap + k] = r;
   } else {
-    // (bounded whatever the counts held on entry: two evaluations of one
-    // object that overlap give wrong sums, not a write past the list)
-    const int o = atomicAdd(d.count + (size_t)d.nb[0] * d.nb[1] * d.nb[2], 1);
-    if (o < d.n) d.over[o] = r;
+    pme_spread_global<P>(d, r);
+    atomicAdd(d.count + (size_t)d.nb[0] * d.nb[1] * d.nb[2], 1);
   }
 }
 
@@ -182,8 +227,6 @@ __device__ __forceinline__ void pme_spread_plane(const PmeDev &d,
 #pragma unroll
   for (int k = 1; k < P; k++) mx = u == k ? tx[k] : mx;
   const double av = r.w * mx;
-  // |value| <= |charge| < 2048: adding 1.5 * 2^12 leaves the value rounded to
-  // 2^-40 in the low bits, the rounding of rint
   const bool small = fabs(r.w) < 2048.0;
 #pragma unroll
   for (int v = 0; v < P; v++) {
@@ -195,17 +238,8 @@ __device__ __forceinline__ void pme_spread_plane(const PmeDev &d,
     for (int w = 0; w < P; w++) {
       const int lz = pme_wrap(iz + d.off[2] + w, d.nz) - t0[2];
       if ((unsigned)lz >= (unsigned)te[2]) continue;
-      double val = ab * tz[w];
-      unsigned long long fix;
-      if (small) {
-        fix = (unsigned long long)__double_as_longlong(val + 6144.0) -
-              0x40B8000000000000ull;
-      } else {
-        val = fmin(fmax(val, -kPmeFixClamp), kPmeFixClamp);
-        fix = (unsigned long long)(long long)__builtin_rint(val * kPmeFixScale);
-      }
-      __hip_atomic_fetch_add(row + lz, fix, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_WORKGROUP);
+      __hip_atomic_fetch_add(row + lz, pme_fixed(ab * tz[w], small),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
   }
 }
@@ -215,9 +249,10 @@ __device__ __forceinline__ void pme_spread_plane(const PmeDev &d,
 // took 156 us for 96,000 atoms of order 4 on a 96^3 grid, plus 8 us to convert
 // and clear the integer grid; this kernel takes 30 us and k_pme_bin 10 (bound by
 // its atomics' latency), this one by its LDS atomics (a tile with margins, which
-// needs no test per point but adds 1.9 times as many, took 51).  Bins half a tile wide: 4 per axis reach a tile, 8 atoms
-// are read for one of the tile's own (27 with bins of a tile).  The listed atoms are spread over the
-// lanes by stencil plane, which evens out what the tile's edge cuts off.
+// needs no test per point but adds 1.9 times as many, took 51).  Bins half a
+// tile wide: 4 per axis reach a tile, 8 atoms are read for one of the tile's own
+// (27 with bins of a tile).  The listed atoms are spread over the lanes by
+// stencil plane, which evens out what the tile's edge cuts off.
 template <int P>
 __global__ __launch_bounds__(kPmeBlock) void k_pme_spread(PmeDev d) {
   __shared__ unsigned long long tile[kPmeTile * kPmePlane];
@@ -246,52 +281,60 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_spread(PmeDev d) {
       cnt[a] = last - first[a] + (last < first[a] ? d.nb[a] : 0) + 1;
     }
   }
-  for (int k = t; k < kPmeTile * kPmePlane; k += kPmeBlock) tile[k] = 0;
+  const bool pre = d.count[(size_t)d.nb[0] * d.nb[1] * d.nb[2]] > 0;
+  for (int k = t; k < kPmeTile * kPmeTile * kPmeTile; k += kPmeBlock) {
+    const int lx = k / (kPmeTile * kPmeTile), ly = k / kPmeTile % kPmeTile,
+              lz = k % kPmeTile;
+    unsigned long long v = 0;
+    if (pre && lx < te[0] && ly < te[1] && lz < te[2]) {
+      unsigned long long *p =
+          d.qfix + ((size_t)(t0[0] + lx) * d.ny + t0[1] + ly) * d.nz + t0[2] + lz;
+      v = *p;
+      *p = 0;
+    }
+    tile[lx * kPmePlane + ly * kPmeRow + lz] = v;
+  }
   const int nbin = cnt[0] * cnt[1] * cnt[2];
-  const int nover = min(d.count[(size_t)d.nb[0] * d.nb[1] * d.nb[2]], d.n);
   auto reach = [&](double c, int a) -> bool {  // the atom's stencil meets it
     int g = (int)c + d.off[a] - t0[a];  // first point, from the tile's
     g = g < 0 ? g + nn[a] : g;
     g = g >= 2 * nn[a] ? g - 2 * nn[a] : (g >= nn[a] ? g - nn[a] : g);
     return g < te[a] || g + P > nn[a];
   };
-  auto take = [&](const double4 &r) {
-    if (!(reach(r.x, 0) && reach(r.y, 1) && reach(r.z, 2))) return;
-    const int k = __hip_atomic_fetch_add(&nlist, 1, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (k < kPmeList) {
-      list[k] = r;
-    } else {  // a full list: this lane adds the atom itself
-      for (int u = 0; u < P; u++) pme_spread_plane<P>(d, r, u, t0, te, tile);
+  // four lanes per bin, 64 bins a turn, as often as the list fills up
+  for (int k0 = 0; k0 < nbin; k0 += 64) {
+    const int k = k0 + (t >> 2);
+    const double4 *rec = d.bucket;
+    int s = t & 3, n = 0;
+    if (k < nbin) {
+      int bx = first[0] + k / (cnt[1] * cnt[2]),
+          by = first[1] + k / cnt[2] % cnt[1], bz = first[2] + k % cnt[2];
+      bx -= bx >= d.nb[0] ? d.nb[0] : 0;
+      by -= by >= d.nb[1] ? d.nb[1] : 0;
+      bz -= bz >= d.nb[2] ? d.nb[2] : 0;
+      const int bin = (bx * d.nb[1] + by) * d.nb[2] + bz;
+      n = min(d.count[bin], d.cap);
+      rec += (size_t)bin * d.cap;
     }
-  };
-  // four lanes per bin, 64 bins a turn; then the overflow list
-  const int turns = (nbin + 63) / 64;
-  for (int turn = 0; turn <= turns; turn++) {
-    if (turn == turns && nover == 0) break;
-    if (t == 0) nlist = 0;
-    __syncthreads();
-    if (turn < turns) {
-      const int k = turn * 64 + (t >> 2);
-      if (k < nbin) {
-        int bx = first[0] + k / (cnt[1] * cnt[2]),
-            by = first[1] + k / cnt[2] % cnt[1], bz = first[2] + k % cnt[2];
-        bx -= bx >= d.nb[0] ? d.nb[0] : 0;
-        by -= by >= d.nb[1] ? d.nb[1] : 0;
-        bz -= bz >= d.nb[2] ? d.nb[2] : 0;
-        const int bin = (bx * d.nb[1] + by) * d.nb[2] + bz;
-        const int n = min(d.count[bin], d.cap);
-        const double4 *rec = d.bucket + (size_t)bin * d.cap;
-        for (int s = t & 3; s < n; s += 4) take(rec[s]);
+    while (true) {
+      if (t == 0) nlist = 0;
+      __syncthreads();
+      for (; s < n; s += 4) {
+        const double4 r = rec[s];
+        if (!(reach(r.x, 0) && reach(r.y, 1) && reach(r.z, 2))) continue;
+        const int at = __hip_atomic_fetch_add(&nlist, 1, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (at >= kPmeList) break;  // again when the list is spread
+        list[at] = r;
       }
-    } else {
-      for (int s = t; s < nover; s += kPmeBlock) take(d.over[s]);
+      __syncthreads();
+      const int listed = nlist;
+      const int items = min(listed, kPmeList) * P;
+      for (int j = t; j < items; j += kPmeBlock)
+        pme_spread_plane<P>(d, list[j / P], j % P, t0, te, tile);
+      __syncthreads();
+      if (listed <= kPmeList) break;
     }
-    __syncthreads();
-    const int items = min(nlist, kPmeList) * P;
-    for (int k = t; k < items; k += kPmeBlock)
-      pme_spread_plane<P>(d, list[k / P], k % P, t0, te, tile);
-    __syncthreads();
   }
   for (int k = t; k < kPmeTile * kPmeTile * kPmeTile; k += kPmeBlock) {
     const int lx = k / (kPmeTile * kPmeTile), ly = k / kPmeTile % kPmeTile,

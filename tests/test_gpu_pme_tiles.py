@@ -34,3 +34,15 @@ def test_large_charges():
     w.topology.scaled_charges *= 1e3
     w.topology.touch()
     check(w, (20, 20, 20), 4, 0.35)
+
+
+@pytest.mark.parametrize("order", [2, 4, 8])
+@pytest.mark.parametrize("squeeze", [0.02, 0.5])
+def test_atoms_in_a_part_of_the_box(order, squeeze):
+    """Far more atoms than a bucket and a tile's list hold, in a few bins."""
+    w = systems.small_water(n_mol=1200, elec="coulomb")
+    w.positions = squeeze * w.positions
+    check(w, (24, 27, 30), order, 0.35)
+    outs, _ = run_device(w, (24, 27, 30), order, 0.35, repeat=3)
+    for f, o in outs[1:]:
+        assert np.array_equal(f, outs[0][0]) and np.array_equal(o, outs[0][1])
