@@ -198,9 +198,8 @@ int pmnb_kernel_timing(pmnb_ctx *ctx, int32_t enable, double *ms,
 /* Pair path a context's evaluations take (known after pmnb_set_box):
    PMNB_PATH_TILE: the algorithm cutoff reaches every pair within the
      switching cutoff, so the pair set does not depend on the cell grid,
-     and at most 8 LJ types: the path's own column grid and tile kernel
-     (9 .. 256 types run that kernel too, with the LJ table in memory, and
-     are reported as the path of their cell grid below);
+     and at most 256 LJ types: the path's own column grid and pair kernel
+     (9 types and more read the LJ table from memory);
    PMNB_PATH_LIST: the reference's cell grid and delta list
      (topology/CellListEnumeratorPeriodicBoundaries.h:46-83) drive a
      neighbour list per evaluation;

@@ -217,7 +217,6 @@ struct pmnb_ctx {
   bool use_list = false;          // neighbour-list path available
   bool use_tile = false;          // LDS-staged path (own column grid)
   bool tile_types = false;        // ... and its types fit the LDS table
-  int ref_shell = 0;              // entries of the reference grid's shell
   // tile path geometry: one replica for a single system, several for a
   // batch (atoms of replica r then carry r in d_rep_of)
   std::vector<TileRep> reps;
@@ -555,7 +554,6 @@ int build_box(pmnb_ctx *ctx, const double *e1, const double *e2,
   ctx->shell.clear();
   ctx->shell.push_back(make_int4(0, 0, 0, 0));
   ctx->shell.insert(ctx->shell.end(), dl.begin(), dl.end());
-  ctx->ref_shell = (int)ctx->shell.size();
   // The mixed kernel takes the image of a neighbour atom from its cell's
   // offset; that is the minimum image only when every cell offset a pair
   // within the cutoff can have, [-reach, reach] with reach taken before the
@@ -567,7 +565,7 @@ int build_box(pmnb_ctx *ctx, const double *e1, const double *e2,
   // Tile path: its own column grid, used when the pair set does not depend
   // on the cell grid (algorithm cutoff >= switching cutoff) and type and atom
   // index fit one word.  More LJ types than the pair kernel's LDS table holds
-  // are read from memory (pmnb_pair_path counts them to the general path).
+  // are read from memory.
   {
     const ForceParams P0 = make_params_for(ctx->prm, ctx->csf);
     const double rcp = std::sqrt(P0.cut2);
@@ -1659,11 +1657,9 @@ int pmnb_kernel_timing(pmnb_ctx *ctx, int32_t enable, double *ms,
 int pmnb_pair_path(const pmnb_ctx *ctx, int32_t *path) {
   if (!ctx || !path) return PMNB_ERR_ARG;
   if (!ctx->have_box || !ctx->have_topo) return PMNB_ERR_STATE;
-  const bool list = ctx->ref_shell <= kMaxShell &&
-                    ctx->n < (1 << kEntryAtomBits);
-  *path = ctx->use_tile && ctx->tile_types ? PMNB_PATH_TILE
-          : list                           ? PMNB_PATH_LIST
-                                           : PMNB_PATH_SCAN;
+  const bool list = ctx->use_list && ctx->n < (1 << kEntryAtomBits);
+  *path = ctx->use_tile ? PMNB_PATH_TILE : (list ? PMNB_PATH_LIST
+                                                 : PMNB_PATH_SCAN);
   return PMNB_OK;
 }
 

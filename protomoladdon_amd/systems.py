@@ -398,8 +398,8 @@ def with_algorithm(w, cutoff, cell_size, name=None):
 
 def many_type_chains(seed=1234, n_chains=60, n_types=12, chain_len=20):
     """small_chains with n_types LJ types (sigma 3.0 .. 4.0 A, epsilon
-    0.05 .. 0.2 kcal/mol, Lorentz-Berthelot): more than the tile path
-    holds, so the force takes the general cell-list path."""
+    0.05 .. 0.2 kcal/mol, Lorentz-Berthelot): more than the tile path's
+    LDS table holds, so its kernel reads the table from memory."""
     L = 138.0 * (n_chains / 12500.0) ** (1.0 / 3.0)
     sigma = tuple(np.linspace(3.0, 4.0, n_types))
     eps = tuple(np.linspace(0.05, 0.2, n_types))

@@ -376,9 +376,9 @@ def test_single_system_of_many_cells():
 # Algorithm cutoff below the switching cutoff (the pair set is the one the
 # reference's cell grid and delta list reach:
 # CellListEnumeratorPeriodicBoundaries.h:46-83,114-134, CubicCellManager.cpp
-# :53-59), and more LJ types than the tile path holds.  The oracle is
-# bitwise equal to the reference's own build on these cases
-# (tests/test_oracle.py).
+# :53-59), and systems whose LJ table does not fit the tile kernel's LDS.  The
+# oracle is bitwise equal to the reference's own build on these cases but the
+# last (tests/test_oracle.py).
 GENERAL = {
     # 6.5 A cell reach, 9 A C2 cutoff, 3 A cells: neighbour-list kernels
     "water_acut": (lambda: systems.with_algorithm(
@@ -390,8 +390,11 @@ GENERAL = {
     # more than 512 cell offsets: the direct-scan kernels
     "water_scan": (lambda: systems.with_algorithm(
         systems.small_water(n_mol=300), 8.9, 1.5), "scan"),
-    # 12 LJ types: the reference grid with its full delta list
-    "chains_12types": (lambda: systems.many_type_chains(), "list"),
+    # 12 LJ types with 1-4 pairs: the tile kernel with its table in memory
+    "chains_12types": (lambda: systems.many_type_chains(), "tile"),
+    # the same with the first case's reach: neighbour-list kernels
+    "chains_12types_acut": (lambda: systems.with_algorithm(
+        systems.many_type_chains(), 6.5, 3.0), "list"),
 }
 
 
