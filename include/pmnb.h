@@ -144,20 +144,23 @@ int pmnb_evaluate_device(pmnb_ctx *ctx, const double *d_positions,
                          void *stream);
 
 /* pmnb_evaluate_device without any allocation: same arguments, results
-   and kernels (bit for bit), with every per-evaluation array (cell counts
-   and starts, the sorted atom arrays, work items, partial sums, the
-   fixed-point force array, the grid and box) in one static device array
-   of 64 MiB per GPU instead of the context's buffers; nothing is
+   and kernels (bit for bit), with every per-evaluation array (bin counts
+   and buckets, cell starts, the sorted atom arrays, work items, partial
+   sums, the grid and box) in one static device array of 64 MiB per GPU
+   instead of the context's buffers; nothing is
    allocated or freed and no host copy is made.  No counterpart in the
    reference: it is for callers that cannot allocate device memory (code
    under HIP graph capture, tight serving loops, harnesses that forbid
    allocation).  Covers one system on the tile path (algorithm cutoff >=
    the switching cutoff, at most 8 LJ types): PMNB_ERR_UNSUPPORTED
-   otherwise; PMNB_ERR_CAPACITY when the system needs more than 64 MiB
-   (100 bytes per atom mixed, 124 FP64, plus 128 per 16 atoms and, per
-   cell, 8 and 4 per bucket slot, at least 4 times the mean occupancy:
-   about 520,000 atoms of water mixed, 425,000 FP64).  Every call on one GPU
-   shares that GPU's array, which
+   otherwise; PMNB_ERR_CAPACITY when the system's size is above 64 MiB.
+   The size is a fixed rule that covers what the arrays take: 100 bytes
+   per atom mixed, 124 FP64; 128 per 16 atoms; 128 per column of one
+   cutoff by one cutoff; and, per cell of a third (FP64 a quarter) of the
+   cutoff of these columns, 8 and 4 times the smallest power of two from 64
+   to 512 that is at least 4 times the mean atoms per cell: about 520,000
+   atoms of water mixed, 425,000 FP64.  Every call on one GPU shares that
+   GPU's array, which
    keeps the last call's contents: calls that overlap on one GPU (other
    streams or threads) race.  pmnb_last_pair_count does not see these
    calls.  PMNB_ERR_STATE while kernel timing is on. */

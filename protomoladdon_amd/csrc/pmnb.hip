@@ -3821,11 +3821,12 @@ EvalBufs carve_bufs(const pmnb_ctx *ctx, unsigned char *base, int cap,
   return B;
 }
 
-// The bytes the documented limit counts for one system: 100 (FP64 124) per
-// atom, 128 per 16 atoms and column and, per cell of a grid of columns one
-// cutoff wide with z cells of a third (FP64 a quarter) of the cutoff, 8 and 4
-// per bucket slot, at least 4 times the mean occupancy.
-size_t scratch_limit_bytes(const pmnb_ctx *ctx) {
+// The size include/pmnb.h gives one system against the 64 MiB: which systems
+// the entry takes is part of its interface and does not follow the layout of
+// carve_bufs, whose arrays are smaller (over boxes of 10 to 4,000 A, cutoffs
+// of 6 to 16 A and 1 to 700,000 atoms within the limit, at most 53 MiB with the
+// shortest bucket rows).
+size_t scratch_limit_size(const pmnb_ctx *ctx) {
   const bool mixed = ctx->prm.precision == PMNB_PREC_MIXED;
   const double rcp = std::sqrt(make_params_for(ctx->prm, ctx->csf).cut2);
   auto cells = [&](int k, double w) {
@@ -3887,7 +3888,11 @@ int pmnb_evaluate_device_noalloc(pmnb_ctx *ctx, const double *d_positions,
   carve_bufs(ctx, nullptr, cap, need);
   while (need > kScratchBytes && cap > 64)
     carve_bufs(ctx, nullptr, cap /= 2, need);
-  need = std::max(need, scratch_limit_bytes(ctx));
+  const size_t size = scratch_limit_size(ctx);
+  if (size > kScratchBytes)
+    return fail(ctx, PMNB_ERR_CAPACITY,
+                "the system's size by the entry's rule is %zu, above the limit "
+                "of %zu (64 MiB)", size, kScratchBytes);
   if (need > kScratchBytes)
     return fail(ctx, PMNB_ERR_CAPACITY,
                 "the evaluation needs %zu bytes of scratch; the static scratch "

@@ -76,7 +76,7 @@ def test_noalloc_refuses_what_it_does_not_cover():
         f.evaluate_device_noalloc(w.topology, pos, frc, out, 1)
     assert e.value.code == 3  # PMNB_ERR_UNSUPPORTED
     f.close()
-    # 600,000 atoms need more than the 64 MiB scratch
+    # 600,000 atoms are above the entry's 64 MiB rule
     n_mol = 200000
     big = systems.water_workload("water600k", n_mol,
                                  (n_mol / systems.WATER_DENSITY) ** (1 / 3),
@@ -87,5 +87,18 @@ def test_noalloc_refuses_what_it_does_not_cover():
     with pytest.raises(PmnbError) as e:
         f.evaluate_device_noalloc(big.topology, pos, frc, out, 1)
     assert e.value.code == 5  # PMNB_ERR_CAPACITY
+    assert "rule" in str(e.value)
     assert not frc.abs().max().item()
     f.close()
+
+
+@pytest.mark.parametrize("precision,n_mol", [("mixed", 173000), ("fp64", 141000)])
+def test_noalloc_up_to_its_limit(precision, n_mol):
+    """Systems just within the entry's size rule fit its arrays."""
+    w = systems.water_workload("water_limit", n_mol,
+                               (n_mol / systems.WATER_DENSITY) ** (1 / 3),
+                               7, 9.0, 7.5, "ewald", alpha=0.32)
+    (f0, o0), (f1, o1) = both(w, precision)
+    assert np.abs(f0).max() > 0
+    np.testing.assert_array_equal(f1, f0)
+    np.testing.assert_array_equal(o1, o0)
