@@ -821,11 +821,15 @@ __global__ void k_xcode(const unsigned long long *__restrict__ xown, int n,
   xcode[a] = c;
 }
 
-// FP32 copy of the LJ table (T*T records {A, B, A14, B14}).
+// FP32 copies of the LJ table (T*T records {A, B, A14, B14}, plain, then
+// scaled).
 __global__ void k_lj_to_f32(const double *__restrict__ lj, int n,
-                            int elec, float4 *__restrict__ ljf) {
+                            float4 *__restrict__ ljf) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) ljf[k] = lj_record(lj + 4 * k, elec);
+  if (k < n) {
+    ljf[k] = lj_record(lj + 4 * k, false);
+    ljf[n + k] = lj_record(lj + 4 * k, true);
+  }
 }
 
 template <typename R>
@@ -995,7 +999,9 @@ Sorted make_sorted(const pmnb_ctx *ctx, const EvalBufs &B,
   S.xown = ctx->d_xown.as<unsigned long long>();
   S.xcode = S.xown + 4 * (size_t)ctx->n;
   S.lj = ctx->d_lj.as<double>();
-  S.ljf = ctx->d_ljf.as<float4>();
+  const bool scaled = ctx->use_tile && ctx->prm.elec != PMNB_ELEC_NONE;
+  S.ljf = ctx->d_ljf.as<float4>() +
+          (scaled ? (size_t)ctx->ntypes * ctx->ntypes : 0);
   S.com = d_com;
   return S;
 }
@@ -1305,13 +1311,14 @@ int pmnb_set_topology(pmnb_ctx *ctx, int32_t n_atoms, const int32_t *type,
   // holds one record per unordered type pair.
   const int T = n_types;
   std::vector<double> ljd((size_t)T * T * 4);
-  std::vector<float4> ljf((size_t)T * T);
+  std::vector<float4> ljf((size_t)2 * T * T);  // plain, then scaled
   for (int i = 0; i < T; i++)
     for (int j = 0; j < T; j++) {
       const int lo = std::min(i, j), hi = std::max(i, j);
       const double *src = lj + 4 * ((size_t)lo * T + hi);
       for (int k = 0; k < 4; k++) ljd[4 * ((size_t)i * T + j) + k] = src[k];
-      ljf[(size_t)i * T + j] = lj_record(src, ctx->prm.elec);
+      ljf[(size_t)i * T + j] = lj_record(src, false);
+      ljf[(size_t)(T + i) * T + j] = lj_record(src, true);
     }
   const size_t N = (size_t)std::max(n_atoms, 1);
   HIPCHK(ctx->d_type.ensure(N * sizeof(int)));
@@ -1722,8 +1729,7 @@ int pmnb_set_parameters_device(pmnb_ctx *ctx, const double *d_lj,
     HIPCHK(hipMemcpyAsync(ctx->d_lj.p, d_lj, (size_t)nlj * 4 * sizeof(double),
                           hipMemcpyDeviceToDevice, s));
     hipLaunchKernelGGL(k_lj_to_f32, dim3(blocks_for(nlj)), dim3(kBlock), 0, s,
-                       ctx->d_lj.as<double>(), nlj, ctx->prm.elec,
-                       ctx->d_ljf.as<float4>());
+                       ctx->d_lj.as<double>(), nlj, ctx->d_ljf.as<float4>());
   }
   if (d_scaled_charge && ctx->n > 0)
     HIPCHK(hipMemcpyAsync(ctx->d_q.p, d_scaled_charge,

@@ -37,20 +37,26 @@ struct Sorted {
                                    // distance d = -15 .. 15 (bits 2 d + 30):
                                    // its class, FULL for the atom itself
   const double *lj;              // T*T*4 {A, B, A14, B14}
-  const float4 *ljf;             // same in FP32
+  const float4 *ljf;             // same in FP32 (lj_record)
   const double *com;             // molecule centres (molecular virial)
   const Box *box;                // device copy of the box (read on demand)
 };
 
-// FP32 record of an LJ table entry {A, B, A14, B14}.  The pair kernels' 1/r^2
-// comes from v_rsq_f32 squared (v_rcp_f32 without electrostatics), which are
-// low by 7.4e-9 (6.8e-9) on average (over all mantissas, measured); in the
-// sixth and seventh power, the same for every pair, that is 1e-7 of the
-// virial.  A and B carry the inverse of what r^-12 and r^-6 (6.5 and 3.5
-// factors 1/r^2, between the energy's and the force's) lose.
+// FP32 records of an LJ table entry {A, B, A14, B14}: as it is, and (scaled)
+// for the tile path with electrostatics, whose 1/r^2 is v_rsq_f32 squared.  That
+// is low by 7.4e-9 a factor on average (over all mantissas, measured): A and B
+// are multiplied by 1 + 9.6e-8 and 1 + 5.2e-8, what r^-12 and r^-6 lose with 6.5
+// and 3.5 factors 1/r^2 (between the energy's and the force's), and rounded.
+// One entry moves by a unit in the last place or not at all, as the rounding
+// falls, so it is the mean over tables and positions that moves.  48 boxes of
+// 700 waters with random tables, Ewald real space, mean error an atom without /
+// with it: LJ energy -4.4e-8 / 2.0e-8 kcal/mol, virial trace -9.0e-7 / 2.3e-7.
+// Without electrostatics (v_rcp_f32) and on the list kernels, whose own roundings
+// go the other way, it took the virial's from 2.1e-7 to 9.2e-7 and from 2.1e-6
+// to 3.4e-6: they read the plain records.
 __host__ __device__ __forceinline__ float4 lj_record(const double *v,
-                                                     int elec) {
-  const double b = elec != 0 ? 2.0 * 7.39e-9 : 6.75e-9;
+                                                     bool scaled) {
+  const double b = scaled ? 2.0 * 7.39e-9 : 0.0;
   const double a = 1.0 + 6.5 * b, c = 1.0 + 3.5 * b;
   return make_float4((float)(v[0] * a), (float)(v[1] * c), (float)(v[2] * a),
                      (float)(v[3] * c));
