@@ -286,12 +286,15 @@ __device__ __forceinline__ void pair_fma64(const ForceParams &P, double d2,
   double f1 = fma(r6, a6, e1) * (6.0 * rd2);
   double f2 = 0.0;
   e2 = 0.0;
+  // coincident atoms: rsq64 is NaN; the electrostatic energy is infinite (fmin
+  // and fmax return the number)
+  const double re = fmin(rr, __builtin_inf());
   if (ELEC == 1) {
-    e2 = qq * rr;
+    e2 = qq * re;
     f2 = e2 * rd2;
   } else if (ELEC == 2) {
     // Abramowitz & Stegun 7.1.26 (base/MathUtilities.cpp:39-49)
-    const double ar = P.alpha * (d2 * rr);
+    const double ar = P.alpha * fmax(d2 * rr, 0.0);
     const double t = rcp64(fma(0.3275911, ar, 1.0));
     const double poly =
         t * fma(t, fma(t, fma(t, fma(t, 1.061405429, -1.453152027),
@@ -299,7 +302,7 @@ __device__ __forceinline__ void pair_fma64(const ForceParams &P, double d2,
                        -0.284496736),
                 0.254829592);
     const double e = qq * exp64_neg(-ar * ar);
-    e2 = poly * e * rr;
+    e2 = poly * e * re;
     f2 = fma(P.two_alpha_pi, e, e2) * rd2;
   }
   auto c2 = [&](const Switch &s, double &v, double &dv) {
@@ -322,7 +325,7 @@ __device__ __forceinline__ void pair_fma64(const ForceParams &P, double d2,
     c2(P.sw_el, v, dv);
   } else {
     // C1SwitchingFunction (switch/C1SwitchingFunction.h:41-50)
-    const double dist = d2 * rr;
+    const double dist = fmax(d2 * rr, 0.0);
     const bool in = d2 <= P.sw_el.cut2;
     v = in ? fma(-dist, fma(-d2, P.sw_el.c1_05c3, P.sw_el.c1_15c1), 1.0) : 0.0;
     dv = in ? fma(dist, P.sw_el.c1_15c3, -P.sw_el.c1_15c1 * rr) : 0.0;

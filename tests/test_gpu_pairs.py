@@ -5,6 +5,7 @@ bit, FP64 forces within 1e-11 of the largest component, mixed forces within
 import numpy as np
 import pytest
 
+from oracle import oracle as O
 from protomoladdon_amd import systems
 from protomoladdon_amd.batch import BatchedCutoffForce
 from protomoladdon_amd.topology import (EXCLUSION_FULL, EXCLUSION_MODIFIED,
@@ -172,3 +173,25 @@ def test_virial_over_tables_and_positions():
         err.append((tr[1] - tr[0]) / w.n_atoms)
     print("mean %.3g, scatter %.3g" % (np.mean(err), np.std(err)), flush=True)
     assert abs(np.mean(err)) <= 6e-7
+
+
+@pytest.mark.parametrize("elec", ["coulomb", "ewald"])
+@pytest.mark.parametrize("switch", ["C2", "other C2", "C1"])
+@pytest.mark.parametrize("who", [(0, 3), (0, 4)])
+def test_coincident_atoms_fp64(elec, switch, who):
+    """The electrostatic energy of two atoms in one place is infinite, of
+    their charges' sign; their forces and the LJ energy are NaN, as the
+    reference's arithmetic gives them."""
+    w = systems.small_water(n_mol=300, elec=elec)
+    if switch == "other C2":
+        w.elec_switch = (7.0, 9.0)
+    elif switch == "C1":
+        w.elec_switch = ("C1", 9.0)
+    p = w.positions.copy()
+    p[who[0]] = p[who[1]]
+    ref = O.evaluate(O.System.from_workload(w, positions=p, flags=0))
+    f, e, _, _ = run_gpu(w, "fp64", 0, positions=p, with_pairs=False)
+    assert np.isinf(ref.energies[1])
+    assert e[SS.COULOMB] == ref.energies[1]
+    assert np.isnan(e[SS.LENNARDJONES]) and np.isnan(ref.energies[0])
+    np.testing.assert_array_equal(np.isnan(f), np.isnan(ref.forces))
