@@ -396,7 +396,6 @@ bool make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
   rep.tg.nx = tx;
   rep.tg.ny = ty;
   rep.tg.nz = tz;
-  rep.tg.rz = rz;
   rep.tg.csx = (float)tg.cs[0];
   rep.tg.csy = (float)tg.cs[1];
   rep.tg.csz = (float)tg.cs[2];

@@ -188,8 +188,6 @@ __device__ __forceinline__ double poly5_exact(double ar) {
   return (t) * (E1 + (t) * (E2 + (t) * (E3 + (t) * (E4 + (t) * E5))));
 }
 
-// Exclusion class of atoms a, b of the same molecule from the per-atom
-// masks (bit d-1 of full[min]/mod[min] holds pair (min, min + d)).
 // Exclusion class of the pair (a, a + d) from atom a's own masks m =
 // {forward FULL, forward MODIFIED, reverse FULL, reverse MODIFIED} (bit
 // |d| - 1; forward for d > 0, reverse for d < 0): the same answer as
@@ -204,6 +202,8 @@ __device__ __forceinline__ int excl_own(const unsigned long long *m, int d) {
   return 0;
 }
 
+// Exclusion class of atoms a, b of the same molecule from the per-atom
+// masks (bit d-1 of full[min]/mod[min] holds pair (min, min + d)).
 __device__ __forceinline__ int excl_class(const unsigned long long *full,
                                           const unsigned long long *mod,
                                           int max_delta, int a, int b) {

@@ -39,7 +39,6 @@ struct Sorted {
   const double *lj;              // T*T*4 {A, B, A14, B14}
   const float4 *ljf;             // same in FP32 (lj_record)
   const double *com;             // molecule centres (molecular virial)
-  const Box *box;                // device copy of the box (read on demand)
 };
 
 // FP32 records of an LJ table entry {A, B, A14, B14}: as it is, and (scaled)

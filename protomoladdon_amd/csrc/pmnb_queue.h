@@ -28,7 +28,7 @@ constexpr int kQTypeShift = 24;  // bits of an atom index beside its type
 struct TileRep {
   Box box;            // FP64 box: minimum image of pairs near the cutoff
   Grid grid;          // FP64 column grid (cell assignment)
-  TileGrid tg;        // FP32 cell sizes and the z reach of the cutoff
+  TileGrid tg;        // FP32 cell sizes
   float L[3], iL[3];  // box lengths and inverses
   float Llo[3];       // what rounding the lengths to FP32 left of them
   int wrap[2];        // x, y: per-pair minimum image, each column once

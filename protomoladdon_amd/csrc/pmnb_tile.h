@@ -19,7 +19,7 @@ namespace pmnb {
 constexpr int kTileAtoms = 16;   // atoms per wave
 
 struct TileGrid {
-  int nx, ny, nz, rz;   // grid and z-cell reach of the cutoff
+  int nx, ny, nz;       // grid
   float csx, csy, csz;  // cell sizes
   float lox, loy, loz;  // ... and what rounding to FP32 left of them
 };
