@@ -949,8 +949,9 @@ int build_cells(pmnb_ctx *ctx, const EvalBufs &B, const double *d_pos,
                            dim3(kBinGroup), 0, s, B.reps, (int)r, B.count,
                            B.group, B.items);
     const int *bin_rep = ctx->batch ? ctx->d_bin_rep.as<int>() : nullptr;
-    hipLaunchKernelGGL(k_sort_bins, dim3(ctx->nbin), dim3(kBlock), 0, s, B.reps,
-                       bin_rep, d_pos, B.count, B.bucket, B.cap, B.cell_of,
+    hipLaunchKernelGGL(ctx->ngroup ? k_sort_bins<true> : k_sort_bins<false>,
+                       dim3(ctx->nbin), dim3(kBlock), 0, s, B.reps, bin_rep,
+                       d_pos, B.count, B.bucket, B.cap, B.cell_of,
                        ctx->d_type.as<int>(), ctx->d_q.as<double>(),
                        ctx->d_mol.as<int>(), O);
     HIPCHK(hipGetLastError());
