@@ -169,12 +169,11 @@ def test_config3_full_size_512_replicas():
 
 
 @pytest.mark.parametrize("precision,shape", [("mixed", 2), ("fp64", 1)])
-def test_half_shell_shape_matches_oracle(replicas, precision, shape):
-    """The half-shell pair kernel (each pair evaluated once, the partner's
-    force added through fixed-point LDS slots and global integer atomics),
-    selected as a batch shape: the pairs it evaluates are the oracle's, bit
-    for bit, forces and energies within the bars of the full shell, and
-    repeated evaluations are bitwise equal."""
+def test_last_shape_matches_oracle(replicas, precision, shape):
+    """The last pair-kernel shape of each precision (mixed: a block per work
+    item, FP64: a wave per item), selected by hand: the pairs it evaluates are
+    the oracle's, bit for bit, forces and energies within the bars of the
+    other shapes, and repeated evaluations are bitwise equal."""
     bf = BatchedCutoffForce.from_workloads(replicas, precision=precision)
     bf.set_shape(shape)
     pos, frc, out = batch_eval(bf, replicas)

@@ -26,7 +26,8 @@ def dimers(n_pairs, L):
     rng = np.random.default_rng(7)
     k = int(np.ceil(n_pairs ** (1 / 3)))
     site = np.stack(np.unravel_index(np.arange(n_pairs), (k, k, k)), 1)
-    O = (site + 0.5) * (L / k) + rng.uniform(-9, 9, (n_pairs, 3))
+    room = min(9.0, 0.5 * (L / k - 15.0))
+    O = (site + 0.5) * (L / k) + rng.uniform(-room, room, (n_pairs, 3))
     d = rng.normal(size=(n_pairs, 3))
     d /= np.linalg.norm(d, axis=1)[:, None]
     r = np.where(np.arange(n_pairs) % 2, rng.uniform(2.8, 3.2, n_pairs),
@@ -39,11 +40,13 @@ def dimers(n_pairs, L):
     return w
 
 
-def test_dimers_in_a_wide_box():
+@pytest.mark.parametrize("n_pairs,L", [(300, 2400.0), (400, 150.0)])
+def test_dimers_in_a_wide_box(n_pairs, L):
     """2,400 A: with columns and cells far wider than the cutoff the FP32
-    offsets in a cell lose the pairs near the cutoff."""
-    check_fp64(dimers(300, 2400.0))
-    check_mixed(dimers(300, 2400.0))
+    offsets in a cell lose the pairs near the cutoff.  150 A: work items whose
+    atoms spread beyond the expanded distance test."""
+    check_fp64(dimers(n_pairs, L))
+    check_mixed(dimers(n_pairs, L))
 
 
 def dense_in_wide_box(n_mol, L, squeeze):

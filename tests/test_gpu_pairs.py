@@ -39,8 +39,8 @@ def stretched(sx, sy, sz, n_mol=500):
 
 
 def gas(n_mol, L):
-    """A thin gas: wide columns and cells, items whose atoms spread beyond
-    the expanded distance test."""
+    """A thin gas, without one pair (tests/test_gpu_density.py has gases
+    with pairs)."""
     return systems.water_workload("gas", n_mol, L, 5, 9.0, 7.5, "ewald", 0.32)
 
 

@@ -345,11 +345,10 @@ def test_large_config_properties(which):
 
 
 def test_single_system_of_many_cells():
-    """A single system of more than 16,384 tile cells (27,000 waters with a
-    5 A cutoff: 18 x 18 columns of 55 z cells mixed, 74 FP64), whose cell
-    starts and work items are built over the columns in three launches
-    instead of one block: the pair record of both precisions equals the
-    oracle's pair set, FP64 forces within 1e-11, mixed RMS within 1e-5."""
+    """A single system of many small tile cells (27,000 waters with a 5 A
+    cutoff: 37 x 37 columns of 60 z cells, more than one atom in few of them):
+    the pair record of both precisions equals the oracle's pair set, FP64
+    forces within 1e-11, mixed RMS within 1e-5."""
     w = systems.small_water(n_mol=27000, rc=5.0, rs=4.0)
     L = (27000 / systems.WATER_DENSITY) ** (1.0 / 3.0)
     assert int(L / 5.0) ** 2 * int(L / (5.0 / 3.0)) > 16384
