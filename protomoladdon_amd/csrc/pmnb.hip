@@ -177,13 +177,14 @@ int host_crew_size() {
 // pmnb_evaluate shares its host copy and add over the crew for systems of
 // at least kHostCrewMin coordinates
 constexpr int kHostCrewMin = 1 << 16;
-// A pair launch of fewer work items than this takes a block per item (a wave
-// per stream of candidates) instead of a wave per item: the chip holds 1,024
-// SIMDs, and below about three items each the longest wave decides.  A block
-// per item repeats the item's setup in four waves.  A whole evaluation with
-// energies of water, a wave / a block per item: 187 items 88 / 43 us, 1,500
-// items 94 / 75, 2,250 101 / 93, 3,000 112.5 / 112.4, 3,750 120 / 132, 6,000
-// 176 / 187.
+// A pair launch of fewer work-item slots than this takes a block per item (a
+// wave per stream of candidates) instead of a wave per item: the chip holds
+// 1,024 SIMDs, and below about three items each the longest wave decides.  A
+// block per item repeats the item's setup in four waves.  The host knows the
+// slots (a sixteenth of the atoms and one per bin), not the items, which are
+// fewer by half a bin's slot in a filled box.  A whole evaluation with energies
+// of water, a wave / a block per item: 223 slots 88 / 43 us, 1,669 slots 94 /
+// 75, 2,475 101 / 93, 3,289 112.5 / 112.4, 4,074 120 / 132, 6,441 176 / 187.
 constexpr int kSplitItems = 3000;
 
 struct pmnb_ctx {

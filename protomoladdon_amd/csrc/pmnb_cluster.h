@@ -41,14 +41,18 @@
 // one comparison per pair; the class then comes from a 62-bit code of the
 // lane's own atom (or from its masks when a distance is over 15).
 //
-// Bound by VALU issue (85% of the issue slots; LDS, L2 and HBM idle most of
-// the time): on the 96,000-atom water (9 A, LJ + Ewald real space) 1.1e4 wave
-// instructions an item, three quarters of them the pairs' arithmetic.
+// The mixed forms are bound by VALU issue (84% of the issue slots with
+// energies, 81% forces only; LDS, L2 and HBM idle most of the time): on the
+// 96,000-atom water (9 A, LJ + Ewald real space) 1.1e4 wave instructions an
+// item, three quarters of them the pairs' arithmetic.  The FP64 forms issue 61%
+// of the slots at three waves a SIMD; what fills the rest is not separated (the
+// quarter-rate instructions, or the waits for a pair's FP64 record and LJ entry,
+// which are read from LDS right before use).
 // Columns of half a cutoff and z runs cut per column leave 2.2 candidates a
 // pair where columns of one cutoff left 4.4.  Measured against that layout
 // with its z-level loop (3 x 3 columns, one z cell of the columns a time):
 //   96,000 atoms   160 -> 137 us forces only, 205 -> 157 with energies
-//   the same, FP64 540 -> 412 (508 with IEEE quotients, roots and exp)
+//   the same, FP64 540 -> 417 (508 with IEEE quotients, roots and exp)
 //   522,000 atoms in 128 boxes  751 -> 603, 1,076 -> 690 (half shell before)
 //   3,000 atoms, 10 A Coulomb   104 -> 35 (a block an item)
 //   30,000 atoms of 12 types    1,293 (neighbour list) -> 83

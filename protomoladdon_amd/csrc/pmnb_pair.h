@@ -269,9 +269,10 @@ __device__ __forceinline__ double exp64_neg(double x) {
 }
 
 // The FP64 pair of the tile path: A, B and qq carry the 1-4 factor, d2 is the
-// exact one that decided the pair.  SAME: one C2 switch for both terms.  421 us
-// for the 96,000-atom water where pair_f64 took 508; the error of forces and
-// energies against 64-bit references is no larger (1.2e-15, 1.6e-15 before).
+// exact one that decided the pair.  SAME: one C2 switch for both terms.  417 us
+// an evaluation of the 96,000-atom water, 508 with IEEE quotients, roots and
+// exp in the reference's order; the error of forces and energies against 64-bit
+// references is no larger (1.2e-15, 1.6e-15 before).
 template <int ELEC, int ELSW, bool SAME>
 __device__ __forceinline__ void pair_fma64(const ForceParams &P, double d2,
                                            double A, double B, double qq,

@@ -247,7 +247,7 @@ __device__ __forceinline__ void pme_spread_plane(const PmeDev &d,
 // One block per tile of 8^3 grid points (fewer at the upper faces).  Its
 // points are written by it alone, so no global atomics: 6.1 million of them
 // took 156 us for 96,000 atoms of order 4 on a 96^3 grid, plus 8 us to convert
-// and clear the integer grid; this kernel takes 30 us and k_pme_bin 10 (bound by
+// and clear the integer grid; this kernel takes 27 us and k_pme_bin 9 (bound by
 // its atomics' latency), this one by its LDS atomics (a tile with margins, which
 // needs no test per point but adds 1.9 times as many, took 51).  Bins half a
 // tile wide: 4 per axis reach a tile, 8 atoms are read for one of the tile's own
