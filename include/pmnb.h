@@ -201,8 +201,9 @@ int pmnb_kernel_timing(pmnb_ctx *ctx, int32_t enable, double *ms,
 /* Pair path a context's evaluations take (known after pmnb_set_box):
    PMNB_PATH_TILE: the algorithm cutoff reaches every pair within the
      switching cutoff, so the pair set does not depend on the cell grid,
-     and at most 256 LJ types: the path's own column grid and pair kernel
-     (9 types and more read the LJ table from memory);
+     at most 256 LJ types, and a box of fewer than 2^26 cells of that cutoff
+     each way: the path's own column grid and pair kernel (9 types and more
+     read the LJ table from memory);
    PMNB_PATH_LIST: the reference's cell grid and delta list
      (topology/CellListEnumeratorPeriodicBoundaries.h:46-83) drive a
      neighbour list per evaluation;
@@ -264,8 +265,9 @@ int pmnb_adjoint_device(pmnb_ctx *ctx, const double *d_positions,
    independent periodic systems that share one force (params, LJ table,
    coulomb scaling factor) and evaluates them all with one launch of each
    kernel; replica r's result is what pmnb_evaluate_device gives for that
-   replica alone.  Replicas use the tile path, which needs the algorithm
-   cutoff >= the switching cutoff and at most 8 LJ types. */
+   replica alone.  Replicas use the tile path (pmnb_pair_path), which needs
+   the algorithm cutoff >= the switching cutoff, at most 8 LJ types here and
+   boxes of fewer than 2^26 cells of the cutoff each way. */
 typedef struct pmnb_batch pmnb_batch;
 
 /* Creates an empty batch; lj and coulomb_scaling_factor as in

@@ -10,6 +10,7 @@ import pytest
 
 from oracle import oracle as O
 from protomoladdon_amd import systems
+from protomoladdon_amd._lib import PmnbError
 from protomoladdon_amd.batch import BatchedCutoffForce
 from protomoladdon_amd.topology import PeriodicBoundaryConditions
 from tests.test_gpu_batch import batch_eval, single_eval
@@ -18,11 +19,11 @@ from tests.test_gpu_parity import check_fp64, check_mixed, rms_rel
 pytestmark = pytest.mark.gpu
 
 
-def dimers(n_pairs, L):
+def dimers(n_pairs, L, cell_size=50.0):
     """Pairs of waters, oxygens 2.8 to 3.2 A or 8.9 to 9.1 A apart (the
     cutoff is 9 A), far from all other pairs."""
     w = systems.water_workload("dimers", 2 * n_pairs, L, 6, 9.0, 7.5, "ewald",
-                               0.32, cell_size=50.0)
+                               0.32, cell_size=cell_size)
     rng = np.random.default_rng(7)
     k = int(np.ceil(n_pairs ** (1 / 3)))
     site = np.stack(np.unravel_index(np.arange(n_pairs), (k, k, k)), 1)
@@ -47,6 +48,22 @@ def test_dimers_in_a_wide_box(n_pairs, L):
     atoms spread beyond the expanded distance test."""
     check_fp64(dimers(n_pairs, L))
     check_mixed(dimers(n_pairs, L))
+
+
+def test_box_beyond_the_tile_grid():
+    """3,800 A are more than 2^26 cells of a 9 A cutoff: one system takes the
+    cell grid of its cell size, a batch refuses the box."""
+    w = dimers(200, 3800.0, 16.0)
+    f = w.make_force("mixed")
+    assert f.pair_path(w.topology) != "tile"
+    f.close()
+    check_fp64(w)
+    check_mixed(w)
+    bf = BatchedCutoffForce.from_workloads([w], precision="mixed")
+    with pytest.raises(PmnbError) as e:
+        batch_eval(bf, [w])
+    assert e.value.code == 3  # PMNB_ERR_UNSUPPORTED
+    bf.close()
 
 
 def dense_in_wide_box(n_mol, L, squeeze):
