@@ -324,6 +324,11 @@ Switch make_c1(double cut) {
 }
 
 // Switching constants and the pair cutoff, from the force parameters alone.
+// |d2_f32 - cut2| below which FP64 decides a pair
+float pair_band(double cut2) {
+  return 1.0e-3f * (float)std::max(1.0, cut2 / 100.0);
+}
+
 ForceParams make_params_for(const pmnb_params &prm, double csf) {
   ForceParams P{};
   P.sw_lj = make_c2(prm.lj_switchon, prm.lj_cutoff);
@@ -341,25 +346,33 @@ ForceParams make_params_for(const pmnb_params &prm, double csf) {
   P.csf = csf;
   P.elec = prm.elec;
   P.el_switch = prm.elec_switch;
-  P.band = 1.0e-3f * (float)std::max(1.0, P.cut2 / 100.0);
+  P.band = pair_band(P.cut2);
   return P;
 }
 
 // Column grid of the tile path for box b, pair cutoff rcp and n atoms: x/y
 // columns at least rcp / 2 wide, z cells of about rcp / 8.  A box whose columns
-// would hold fewer than 16 atoms on average gets columns of up to rcp and z
-// cells of up to rcp / 3, so that a work item still holds several atoms; never
-// wider, whatever the mean density: the atoms may be a dense part of a large
+// would hold fewer than 32 atoms on average gets columns of up to rcp and z
+// cells of up to rcp / 3, so that work items are filled (90,000 atoms in a flat
+// box of 310 x 310 x 9.3 A, 18 an rcp / 2 column: 213 us with 16 atoms on
+// average, 193 with 32, 181 with 48, which slows the FP64 rods of 18.6 x 18.6 A
+// from 297 to 319); never wider, whatever the mean density: the atoms may be a dense part of a large
 // box (a droplet of 32,000 atoms in an 830 A box: 8,180 us with columns of
 // 16 atoms on average, 19 A wide, 372 with these), and coordinates are
 // FP32 offsets from the corner of a cell (columns of 300 A leave them an error
 // beyond `band`, and so another pair set).  False: more than 2^26 columns of
 // rcp by cells of rcp, which the reference's grid takes.
-// An axis with fewer than five columns is marked for the per-pair minimum
-// image.  A column's z cells are split into bins of at most 256 cells and about
+// An axis with fewer than four columns is marked for the per-pair minimum
+// image, and so is one with four in FP64.  In mixed precision the column offsets
+// -2 and 2 of four columns reach the same column at images one box length apart,
+// at most one of which is within the cutoff and its band (a box shorter than
+// that is marked too).  64 boxes of 240 / 300 / 330 waters, the image of every
+// pair: mixed 132 / 190 / 197 us, FP64 283 / 367 / 401; the column at two images:
+// 134 / 180 / 191, 333 / 420 / 423; 1,200 x 7 x 7 waters mixed 449 and 409.  A
+// column's z cells are split into bins of at most 256 cells and about
 // 256 atoms.  shell receives the distinct cell offsets within reach ((0,0,0)
 // first), which the pair-set extraction walks.
-bool make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
+bool make_tile_rep(const Box &b, double rcp, int n, bool mixed, TileRep &rep,
                    std::vector<int4> &shell) {
   auto cells = [&](int axis, double w) {
     return std::max(1.0, std::floor(b.H[axis] / w));
@@ -370,7 +383,7 @@ bool make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
   // the fewest columns of an axis: rcp wide, five where there are five
   const int mx = std::max((int)cells(0, rcp), std::min(tx, 5)),
             my = std::max((int)cells(1, rcp), std::min(ty, 5));
-  const double most = n / 16.0;
+  const double most = n / 32.0;  // columns of 32 atoms, two items, on average
   while ((double)tx * ty > most && (tx > mx || ty > my)) {
     const bool x = ty <= my || (tx > mx && tx >= ty);
     int &k = x ? tx : ty;
@@ -408,8 +421,9 @@ bool make_tile_rep(const Box &b, double rcp, int n, TileRep &rep,
     rep.Llo[k] = (float)(b.e[k] - (double)rep.L[k]);
     rep.iL[k] = (float)b.er[k];
   }
-  rep.wrap[0] = tx < 5;
-  rep.wrap[1] = ty < 5;
+  const double twice = rcp + std::sqrt(rcp * rcp + 4.0 * pair_band(rcp * rcp));
+  rep.wrap[0] = tx < 4 || (tx == 4 && (!mixed || b.H[0] < twice));
+  rep.wrap[1] = ty < 4 || (ty == 4 && (!mixed || b.H[1] < twice));
   const int want = std::max((tz + kBinCells - 1) / kBinCells,
                             (col_atoms + 255) / 256);
   rep.fz = std::max(1, (tz + want - 1) / want);
@@ -573,7 +587,9 @@ int build_box(pmnb_ctx *ctx, const double *e1, const double *e2,
     std::vector<int4> tshell;
     TileRep rep{};
     ctx->use_tile = ctx->prm.algorithm_cutoff >= rcp && packs &&
-                    make_tile_rep(b, rcp, ctx->n, rep, tshell);
+                    make_tile_rep(b, rcp, ctx->n,
+                                  ctx->prm.precision == PMNB_PREC_MIXED, rep,
+                                  tshell);
     ctx->tile_types = ctx->ntypes * ctx->ntypes <= kQLj;
     if (ctx->use_tile) {
       g = rep.grid;
@@ -1918,7 +1934,8 @@ int batch_finalize(pmnb_batch *b) {
     TileRep rep{};
     int na = 0;
     while (a + na < (int)b->rep_of.size() && b->rep_of[a + na] == r) na++;
-    if (!make_tile_rep(b->boxes[r], rcp, na, rep, shell))
+    if (!make_tile_rep(b->boxes[r], rcp, na,
+                       ctx->prm.precision == PMNB_PREC_MIXED, rep, shell))
       return fail(ctx, PMNB_ERR_UNSUPPORTED, "replica %d grid too large", r);
     rep.cell_off = (int)cells;
     rep.bin_off = (int)bins;

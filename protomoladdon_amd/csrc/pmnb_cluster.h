@@ -7,12 +7,13 @@
 // added once into the caller's array, each visit takes half the pair's energy
 // and virial: no atomics, fixed order.
 //
-// Candidates.  The neighbour columns (5 x 5; on an axis with fewer than five
-// columns each column once) give one or two runs of sorted slots each, the z
-// range of a column cut to what its x/y distance leaves of the cutoff.  Lane
-// l holds the bounds of run l (column l / 2, part l % 2); the runs laid end to
-// end are the positions 0 .. total - 1, read in rounds of 64.  A candidate
-// within the cutoff of the item's bounding box goes into the wave's LDS buffer.
+// Candidates.  The neighbour columns (5 x 5; on an axis with fewer than four
+// columns, FP64 five, each column once; with four one column at two images)
+// give one or two runs of sorted slots each, the z range of a column cut to
+// what its x/y distance leaves of the cutoff.  Lane l holds the bounds of run l
+// (column l / 2, part l % 2); the runs laid end to end are the positions 0 ..
+// total - 1, read in rounds of 64.  A candidate within the cutoff of the item's
+// bounding box goes into the wave's LDS buffer.
 //
 // Streams.  Position p belongs to stream (p / 16) % 4; each stream has its own
 // buffer contents and its own partial sums, and the four sums are added in

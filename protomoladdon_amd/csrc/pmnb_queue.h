@@ -4,8 +4,8 @@
 //
 // Each replica has its own column grid (TileRep): x/y columns at least half
 // a pair cutoff wide, so a neighbour's column offset is -2 .. 2.  On an axis
-// with fewer than five columns (box shorter than 2.5 cutoffs) every column
-// is taken once with the minimum image of every pair along it (as z is when
+// with fewer than four columns (box shorter than 2 cutoffs; FP64: five, 2.5
+// cutoffs) every column is taken once with the minimum image of every pair along it (as z is when
 // the cutoff reaches all z cells), so small boxes keep the reference's
 // one-image pair set.
 #pragma once

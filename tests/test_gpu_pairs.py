@@ -25,8 +25,8 @@ def types(n):
 
 def stretched(sx, sy, sz, n_mol=500):
     """Water in a box of sx, sy, sz times the cube's side (25 A at 500):
-    columns are 4.5 A wide, so an axis below 22.5 A has fewer than five and
-    takes the minimum image of every pair."""
+    columns are 4.5 A wide, so an axis below 18 A has fewer than four and
+    takes the minimum image of every pair, one below 22.5 A has four."""
     w = systems.small_water(n_mol=n_mol)
     L = float(w.topology.boundary_conditions.lengths()[0])
     s = np.array([sx, sy, sz])
@@ -36,6 +36,12 @@ def stretched(sx, sy, sz, n_mol=500):
         (a, 0, 0), (0, b, 0), (0, 0, c), (0.5 * a, 0.5 * b, 0.5 * c))
     w.name = "water_%g_%g_%g" % (sx, sy, sz)
     return w
+
+
+def side_lengths(a, b, c):
+    w = systems.small_water(n_mol=300)
+    L = float(w.topology.boundary_conditions.lengths()[0])
+    return stretched(a / L, b / L, c / L, n_mol=300)
 
 
 def gas(n_mol, L):
@@ -66,6 +72,11 @@ CASES = {
     "types257": lambda: types(257),
     "four_columns_x": lambda: stretched(0.85, 1.2, 1.0),
     "two_columns_y_flat_z": lambda: stretched(1.2, 0.73, 0.75),
+    # 18 A and what the band of the cutoff adds is the shortest axis whose
+    # fourth column is taken at two images
+    "four_columns_shortest": lambda: side_lengths(18.0003, 18.0001, 22.0),
+    "four_columns_short": lambda: side_lengths(18.0001, 18.01, 18.02),
+    "four_columns_long": lambda: side_lengths(18.3, 22.49, 31.0),
     "gas": lambda: gas(600, 120.0), "gas_no_pairs": lambda: gas(60, 90.0),
     "gas_three_molecules": lambda: gas(3, 200.0),
     "dense_column": lambda: stretched(0.8, 0.8, 12.0, n_mol=900),
