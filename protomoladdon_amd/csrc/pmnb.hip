@@ -3605,9 +3605,13 @@ int pmnb_pme_create(pmnb_ctx *ctx, int32_t nx, int32_t ny, int32_t nz,
   pm->n_cpart = blocks_for(std::max(n_atoms, 1), kPmeBlock / kPmeLanes);
   long long bins = 1;
   for (int a = 0; a < 3; a++) bins *= pm->nb[a] = blocks_for(nn[a], kPmeBin);
-  // four times the mean occupancy and 8 more, between 32 and 256
+  // four times the mean occupancy and 8 more, between 32 and 256; none where
+  // the tiles are few and full
+  const long long tiles = (long long)blocks_for(nx, kPmeTile) *
+                          blocks_for(ny, kPmeTile) * blocks_for(nz, kPmeTile);
   pm->cap = (int)std::max<long long>(
       32, std::min<long long>(256, 4 * (n_atoms / bins) + 8));
+  if (pme_all_atomic(tiles, order, n_atoms)) pm->cap = 0;
   auto up = [&](DevBuf &d, const void *src, size_t bytes) -> hipError_t {
     hipError_t e = d.ensure(std::max<size_t>(bytes, 16));
     if (e == hipSuccess && bytes && src)

@@ -47,6 +47,10 @@ constexpr int kPmeBlock = 256;
 constexpr int kPmeTile = 8;      // grid points of a spread tile, per axis
 constexpr int kPmeBin = 4;       // grid cells of an atom bin, per axis
 constexpr int kPmeList = 512;    // atoms of a tile listed in LDS
+// From this order on a lane that finds a tile's list full spreads its atom
+// alone: its weights are then formed once, not once a plane (96,000 atoms, 32^3,
+// order 8: 1,432 us, 1,730 with another turn of the list; order 4: 376 and 318).
+constexpr int kPmeLaneOrder = 6;
 constexpr int kPmeRow = kPmeTile + 1;  // LDS row and plane strides of a tile:
 constexpr int kPmePlane = kPmeTile * kPmeRow;  // an atom's planes on other banks
 constexpr int kPmeScalarBlocks = 4096;
@@ -59,6 +63,16 @@ constexpr double kPmeFixScale = 1099511627776.0;       // 2^40
 constexpr double kPmeFixInv = 1.0 / 1099511627776.0;
 constexpr double kPmeFixClamp = 4194304.0;             // 2^22
 
+// Whether all charges are added in memory: grids of few tiles, of more than 64
+// atoms each.  A whole evaluation of 96,000 atoms by tiles / in memory, orders
+// 2, 4, 6 and 8: 27 tiles 312 / 70, 627 / 295, 1,420 / 951, 3,094 / 2,338 us; 64
+// tiles 178 / 61, 318 / 270, 700 / 876, 1,430 / 2,052; 125 tiles 112 / 64, 183 /
+// 226; 900 atoms, 27 tiles 42 / 41, 47 / 55, 63 / 93, 105 / 164.
+inline bool pme_all_atomic(long long tiles, int order, int n_atoms) {
+  const int few = order == 2 ? 200 : (order == 4 ? 100 : 64);
+  return tiles < few && n_atoms / tiles > 64;
+}
+
 struct PmeDev {
   int n;                   // atoms
   int nx, ny, nz, nzh;     // grid, nz / 2 + 1
@@ -69,10 +83,10 @@ struct PmeDev {
   double fac;              // pi^2 / alpha^2
   const double *q;         // scaled charges
   int nb[3];               // atom bins per axis
-  int *count;              // atoms per bin, then all beyond their buckets
-                           // (zero between runs)
+  int *count;              // atoms per bin, then whether any is beyond its
+                           // bucket (zero between runs)
   double4 *bucket;         // cap records {grid x, y, z, charge} per bin
-  int cap;
+  int cap;                 // 0: all atoms are spread by k_pme_bin
   unsigned long long *qfix;  // nx ny nz: charges of the atoms beyond their
                            // buckets, 2^-40 (zero between runs)
   double *qreal;           // nx ny nz real grid
@@ -189,6 +203,8 @@ __device__ __forceinline__ void pme_spread_global(const PmeDev &d,
 // than on average.  32,000 atoms in a 68 A cube, 256^3 grid, with a list of
 // those atoms that every tile reads / with their charges added in memory: box
 // of 300 A 783 / 582 us (none beyond its bucket), of 830 A 1,472 / 693.
+// A grid of few tiles leaves the chip idle in k_pme_spread, one block a tile;
+// there (pme_all_atomic) all atoms are spread here and the tiles only convert.
 template <int P>
 __global__ __launch_bounds__(kPmeBlock) void k_pme_bin(PmeDev d,
                                                        const double *x) {
@@ -199,12 +215,12 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_bin(PmeDev d,
                                  pme_coord(x[3 * i + 2], d.hr[2], d.nz), d.q[i]);
   const int b = (((int)r.x / kPmeBin) * d.nb[1] + (int)r.y / kPmeBin) * d.nb[2] +
                 (int)r.z / kPmeBin;
-  const int k = atomicAdd(d.count + b, 1);
+  const int k = d.cap ? atomicAdd(d.count + b, 1) : 0;
   if (k < d.cap) {
     d.bucket[(size_t)b * d.cap + k] = r;
   } else {
     pme_spread_global<P>(d, r);
-    atomicAdd(d.count + (size_t)d.nb[0] * d.nb[1] * d.nb[2], 1);
+    d.count[(size_t)d.nb[0] * d.nb[1] * d.nb[2]] = 1;
   }
 }
 
@@ -324,8 +340,14 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_spread(PmeDev d) {
         if (!(reach(r.x, 0) && reach(r.y, 1) && reach(r.z, 2))) continue;
         const int at = __hip_atomic_fetch_add(&nlist, 1, __ATOMIC_RELAXED,
                                               __HIP_MEMORY_SCOPE_WORKGROUP);
-        if (at >= kPmeList) break;  // again when the list is spread
-        list[at] = r;
+        if (at < kPmeList) {
+          list[at] = r;
+        } else if (P < kPmeLaneOrder) {
+          break;  // again when the list is spread
+        } else {
+          for (int u = 0; u < P; u++)
+            pme_spread_plane<P>(d, r, u, t0, te, tile);
+        }
       }
       __syncthreads();
       const int listed = nlist;
@@ -333,7 +355,7 @@ __global__ __launch_bounds__(kPmeBlock) void k_pme_spread(PmeDev d) {
       for (int j = t; j < items; j += kPmeBlock)
         pme_spread_plane<P>(d, list[j / P], j % P, t0, te, tile);
       __syncthreads();
-      if (listed <= kPmeList) break;
+      if (P >= kPmeLaneOrder || listed <= kPmeList) break;
     }
   }
   for (int k = t; k < kPmeTile * kPmeTile * kPmeTile; k += kPmeBlock) {

@@ -40,9 +40,22 @@ def test_large_charges():
 @pytest.mark.parametrize("squeeze", [0.02, 0.5])
 def test_atoms_in_a_part_of_the_box(order, squeeze):
     """Far more atoms than a bucket and a tile's list hold, in a few bins."""
-    w = systems.small_water(n_mol=1200, elec="coulomb")
+    w = systems.small_water(n_mol=1000, elec="coulomb")
     w.positions = squeeze * w.positions
     check(w, (24, 27, 30), order, 0.35)
     outs, _ = run_device(w, (24, 27, 30), order, 0.35, repeat=3)
+    for f, o in outs[1:]:
+        assert np.array_equal(f, outs[0][0]) and np.array_equal(o, outs[0][1])
+
+
+@pytest.mark.parametrize("order,grid", [(2, (2, 3, 4)), (4, (4, 5, 9)),
+                                        (8, (8, 8, 8)), (6, (17, 8, 10))])
+@pytest.mark.parametrize("n_mol", [20, 500])
+def test_few_tiles(order, grid, n_mol):
+    """Grids of one to six tiles, by tiles (60 atoms) and by atomics in memory
+    (1,500 atoms: more than 64 a tile), which repeat bit for bit."""
+    w = systems.small_water(n_mol=n_mol, elec="coulomb")
+    check(w, grid, order, 0.35)
+    outs, _ = run_device(w, grid, order, 0.35, repeat=3)
     for f, o in outs[1:]:
         assert np.array_equal(f, outs[0][0]) and np.array_equal(o, outs[0][1])
