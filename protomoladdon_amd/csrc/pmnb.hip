@@ -3852,7 +3852,7 @@ EvalBufs carve_bufs(const pmnb_ctx *ctx, unsigned char *base, int cap,
 // The size include/pmnb.h gives one system against the 64 MiB: which systems
 // the entry takes is part of its interface and does not follow the layout of
 // carve_bufs, whose arrays are smaller (over boxes of 10 to 4,000 A, cutoffs
-// of 6 to 16 A and 1 to 700,000 atoms within the limit, at most 53 MiB with the
+// of 6 to 16 A and 1 to 700,000 atoms within the limit, at most 48 MiB with the
 // shortest bucket rows).
 size_t scratch_limit_size(const pmnb_ctx *ctx) {
   const bool mixed = ctx->prm.precision == PMNB_PREC_MIXED;
